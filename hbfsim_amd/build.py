@@ -18,9 +18,10 @@ LIB = HERE / "libhbfsim_amd.so"
 
 SOURCES = [CSRC / "engine.hip", CSRC / "gen.hip", CSRC / "thermal.hip", CSRC / "servers.hip",
            CSRC / "hybrid.hip", CSRC / "link.hip", CSRC / "admission.hip", CSRC / "order.hip",
-           CSRC / "probe.hip", CSRC / "api.cpp",
+           CSRC / "probe.hip", CSRC / "scratch.cpp", CSRC / "api.cpp",
            CSRC / "profile.cpp"]
-HEADERS = [CSRC / "engine.hpp", CSRC / "thermal.hpp", CSRC / "link.hpp", CSRC / "profile.hpp",
+HEADERS = [CSRC / "engine.hpp", CSRC / "thermal.hpp", CSRC / "link.hpp", CSRC / "scratch.hpp",
+           CSRC / "profile.hpp",
            CSRC / "json_min.hpp", ROOT / "include" / "hbfsim_amd.h"]
 
 
