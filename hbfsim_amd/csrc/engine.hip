@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include "engine.hpp"
+#include "scratch.hpp"
 #include "thermal.hpp"
 
 #include <algorithm>
@@ -4184,6 +4185,7 @@ struct engine {
     hipEvent_t ev[4]{};
     float last_ms[3]{0, 0, 0};
     std::uint64_t burst{0};
+    std::uint64_t* d_emp_svc{nullptr};  // the empirical model's services by run
     // the last completed run's modeled records and page-register hits: a
     // large stream with few hits is mostly general steps, and its next run
     // takes the four-wave apply pass (results are the same either way)
@@ -4275,7 +4277,14 @@ void hfree(T*& p)
 template <typename T>
 hipError_t halloc(T*& p, std::size_t count)
 {
-    return hipMalloc(reinterpret_cast<void**>(&p), sizeof(T) * (count == 0 ? 1 : count));
+    const std::size_t bytes = sizeof(T) * (count == 0 ? 1 : count);
+    hipError_t err = hipMalloc(reinterpret_cast<void**>(&p), bytes);
+    if (err != hipSuccess) {
+        (void)hipGetLastError();
+        scratch_trim();  // idle scratch goes first
+        err = hipMalloc(reinterpret_cast<void**>(&p), bytes);
+    }
+    return err;
 }
 
 std::uint32_t bits_for(std::uint32_t n)
@@ -4473,434 +4482,611 @@ __global__ __launch_bounds__(256) void k_window_counts(KArgs a, const hbf_record
 // One busy-until tail; a read's service is the cumulative curve's increment
 // at its burst run (streak of consecutive ascending pages with one
 // operation, capped at 1023, hbf_device.cuh:1031-1080), a write's is tPROG.
-// Three scans over tiles of 4096 records (256 threads x 16 consecutive
-// records): the streak summaries (associative, below) give every tile its
-// incoming burst state; with services known, the tail's (max,+) maps give
-// every tile its incoming busy time; the apply pass replays each thread's
-// records from both.  Services per run come from a 1024-entry table.
+//
+//   k_emp_tile<false>  per tile of 2,048 records: where its streaks start,
+//                      and the tail's (max,+) map of the records after the
+//                      first streak (whose runs do not depend on what came
+//                      before the tile);
+//   k_emp_chain        the burst state and sequence before every tile;
+//   k_emp_lead         per tile, the map of the first streak from that
+//                      state, joined to the rest: only those records are
+//                      read again (24 of 2,048 at a mean streak of 24);
+//   k_emp_tail         the tail before every tile, and the engine state;
+//   k_emp_tile<true>   completions, status and the tile report.
+//
+// A page and its operation are one number, key = page << 1 | op, so that a
+// record continues the streak when its key is the last one plus two.  Both
+// tile passes load record-per-lane, decode once and hand the records to the
+// threads eight in a row through LDS: a thread walks its records serially
+// (a wave scan per 64 records would spend six rounds of 64-bit moves on
+// each), and runs follow from two 32-bit scans over the threads (records so
+// far, and where the current streak started).  6M records: 104 us for the two
+// tile passes (43 + 61, 5.2 TB/s of records read and results written), against
+// 545 us for three when every pass gathered 16 records per thread at a
+// 512-byte stride, decoded them up to three times and folded the tile report
+// in one thread.
 constexpr int kEmpThreads = 256;
-constexpr std::uint32_t kEmpPer = 16;
+constexpr int kEmpWaves = kEmpThreads / kWave;
+constexpr int kEmpPer = 8;
 constexpr std::uint32_t kEmpTile = kEmpThreads * kEmpPer;
 constexpr std::uint64_t kRunCap = 1023;
-constexpr std::uint64_t kMaxEmpPage = (1ull << 53) - 2;
+// LDS slot of a tile's record: one pad per eight, so that threads reading
+// their eight in a row spread over the banks.
+constexpr std::uint32_t kEmpSlots = kEmpTile + kEmpTile / kEmpPer;
+__device__ __forceinline__ std::uint32_t emp_slot(std::uint32_t i) { return i + i / kEmpPer; }
 
-struct alignas(16) Burst {
-    std::uint64_t fpage, lpage;  // first / last page of the streak records
-    std::uint64_t lead, tail;    // lengths of the first and last streaks
-    std::uint64_t nburst;        // records taking part in streaks
-    std::uint64_t nmod;          // modeled records
-    std::uint32_t fop, lop, all, pad;
-};
-struct alignas(16) BState {
-    std::uint64_t page, run;
-    std::uint32_t op, valid;
-};
 struct alignas(16) TailMap {
     std::uint64_t A, B;  // b -> max(b + A, B)
 };
 
-__device__ __forceinline__ Burst burst_zero()
-{
-    Burst b;
-    b.fpage = b.lpage = b.lead = b.tail = b.nburst = b.nmod = 0;
-    b.fop = b.lop = b.all = b.pad = 0;
-    return b;
-}
+// A tile's streaks.
+struct alignas(16) EmpTile {
+    std::uint64_t fkey, lkey;  // first and last modeled record
+    std::uint32_t count;       // modeled records (0: the rest is unset)
+    std::uint32_t tail;        // length of the last streak, at most kRunCap
+    std::uint32_t all;         // 1: one streak
+    std::uint32_t lead_end;    // records up to the first streak's last one
+};
 
-// a then b
-__device__ __forceinline__ Burst burst_combine(const Burst& a, const Burst& b)
-{
-    if (b.nburst == 0) {
-        Burst r = a;
-        r.nmod = a.nmod + b.nmod;
-        return r;
-    }
-    if (a.nburst == 0) {
-        Burst r = b;
-        r.nmod = a.nmod + b.nmod;
-        return r;
-    }
-    const bool cont = a.lop == b.fop && a.lpage + 1 == b.fpage;
-    Burst r;
-    r.fpage = a.fpage;
-    r.fop = a.fop;
-    r.lpage = b.lpage;
-    r.lop = b.lop;
-    r.lead = (a.all && cont) ? a.lead + b.lead : a.lead;
-    r.tail = (b.all && cont) ? a.tail + b.tail : b.tail;
-    r.all = (a.all && b.all && cont) ? 1u : 0u;
-    r.nburst = a.nburst + b.nburst;
-    r.nmod = a.nmod + b.nmod;
-    r.pad = 0;
-    return r;
-}
-
-__device__ __forceinline__ BState burst_apply(const BState& st, const Burst& s)
-{
-    if (s.nburst == 0) {
-        return st;
-    }
-    const bool cont = st.valid && st.op == s.fop && st.page + 1 == s.fpage;
-    BState r;
-    r.page = s.lpage;
-    r.op = s.lop;
-    r.valid = 1;
-    const std::uint64_t len = (s.all && cont) ? st.run + s.tail : s.tail;
-    r.run = len < kRunCap ? len : kRunCap;
-    return r;
-}
-
-__device__ __forceinline__ void burst_add(Burst& b, std::uint64_t page, std::uint32_t op)
-{
-    if (b.nburst == 0) {
-        b.fpage = b.lpage = page;
-        b.fop = b.lop = op;
-        b.lead = b.tail = 1;
-        b.all = 1;
-    } else {
-        const bool cont = b.lop == op && b.lpage + 1 == page;
-        if (cont) {
-            ++b.tail;
-            if (b.all) {
-                ++b.lead;
-            }
-        } else {
-            b.all = 0;
-            b.tail = 1;
-        }
-        b.lpage = page;
-        b.lop = op;
-    }
-    ++b.nburst;
-}
-
-// One modeled record through the burst state (orc_update_empirical_burst):
-// its service in ps.
-__device__ __forceinline__ std::uint64_t emp_step(BState& st, std::uint64_t page,
-                                                  std::uint32_t op, const std::uint64_t* svc_ps,
-                                                  std::uint64_t program_ps)
-{
-    if (page > kMaxEmpPage) {
-        return 0;
-    }
-    const bool cont = st.valid && st.op == op && st.page + 1 == page;
-    const std::uint64_t run = cont ? (st.run < kRunCap ? st.run + 1 : kRunCap) : 1;
-    st.page = page;
-    st.op = op;
-    st.run = run;
-    st.valid = 1;
-    return op == 0 ? svc_ps[run] : program_ps;
-}
+// The burst state before a tile, and the modeled records before it.
+struct alignas(16) EmpState {
+    std::uint64_t key;
+    std::uint64_t seq;
+    std::uint32_t run, valid;
+    std::uint32_t pad[2];
+};
 
 __device__ __forceinline__ TailMap tail_compose(const TailMap& f, const TailMap& s)
 {
-    const std::uint64_t b = f.B + s.A;
-    return TailMap{f.A + s.A, b > s.B ? b : s.B};
+    return TailMap{f.A + s.A, umax64(f.B + s.A, s.B)};
 }
 
-// Inclusive scan over the block's threads, in thread order.
-template <class T, class F>
-__device__ T block_scan_incl(T v, T* buf, F op)
+__device__ __forceinline__ std::uint32_t wave_prefix_add32(std::uint32_t v)
 {
-    const int t = threadIdx.x;
-    buf[t] = v;
-    __syncthreads();
-    for (int o = 1; o < kEmpThreads; o <<= 1) {
-        T x = buf[t];
-        if (t >= o) {
-            x = op(buf[t - o], x);
-        }
-        __syncthreads();
-        buf[t] = x;
-        __syncthreads();
+    v += dpp32<0x111, 0xF>(v);
+    v += dpp32<0x112, 0xF>(v);
+    v += dpp32<0x114, 0xF>(v);
+    v += dpp32<0x118, 0xF>(v);
+    v += dpp32<0x142, 0xA>(v);
+    v += dpp32<0x143, 0xC>(v);
+    return v;
+}
+
+__device__ __forceinline__ std::uint64_t emp_service(std::uint64_t key, std::uint64_t run,
+                                                     const std::uint64_t* svc_ps,
+                                                     std::uint64_t program_ps)
+{
+    return (key & 1u) != 0 ? program_ps : svc_ps[run < kRunCap ? run : kRunCap];
+}
+
+// Media pages are below 2^52 here (4-KiB pages), far below the reference's
+// limit on burst pages (hbf_device.cuh:1031-1080), so every modeled record
+// takes part in streaks and key, operation and class share one word.
+template <bool kApply>
+__global__ __launch_bounds__(kEmpThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void k_emp_tile(KArgs a, const hbf_record32* rec, std::size_t n, std::uint64_t base_ps,
+                const std::uint64_t* svc_ps, std::uint64_t program_ps, EmpTile* tiles,
+                TailMap* maps, const EmpState* tile_in, const std::uint64_t* tile_tail,
+                std::uint64_t* completion, std::uint8_t* status, DevReport* tile_rep)
+{
+    extern __shared__ std::uint64_t fence[];
+    __shared__ ulonglong2 sh[kEmpSlots];  // issue (then completion), key << 2 | class
+    __shared__ std::uint32_t w_count[kEmpWaves], w_start[kEmpWaves], w_lead[kEmpWaves];
+    __shared__ std::uint64_t w_last[kEmpWaves];
+    __shared__ TailMap w_map[kEmpWaves];
+    // hybrid runs: the records' range ids (the sampler's key)
+    std::uint32_t* rid = reinterpret_cast<std::uint32_t*>(fence + a.r_nfence);
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const std::size_t begin = static_cast<std::size_t>(blockIdx.x) * kEmpTile;
+    uint4 x[kEmpPer], y[kEmpPer];
+#pragma unroll
+    for (int k = 0; k < kEmpPer; ++k) {
+        const std::size_t i = begin + static_cast<std::size_t>(k) * kEmpThreads + tid;
+        load_record(rec, i < n ? i : n - 1, x[k], y[k]);
     }
-    return buf[t];
-}
-
-struct EmpRec {
-    Dec d;
-    bool valid, modeled;
-};
-
-__device__ __forceinline__ EmpRec emp_decode(const KArgs& a, const std::uint64_t* fence,
-                                             RangeCache& rc, const hbf_record32* rec,
-                                             std::size_t n, std::size_t i, std::uint64_t base_ps)
-{
-    EmpRec r;
-    r.valid = i < n;
-    if (r.valid) {
-        uint4 x, y;
-        load_record(rec, i, x, y);
-        r.d = decode<false>(a, fence, rc, x, y, base_ps);
-    } else {
-        r.d = invalid_dec();
+    std::uint64_t before = base_ps;  // the issue time of the record before the tile
+    if (!kApply && a.disorder != nullptr && tid == 0 && begin != 0) {
+        before = base_ps + rec[begin - 1].issue_ps;
     }
-    r.modeled = r.valid && r.d.cls == kClsModeled;
-    return r;
-}
-
-__device__ __forceinline__ void emp_load_fences(const KArgs& a, std::uint64_t* fence)
-{
-    for (std::uint32_t j = threadIdx.x; j < a.r_nfence; j += kEmpThreads) {
+    for (std::uint32_t j = tid; j < a.r_nfence; j += kEmpThreads) {
         fence[j] = a.r_base[static_cast<std::size_t>(j) * a.r_stride];
     }
-}
-
-// The burst summary of this thread's records, and the block's.
-__device__ Burst emp_thread_burst(const KArgs& a, const std::uint64_t* fence,
-                                  const hbf_record32* rec, std::size_t n, std::size_t begin,
-                                  std::uint64_t base_ps)
-{
+    __syncthreads();
     RangeCache rc = empty_cache();
-    Burst b = burst_zero();
-    for (std::uint32_t k = 0; k < kEmpPer; ++k) {
-        const EmpRec r = emp_decode(a, fence, rc, rec, n, begin + k, base_ps);
-        if (r.modeled) {
-            ++b.nmod;
-            const std::uint64_t page = r.d.page1 - 1;
-            if (page <= kMaxEmpPage) {
-                burst_add(b, page, dec_op(r.d.bits));
+#pragma unroll
+    for (int k = 0; k < kEmpPer; ++k) {
+        const std::uint32_t at = k * kEmpThreads + tid;
+        const Dec d = decode<false>(a, fence, rc, x[k], y[k], base_ps);
+        const std::uint32_t cls = begin + at < n ? d.cls : kClsInvalid;
+        const std::uint64_t key =
+            cls == kClsModeled ? ((d.page1 - 1) << 1) | dec_op(d.bits) : 0ull;
+        sh[emp_slot(at)] = make_ulonglong2(d.issue, (key << 2) | cls);
+        if (kApply && a.hybrid) {
+            rid[emp_slot(at)] = d.range_id;
+        }
+    }
+    __syncthreads();
+    // this thread's eight records: modeled ones, first and last key, and the
+    // place (among them) where the last streak that starts inside starts
+    const std::uint32_t own = tid * kEmpPer;
+    std::uint64_t issue[kEmpPer], key[kEmpPer];
+    std::uint32_t cls[kEmpPer];
+#pragma unroll
+    for (int k = 0; k < kEmpPer; ++k) {
+        const ulonglong2 v = sh[emp_slot(own + k)];
+        issue[k] = v.x;
+        key[k] = v.y >> 2;
+        cls[k] = static_cast<std::uint32_t>(v.y) & 3u;
+    }
+    if (!kApply && a.disorder != nullptr) {
+        std::uint64_t prev = tid == 0 ? before : sh[emp_slot(own - 1)].x;
+        bool back = false;
+#pragma unroll
+        for (int k = 0; k < kEmpPer; ++k) {
+            back = back || (cls[k] != kClsInvalid && issue[k] - base_ps < prev - base_ps);
+            prev = issue[k];
+        }
+        if (__ballot(back) != 0 && lane == 0) {
+            *a.disorder = 1u;
+        }
+    }
+    std::uint32_t mine = 0, brk = 0;  // brk: 1 + the last inner start, 0: none
+    std::uint64_t first = 0, last = 0;
+#pragma unroll
+    for (int k = 0; k < kEmpPer; ++k) {
+        if (cls[k] == kClsModeled) {
+            if (mine == 0) {
+                first = key[k];
+            } else if (key[k] != last + 2) {
+                brk = mine + 1;
             }
+            last = key[k];
+            ++mine;
         }
     }
-    return b;
-}
-
-__global__ __launch_bounds__(kEmpThreads) void k_emp_burst(KArgs a, const hbf_record32* rec,
-                                                           std::size_t n, std::uint64_t base_ps,
-                                                           Burst* tiles)
-{
-    extern __shared__ std::uint64_t fence[];
-    __shared__ Burst buf[kEmpThreads];
-    emp_load_fences(a, fence);
+    const std::uint32_t incl = wave_prefix_add32(mine);
+    const std::uint64_t has = __ballot(mine != 0);
+    if (lane == kWave - 1) {
+        w_count[wave] = incl;
+    }
+    if (has != 0 && lane == 63 - __clzll(static_cast<long long>(has))) {
+        w_last[wave] = last;
+    }
     __syncthreads();
-    const std::size_t begin = static_cast<std::size_t>(blockIdx.x) * kEmpTile + threadIdx.x * kEmpPer;
-    const Burst b = emp_thread_burst(a, fence, rec, n, begin, base_ps);
-    const Burst incl = block_scan_incl(b, buf, burst_combine);
-    if (threadIdx.x == kEmpThreads - 1) {
-        tiles[blockIdx.x] = incl;
-    }
-}
-
-// One block: the burst state and modeled-request sequence before every
-// tile, and after the last.
-__global__ __launch_bounds__(kEmpThreads) void k_emp_burst_carry(const Burst* tiles,
-                                                                 std::size_t ntiles, BState init,
-                                                                 std::uint64_t seq0,
-                                                                 BState* tile_in,
-                                                                 std::uint64_t* tile_seq,
-                                                                 BState* final_state,
-                                                                 std::uint64_t* final_seq)
-{
-    __shared__ Burst buf[kEmpThreads];
-    const std::size_t per = (ntiles + kEmpThreads - 1) / kEmpThreads;
-    const std::size_t b = threadIdx.x * per;
-    const std::size_t e = b + per < ntiles ? b + per : ntiles;
-    Burst m = burst_zero();
-    for (std::size_t t = b; t < e; ++t) {
-        m = burst_combine(m, tiles[t]);
-    }
-    const Burst incl = block_scan_incl(m, buf, burst_combine);
-    Burst ex = burst_zero();
-    if (threadIdx.x > 0) {
-        ex = buf[threadIdx.x - 1];
-    }
-    BState st = burst_apply(init, ex);
-    std::uint64_t seq = seq0 + ex.nmod;
-    for (std::size_t t = b; t < e; ++t) {
-        tile_in[t] = st;
-        tile_seq[t] = seq;
-        st = burst_apply(st, tiles[t]);
-        seq += tiles[t].nmod;
-    }
-    if (threadIdx.x == kEmpThreads - 1) {
-        *final_state = burst_apply(init, incl);
-        *final_seq = seq0 + incl.nmod;
-    }
-}
-
-// Per thread: burst state at its first record (block scan of the thread
-// summaries from the tile's incoming state); returns it and the number of
-// modeled records before the thread within the tile.
-__device__ BState emp_thread_state(const KArgs& a, const std::uint64_t* fence,
-                                   const hbf_record32* rec, std::size_t n, std::size_t begin,
-                                   std::uint64_t base_ps, const BState& tile_state, Burst* buf,
-                                   std::uint64_t& nmod_before)
-{
-    const Burst mine = emp_thread_burst(a, fence, rec, n, begin, base_ps);
-    block_scan_incl(mine, buf, burst_combine);
-    Burst ex = burst_zero();
-    if (threadIdx.x > 0) {
-        ex = buf[threadIdx.x - 1];
-    }
-    nmod_before = ex.nmod;
-    return burst_apply(tile_state, ex);
-}
-
-__device__ TailMap emp_thread_map(const KArgs& a, const std::uint64_t* fence,
-                                  const hbf_record32* rec, std::size_t n, std::size_t begin,
-                                  std::uint64_t base_ps, BState st, const std::uint64_t* svc_ps,
-                                  std::uint64_t program_ps)
-{
-    RangeCache rc = empty_cache();
-    TailMap m{0, 0};
-    for (std::uint32_t k = 0; k < kEmpPer; ++k) {
-        const EmpRec r = emp_decode(a, fence, rc, rec, n, begin + k, base_ps);
-        if (r.modeled) {
-            const std::uint64_t svc =
-                emp_step(st, r.d.page1 - 1, dec_op(r.d.bits), svc_ps, program_ps);
-            m = tail_compose(m, TailMap{svc, r.d.issue + svc});
+    // records before this thread, and the key before its first one
+    std::uint32_t c = incl - mine;
+    std::uint64_t prev_key = 0;
+#pragma unroll
+    for (int w = 0; w < kEmpWaves; ++w) {
+        if (w < wave) {
+            c += w_count[w];
+            prev_key = w_count[w] != 0 ? w_last[w] : prev_key;
         }
     }
-    return m;
-}
-
-__global__ __launch_bounds__(kEmpThreads) void k_emp_map(KArgs a, const hbf_record32* rec,
-                                                         std::size_t n, std::uint64_t base_ps,
-                                                         const BState* tile_in,
-                                                         const std::uint64_t* svc_ps,
-                                                         std::uint64_t program_ps,
-                                                         TailMap* tiles)
-{
-    extern __shared__ std::uint64_t fence[];
-    __shared__ Burst buf[kEmpThreads];
-    __shared__ TailMap mbuf[kEmpThreads];
-    emp_load_fences(a, fence);
-    __syncthreads();
-    const std::size_t begin = static_cast<std::size_t>(blockIdx.x) * kEmpTile + threadIdx.x * kEmpPer;
-    std::uint64_t before = 0;
-    const BState st = emp_thread_state(a, fence, rec, n, begin, base_ps, tile_in[blockIdx.x], buf,
-                                       before);
-    const TailMap m = emp_thread_map(a, fence, rec, n, begin, base_ps, st, svc_ps, program_ps);
-    const TailMap incl = block_scan_incl(m, mbuf, tail_compose);
-    if (threadIdx.x == kEmpThreads - 1) {
-        tiles[blockIdx.x] = incl;
+    {
+        const std::uint64_t lower = has & lanemask_lt(lane);
+        const std::uint64_t pk =
+            shfl64(last, lower != 0 ? 63 - __clzll(static_cast<long long>(lower)) : lane);
+        prev_key = lower != 0 ? pk : prev_key;
     }
-}
-
-// One block: the tail before every tile and after the last.
-__global__ __launch_bounds__(kEmpThreads) void k_emp_tail_carry(const TailMap* tiles,
-                                                                std::size_t ntiles,
-                                                                std::uint64_t tail0,
-                                                                std::uint64_t* tile_tail,
-                                                                std::uint64_t* final_tail)
-{
-    __shared__ TailMap buf[kEmpThreads];
-    const std::size_t per = (ntiles + kEmpThreads - 1) / kEmpThreads;
-    const std::size_t b = threadIdx.x * per;
-    const std::size_t e = b + per < ntiles ? b + per : ntiles;
+    // where the streak starts that reaches this thread's end: 1 + the place
+    // among the tile's modeled records (1: the tile's first streak)
+    const bool cont = c != 0 && mine != 0 && first == prev_key + 2;
+    std::uint32_t start = 0;
+    if (mine != 0) {
+        start = brk != 0 ? c + brk : (cont ? 0u : c + 1);
+    }
+    const std::uint32_t smax = wave_prefix_max32(start);
+    if (lane == kWave - 1) {
+        w_start[wave] = smax;
+    }
+    __syncthreads();
+    std::uint32_t s_in = static_cast<std::uint32_t>(__shfl_up(static_cast<int>(smax), 1));
+    s_in = lane == 0 ? 0u : s_in;
+    std::uint32_t s_all = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < kEmpWaves; ++w) {
+        if (w < wave && w_start[w] > s_in) {
+            s_in = w_start[w];
+        }
+        s_all = w_start[w] > s_all ? w_start[w] : s_all;
+        total += w_count[w];
+    }
+    // services and this thread's map
+    EmpState in{};
+    std::uint64_t r0 = 0;  // the first streak's run before the tile
+    if (kApply) {
+        in = tile_in[blockIdx.x];
+        if (c == 0 && mine != 0) {
+            // the tile's first modeled record decides
+            r0 = in.valid != 0 && first == in.key + 2 ? in.run : 0;
+            w_lead[0] = static_cast<std::uint32_t>(r0);
+        }
+        __syncthreads();
+        r0 = total != 0 ? w_lead[0] : 0;
+    }
+    std::uint64_t svc[kEmpPer];
     TailMap m{0, 0};
-    for (std::size_t t = b; t < e; ++t) {
-        m = tail_compose(m, tiles[t]);
+    std::uint32_t lead_end = 0;
+    {
+        std::uint32_t at = c, s = s_in;
+        std::uint64_t pk = prev_key;
+#pragma unroll
+        for (int k = 0; k < kEmpPer; ++k) {
+            svc[k] = 0;
+            if (cls[k] != kClsModeled) {
+                continue;
+            }
+            if (at == 0 || key[k] != pk + 2) {
+                s = at + 1;
+            }
+            pk = key[k];
+            ++at;
+            const std::uint64_t run = at - s + 1 + (s == 1 ? r0 : 0);
+            if (!kApply && s == 1) {
+                lead_end = own + k + 1;  // left to k_emp_lead
+                continue;
+            }
+            svc[k] = emp_service(key[k], run, svc_ps, program_ps);
+            m = tail_compose(m, TailMap{svc[k], issue[k] + svc[k]});
+        }
     }
-    const TailMap incl = block_scan_incl(m, buf, tail_compose);
-    std::uint64_t g = tail0;
-    if (threadIdx.x > 0) {
-        const TailMap ex = buf[threadIdx.x - 1];
-        g = umax64(tail0 + ex.A, ex.B);
+    TailMap scan = m;
+    wave_scan(scan.A, scan.B);
+    if (lane == kWave - 1) {
+        w_map[wave] = scan;
     }
-    for (std::size_t t = b; t < e; ++t) {
-        tile_tail[t] = g;
-        g = umax64(g + tiles[t].A, tiles[t].B);
+    if (!kApply) {
+        lead_end = wave_prefix_max32(lead_end);
+        if (lane == kWave - 1) {
+            w_lead[wave] = lead_end;
+        }
+        __syncthreads();
+        if (tid == kEmpThreads - 1) {
+            TailMap all = w_map[0];
+            std::uint32_t le = w_lead[0];
+#pragma unroll
+            for (int w = 1; w < kEmpWaves; ++w) {
+                all = tail_compose(all, w_map[w]);
+                le = w_lead[w] > le ? w_lead[w] : le;
+            }
+            maps[blockIdx.x] = all;
+            EmpTile& t = tiles[blockIdx.x];
+            t.lkey = mine != 0 ? last : prev_key;
+            t.count = total;
+            const std::uint32_t len = total != 0 ? total - s_all + 1 : 0u;
+            t.tail = len < kRunCap ? len : static_cast<std::uint32_t>(kRunCap);
+            t.all = s_all == 1 ? 1u : 0u;
+            t.lead_end = le;
+        }
+        if (c == 0 && mine != 0) {
+            tiles[blockIdx.x].fkey = first;
+        }
+        return;
     }
-    if (threadIdx.x == kEmpThreads - 1) {
-        *final_tail = umax64(tail0 + incl.A, incl.B);
-    }
-}
-
-__global__ __launch_bounds__(kEmpThreads) void k_emp_apply(
-    KArgs a, const hbf_record32* rec, std::size_t n, std::uint64_t base_ps, const BState* tile_in,
-    const std::uint64_t* tile_seq, const std::uint64_t* tile_tail, const std::uint64_t* svc_ps,
-    std::uint64_t program_ps, std::uint64_t* completion, std::uint8_t* status, DevReport* tile_rep)
-{
-    extern __shared__ std::uint64_t fence[];
-    __shared__ Burst buf[kEmpThreads];
-    __shared__ TailMap mbuf[kEmpThreads];
-    emp_load_fences(a, fence);
     __syncthreads();
-    const std::size_t begin = static_cast<std::size_t>(blockIdx.x) * kEmpTile + threadIdx.x * kEmpPer;
-    std::uint64_t before = 0;
-    BState st = emp_thread_state(a, fence, rec, n, begin, base_ps, tile_in[blockIdx.x], buf,
-                                 before);
-    const TailMap mine = emp_thread_map(a, fence, rec, n, begin, base_ps, st, svc_ps, program_ps);
-    block_scan_incl(mine, mbuf, tail_compose);
+    // the tail before this thread's records
+    TailMap ex;
+    ex.A = shfl64(scan.A, lane == 0 ? 0 : lane - 1);
+    ex.B = shfl64(scan.B, lane == 0 ? 0 : lane - 1);
+    ex = lane == 0 ? TailMap{0, 0} : ex;
     std::uint64_t tail = tile_tail[blockIdx.x];
-    if (threadIdx.x > 0) {
-        const TailMap ex = mbuf[threadIdx.x - 1];
-        tail = umax64(tail + ex.A, ex.B);
-    }
-    std::uint64_t seq = tile_seq[blockIdx.x] + before;
-    unsigned long long v[14] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    RangeCache rc = empty_cache();
-    for (std::uint32_t k = 0; k < kEmpPer; ++k) {
-        const std::size_t i = begin + k;
-        const EmpRec r = emp_decode(a, fence, rc, rec, n, i, base_ps);
-        if (!r.valid) {
-            break;
+#pragma unroll
+    for (int w = 0; w < kEmpWaves; ++w) {
+        if (w < wave) {
+            tail = umax64(tail + w_map[w].A, w_map[w].B);
         }
-        ++v[R_RECORDS];
-        std::uint8_t sb = static_cast<std::uint8_t>(r.d.cls);
-        std::uint64_t done;
-        if (r.d.cls == kClsBypass) {
-            done = r.d.issue;
-            ++v[R_BYPASS];
-        } else if (r.d.cls == kClsUnsupported) {
+    }
+    tail = umax64(tail + ex.A, ex.B);
+    // counts of at most 2,048 a tile, 12 bits each: modeled, bypass,
+    // unsupported, reads, sampled
+    std::uint64_t counts = 0, makespan = 0, lat_lo = 0, lat_hi = 0, lat_max = 0, service = 0;
+    std::uint64_t seq = in.seq + c;
+#pragma unroll
+    for (int k = 0; k < kEmpPer; ++k) {
+        std::uint32_t sb = cls[k];
+        std::uint64_t done = issue[k];
+        if (cls[k] == kClsBypass) {
+            counts += 1ull << 12;
+        } else if (cls[k] == kClsUnsupported) {
             done = ~0ull;
-            ++v[R_UNSUPPORTED];
-        } else {
-            const std::uint32_t op = dec_op(r.d.bits);
-            const std::uint64_t page = r.d.page1 - 1;
+            counts += 1ull << 24;
+        } else if (cls[k] == kClsModeled) {
+            const std::uint32_t op = static_cast<std::uint32_t>(key[k]) & 1u;
             if (a.hybrid) {
-                const std::uint64_t key = (page << a.page_shift) ^
-                                          (static_cast<std::uint64_t>(r.d.range_id) << 32) ^ op;
+                const std::uint64_t h =
+                    ((key[k] >> 1) << a.page_shift) ^
+                    (static_cast<std::uint64_t>(rid[emp_slot(own + k)]) << 32) ^ op;
                 if (seq < a.hybrid_warmup ||
-                    (a.hybrid_threshold != 0 && mix64(seq ^ key) <= a.hybrid_threshold)) {
+                    (a.hybrid_threshold != 0 && mix64(seq ^ h) <= a.hybrid_threshold)) {
                     sb |= 8u;
-                    ++v[R_HYBRID];
+                    counts += 1ull << 48;
                 }
             }
             ++seq;
-            const std::uint64_t svc = emp_step(st, page, op, svc_ps, program_ps);
-            done = umax64(tail, r.d.issue) + svc;
+            done = umax64(tail, issue[k]) + svc[k];
             tail = done;
-            ++v[R_MODELED];
-            ++v[op == 0 ? R_READS : R_WRITES];
-            v[R_MAKESPAN] = umax64(v[R_MAKESPAN], done);
-            const std::uint64_t lat = done - r.d.issue;
-            const unsigned long long lo = v[R_LAT_LO] + lat;
-            v[R_LAT_HI] += lo < v[R_LAT_LO] ? 1u : 0u;
-            v[R_LAT_LO] = lo;
-            v[R_LAT_MAX] = umax64(v[R_LAT_MAX], lat);
-            v[R_SERVICE] += svc;
+            counts += 1ull + (op == 0 ? 1ull << 36 : 0ull);
+            makespan = umax64(makespan, done);
+            const std::uint64_t lat = done - issue[k];
+            lat_lo += lat;
+            lat_hi += lat_lo < lat ? 1u : 0u;
+            lat_max = umax64(lat_max, lat);
+            service += svc[k];
         }
-        put_done(&completion[i], done);
-        if (status != nullptr) {
-            status[i] = sb;
-        }
-    }
-    // block report
-    __shared__ unsigned long long part[kEmpThreads * 14];
-    for (int k = 0; k < 14; ++k) {
-        part[threadIdx.x * 14 + k] = v[k];
+        sh[emp_slot(own + k)] = make_ulonglong2(done, sb);
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        DevReport out{};
-        for (int t = 0; t < kEmpThreads; ++t) {
-            const unsigned long long* q = part + t * 14;
-            for (int k = 0; k < 14; ++k) {
-                if (k == R_MAKESPAN || k == R_LAT_MAX) {
-                    out.v[k] = umax64(out.v[k], q[k]);
-                } else if (k == R_LAT_LO) {
-                    const unsigned long long s2 = out.v[k] + q[k];
-                    out.v[R_LAT_HI] += s2 < out.v[k] ? 1u : 0u;
-                    out.v[k] = s2;
-                } else {
-                    out.v[k] += q[k];
-                }
+#pragma unroll
+    for (int k = 0; k < kEmpPer; ++k) {
+        const std::uint32_t at = k * kEmpThreads + tid;
+        const std::size_t i = begin + at;
+        if (i < n) {
+            const ulonglong2 v = sh[emp_slot(at)];
+            put_done(&completion[i], v.x);
+            if (status != nullptr) {
+                status[i] = static_cast<std::uint8_t>(v.y);
             }
         }
+    }
+    // tile report: wave reductions, then the four waves by one thread
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        counts += shfl64(counts, lane ^ o);
+        makespan = umax64(makespan, shfl64(makespan, lane ^ o));
+        lat_max = umax64(lat_max, shfl64(lat_max, lane ^ o));
+        service += shfl64(service, lane ^ o);
+        const std::uint64_t lo = shfl64(lat_lo, lane ^ o);
+        lat_hi += shfl64(lat_hi, lane ^ o);
+        lat_lo += lo;
+        lat_hi += lat_lo < lo ? 1u : 0u;
+    }
+    __shared__ std::uint64_t part[kEmpWaves][6];
+    if (lane == 0) {
+        part[wave][0] = counts;
+        part[wave][1] = makespan;
+        part[wave][2] = lat_max;
+        part[wave][3] = service;
+        part[wave][4] = lat_lo;
+        part[wave][5] = lat_hi;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < kEmpWaves; ++w) {
+            counts += part[w][0];
+            makespan = umax64(makespan, part[w][1]);
+            lat_max = umax64(lat_max, part[w][2]);
+            service += part[w][3];
+            lat_lo += part[w][4];
+            lat_hi += part[w][5] + (lat_lo < part[w][4] ? 1u : 0u);
+        }
+        const auto count = [&](int k) { return (counts >> (12 * k)) & 0xfffull; };
+        DevReport out{};
+        out.v[R_RECORDS] = n - begin < kEmpTile ? n - begin : kEmpTile;
+        out.v[R_MODELED] = count(0);
+        out.v[R_BYPASS] = count(1);
+        out.v[R_UNSUPPORTED] = count(2);
+        out.v[R_READS] = count(3);
+        out.v[R_WRITES] = count(0) - count(3);
+        out.v[R_HYBRID] = count(4);
+        out.v[R_MAKESPAN] = makespan;
+        out.v[R_LAT_LO] = lat_lo;
+        out.v[R_LAT_HI] = lat_hi;
+        out.v[R_LAT_MAX] = lat_max;
+        out.v[R_SERVICE] = service;
         tile_rep[blockIdx.x] = out;
+    }
+}
+
+// Streaks of a range of tiles, for the chain's scan.
+struct EmpSpan {
+    std::uint64_t fkey, lkey, count;
+    std::uint32_t tail, all;
+};
+
+// a then b
+__device__ __forceinline__ EmpSpan span_join(const EmpSpan& a, const EmpSpan& b)
+{
+    if (b.count == 0) {
+        return a;
+    }
+    if (a.count == 0) {
+        return b;
+    }
+    const bool cont = b.fkey == a.lkey + 2;
+    const std::uint32_t sum = a.tail + b.tail;
+    EmpSpan r;
+    r.fkey = a.fkey;
+    r.lkey = b.lkey;
+    r.count = a.count + b.count;
+    r.tail = !(b.all && cont) ? b.tail
+                              : (sum < kRunCap ? sum : static_cast<std::uint32_t>(kRunCap));
+    r.all = a.all && b.all && cont ? 1u : 0u;
+    return r;
+}
+
+__device__ __forceinline__ EmpState span_apply(const EmpState& st, const EmpSpan& s)
+{
+    if (s.count == 0) {
+        return st;
+    }
+    const bool cont = st.valid != 0 && s.fkey == st.key + 2;
+    const std::uint32_t sum = st.run + s.tail;
+    EmpState r{};
+    r.key = s.lkey;
+    r.valid = 1;
+    r.run = !(s.all && cont) ? s.tail
+                             : (sum < kRunCap ? sum : static_cast<std::uint32_t>(kRunCap));
+    r.seq = st.seq + s.count;
+    return r;
+}
+
+__device__ __forceinline__ EmpSpan span_of(const EmpTile& t)
+{
+    EmpSpan s;
+    s.count = t.count;
+    s.fkey = t.fkey;
+    s.lkey = t.lkey;
+    s.tail = t.tail;
+    s.all = t.all;
+    return s;
+}
+
+constexpr int kEmpChain = 1024;
+
+// One block, a run of tiles per thread: the burst state and sequence before
+// every tile, and after the last (`fin`).
+__global__ __launch_bounds__(kEmpChain) void k_emp_chain(const EmpTile* tiles, std::size_t ntiles,
+                                                         EmpState init, const std::uint64_t* seq0,
+                                                         EmpState* tile_in, EmpState* fin)
+{
+    __shared__ EmpSpan w_span[kEmpChain / kWave];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const std::size_t per = (ntiles + kEmpChain - 1) / kEmpChain;
+    const std::size_t b = threadIdx.x * per;
+    const std::size_t e = b + per < ntiles ? b + per : ntiles;
+    EmpSpan s{};
+    for (std::size_t t = b; t < e; ++t) {
+        s = span_join(s, span_of(tiles[t]));
+    }
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int src = lane >= o ? lane - o : lane;
+        EmpSpan p;
+        p.fkey = shfl64(s.fkey, src);
+        p.lkey = shfl64(s.lkey, src);
+        p.count = shfl64(s.count, src);
+        p.tail = static_cast<std::uint32_t>(__shfl(static_cast<int>(s.tail), src));
+        p.all = static_cast<std::uint32_t>(__shfl(static_cast<int>(s.all), src));
+        s = lane >= o ? span_join(p, s) : s;
+    }
+    if (lane == kWave - 1) {
+        w_span[wave] = s;
+    }
+    const int src = lane == 0 ? 0 : lane - 1;
+    EmpSpan ex;
+    ex.fkey = shfl64(s.fkey, src);
+    ex.lkey = shfl64(s.lkey, src);
+    ex.count = shfl64(s.count, src);
+    ex.tail = static_cast<std::uint32_t>(__shfl(static_cast<int>(s.tail), src));
+    ex.all = static_cast<std::uint32_t>(__shfl(static_cast<int>(s.all), src));
+    ex.count = lane == 0 ? 0ull : ex.count;
+    __syncthreads();
+    init.seq = *seq0;
+    EmpState st = init;
+    for (int w = 0; w < wave; ++w) {
+        st = span_apply(st, w_span[w]);
+    }
+    st = span_apply(st, ex);
+    for (std::size_t t = b; t < e; ++t) {
+        tile_in[t] = st;
+        st = span_apply(st, span_of(tiles[t]));
+    }
+    if (e == ntiles && b < e) {
+        *fin = st;
+    }
+}
+
+// One wave per tile: the map of the tile's first streak from its incoming
+// state, joined to the map of the rest.
+__global__ __launch_bounds__(kEmpThreads) void k_emp_lead(KArgs a, const hbf_record32* rec,
+                                                          std::size_t n, std::size_t ntiles,
+                                                          std::uint64_t base_ps,
+                                                          const std::uint64_t* svc_ps,
+                                                          std::uint64_t program_ps,
+                                                          const EmpTile* tiles,
+                                                          const EmpState* tile_in, TailMap* maps)
+{
+    extern __shared__ std::uint64_t fence[];
+    const int lane = threadIdx.x & (kWave - 1);
+    for (std::uint32_t j = threadIdx.x; j < a.r_nfence; j += kEmpThreads) {
+        fence[j] = a.r_base[static_cast<std::size_t>(j) * a.r_stride];
+    }
+    __syncthreads();
+    const std::size_t t = static_cast<std::size_t>(blockIdx.x) * kEmpWaves + threadIdx.x / kWave;
+    if (t >= ntiles) {
+        return;
+    }
+    const EmpTile et = tiles[t];
+    if (et.count == 0) {
+        return;  // nothing modeled: the rest's map is the identity already
+    }
+    const EmpState in = tile_in[t];
+    std::uint64_t run = in.valid != 0 && et.fkey == in.key + 2 ? in.run : 0;
+    const std::size_t begin = t * kEmpTile;
+    RangeCache rc = empty_cache();
+    TailMap m{0, 0};
+    for (std::uint32_t s = 0; s < et.lead_end; s += kWave) {
+        TailMap one{0, 0};
+        bool modeled = false;
+        Dec d = invalid_dec();
+        if (s + lane < et.lead_end) {
+            uint4 x, y;
+            load_record(rec, begin + s + lane, x, y);
+            d = decode<false>(a, fence, rc, x, y, base_ps);
+            modeled = d.cls == kClsModeled;
+        }
+        const std::uint64_t mask = __ballot(modeled);
+        if (modeled) {
+            const std::uint64_t key = ((d.page1 - 1) << 1) | dec_op(d.bits);
+            const std::uint64_t svc = emp_service(
+                key, run + 1 + __popcll(mask & lanemask_lt(lane)), svc_ps, program_ps);
+            one = TailMap{svc, d.issue + svc};
+        }
+        run += __popcll(mask);
+        wave_scan(one.A, one.B);
+        m = tail_compose(m, TailMap{readlane64(one.A, 63), readlane64(one.B, 63)});
+    }
+    if (lane == 0) {
+        maps[t] = tail_compose(m, maps[t]);
+    }
+}
+
+// One block: the tail before every tile.  Unless the stream went back in
+// time, also the engine state after the run: tail, sequence and the service
+// charged (the maps' sums).
+__global__ __launch_bounds__(kEmpChain) void k_emp_tail(const TailMap* maps, std::size_t ntiles,
+                                                        const EmpState* fin,
+                                                        const std::uint32_t* disorder,
+                                                        std::uint64_t* tile_tail,
+                                                        std::uint64_t* cursor, std::uint64_t* seq,
+                                                        std::uint64_t* total)
+{
+    __shared__ TailMap w_map[kEmpChain / kWave];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const std::size_t per = (ntiles + kEmpChain - 1) / kEmpChain;
+    const std::size_t b = threadIdx.x * per;
+    const std::size_t e = b + per < ntiles ? b + per : ntiles;
+    const std::uint64_t tail0 = *cursor;
+    TailMap m{0, 0};
+    for (std::size_t t = b; t < e; ++t) {
+        m = tail_compose(m, maps[t]);
+    }
+    wave_scan(m.A, m.B);
+    if (lane == kWave - 1) {
+        w_map[wave] = m;
+    }
+    TailMap ex;
+    ex.A = shfl64(m.A, lane == 0 ? 0 : lane - 1);
+    ex.B = shfl64(m.B, lane == 0 ? 0 : lane - 1);
+    ex = lane == 0 ? TailMap{0, 0} : ex;
+    __syncthreads();  // (every thread has read the cursor)
+    std::uint64_t g = tail0;
+    for (int w = 0; w < wave; ++w) {
+        g = umax64(g + w_map[w].A, w_map[w].B);
+    }
+    g = umax64(g + ex.A, ex.B);
+    for (std::size_t t = b; t < e; ++t) {
+        tile_tail[t] = g;
+        g = umax64(g + maps[t].A, maps[t].B);
+    }
+    if (threadIdx.x == 0 && (disorder == nullptr || *disorder == 0)) {
+        TailMap all{0, 0};
+        for (int w = 0; w < kEmpChain / kWave; ++w) {
+            all = tail_compose(all, w_map[w]);
+        }
+        *cursor = umax64(tail0 + all.A, all.B);
+        *seq = fin->seq;
+        *total += all.A;
     }
 }
 
@@ -5322,58 +5508,92 @@ int run_empirical(engine* e, const hbf_record32* d_rec, std::size_t n, std::uint
     if (c.page_shift != 12 || !emp_control_valid(c)) {
         return HBFSIM_UNSUPPORTED;
     }
-    const KArgs& a = e->args;
+    KArgs a = e->args;
+    a.disorder = in_order ? nullptr : e->d_disorder;
     const std::size_t ntiles = (n + kEmpTile - 1) / kEmpTile;
-    const std::vector<std::uint64_t> table = emp_service_table(c);
-    std::uint64_t* d_svc = nullptr;
-    Burst* d_bt = nullptr;
-    BState* d_in = nullptr;
-    std::uint64_t* d_tseq = nullptr;
-    TailMap* d_maps = nullptr;
-    std::uint64_t* d_tail = nullptr;
-    DevReport* d_trep = nullptr;
-    BState* d_final = nullptr;
-    std::uint64_t* d_fin = nullptr;  // [0] sequence, [1] tail
-    auto release = [&]() {
-        hfree(d_svc); hfree(d_bt); hfree(d_in); hfree(d_tseq); hfree(d_maps); hfree(d_tail);
-        hfree(d_trep); hfree(d_final); hfree(d_fin);
-    };
-    hipError_t err = halloc(d_svc, table.size());
-    if (err == hipSuccess) err = halloc(d_bt, ntiles);
-    if (err == hipSuccess) err = halloc(d_in, ntiles);
-    if (err == hipSuccess) err = halloc(d_tseq, ntiles);
-    if (err == hipSuccess) err = halloc(d_maps, ntiles);
-    if (err == hipSuccess) err = halloc(d_tail, ntiles);
-    if (err == hipSuccess) err = halloc(d_trep, ntiles);
-    if (err == hipSuccess) err = halloc(d_final, 1);
-    if (err == hipSuccess) err = halloc(d_fin, 2);
-    std::uint64_t seq0 = 0, tail0 = 0;
-    std::uint32_t back = 0;
-    const std::uint32_t zero = 0;
-    if (err == hipSuccess && !in_order &&
-        order_check(d_rec, false, n, e->d_disorder, stream) != HBFSIM_OK) {
-        err = hipErrorLaunchFailure;
+    if (ntiles > 0x7fffffffull) {
+        return HBFSIM_UNSUPPORTED;
     }
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(d_svc, table.data(), table.size() * 8, hipMemcpyHostToDevice, stream);
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(&seq0, e->d_seq, 8, hipMemcpyDeviceToHost, stream);
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(&tail0, e->d_cbusy, 8, hipMemcpyDeviceToHost, stream);
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(&back, e->d_disorder, 4, hipMemcpyDeviceToHost, stream);
-    if (err == hipSuccess) err = hipStreamSynchronize(stream);
-    if (err == hipSuccess && back != 0) {
-        err = hipMemcpyAsync(e->d_disorder, &zero, 4, hipMemcpyHostToDevice, stream);
-        if (err == hipSuccess) err = hipStreamSynchronize(stream);
+    if (e->d_emp_svc == nullptr) {
+        // (the profile's; made by the engine's first run)
+        const std::vector<std::uint64_t> table = emp_service_table(c);
+        if (halloc(e->d_emp_svc, table.size()) != hipSuccess) {
+            return HBFSIM_CUDA_ERROR;
+        }
+        if (hipMemcpy(e->d_emp_svc, table.data(), table.size() * 8, hipMemcpyHostToDevice) !=
+            hipSuccess) {
+            hfree(e->d_emp_svc);
+            return HBFSIM_CUDA_ERROR;
+        }
     }
-    if (err != hipSuccess) {
-        release();
+    const std::uint64_t* d_svc = e->d_emp_svc;
+    ScratchPlan plan;
+    const std::size_t o_tiles = plan.add<EmpTile>(ntiles);
+    const std::size_t o_in = plan.add<EmpState>(ntiles);
+    const std::size_t o_maps = plan.add<TailMap>(ntiles);
+    const std::size_t o_tail = plan.add<std::uint64_t>(ntiles);
+    const std::size_t o_rep = plan.add<DevReport>(ntiles);
+    const std::size_t o_fin = plan.add<EmpState>(1);
+    ScratchLease lease(plan.bytes, stream);
+    if (!lease.ok()) {
         return HBFSIM_CUDA_ERROR;
     }
-    if (back != 0) {
-        // a record's issue time goes back: served in (issue, position) order
-        release();
+    auto* d_tiles = lease.at<EmpTile>(o_tiles);
+    auto* d_in = lease.at<EmpState>(o_in);
+    auto* d_maps = lease.at<TailMap>(o_maps);
+    auto* d_tail = lease.at<std::uint64_t>(o_tail);
+    auto* d_trep = lease.at<DevReport>(o_rep);
+    auto* d_fin = lease.at<EmpState>(o_fin);
+    EmpState init{};
+    {
+        const std::uint64_t packed = e->burst;
+        const std::uint64_t p1 = packed >> 11;
+        init.valid = (packed != 0 && (packed & kRunCap) != 0 && p1 != 0) ? 1u : 0u;
+        init.key = ((p1 == 0 ? 0 : p1 - 1) << 1) | ((packed >> 10) & 1u);
+        init.run = static_cast<std::uint32_t>(packed & kRunCap);
+    }
+    const std::size_t lds = 8ull * a.r_nfence;
+    const std::size_t lds_apply = lds + (a.hybrid ? 4ull * kEmpSlots : 0ull);
+    const std::uint64_t program_ps = c.emp_program_ns * 1000ull;
+    const dim3 grid(static_cast<unsigned>(ntiles));
+    (void)hipEventRecord(e->ev[0], stream);
+    hipLaunchKernelGGL(k_emp_tile<false>, grid, dim3(kEmpThreads), lds, stream, a, d_rec, n,
+                       base_ps, d_svc, program_ps, d_tiles, d_maps,
+                       static_cast<const EmpState*>(nullptr),
+                       static_cast<const std::uint64_t*>(nullptr),
+                       static_cast<std::uint64_t*>(nullptr), static_cast<std::uint8_t*>(nullptr),
+                       static_cast<DevReport*>(nullptr));
+    (void)hipEventRecord(e->ev[1], stream);
+    hipLaunchKernelGGL(k_emp_chain, dim3(1), dim3(kEmpChain), 0, stream, d_tiles, ntiles, init,
+                       e->d_seq, d_in, d_fin);
+    hipLaunchKernelGGL(k_emp_lead, dim3(static_cast<unsigned>((ntiles + kEmpWaves - 1) / kEmpWaves)),
+                       dim3(kEmpThreads), lds, stream, a, d_rec, n, ntiles, base_ps, d_svc,
+                       program_ps, d_tiles, d_in, d_maps);
+    hipLaunchKernelGGL(k_emp_tail, dim3(1), dim3(kEmpChain), 0, stream, d_maps, ntiles, d_fin,
+                       a.disorder, d_tail, e->d_cbusy, e->d_seq, e->d_ctot);
+    (void)hipEventRecord(e->ev[2], stream);
+    hipLaunchKernelGGL(k_emp_tile<true>, grid, dim3(kEmpThreads), lds_apply, stream, a, d_rec, n,
+                       base_ps, d_svc, program_ps, static_cast<EmpTile*>(nullptr),
+                       static_cast<TailMap*>(nullptr), d_in, d_tail, d_comp, d_status, d_trep);
+    (void)hipEventRecord(e->ev[3], stream);
+    launch_report(stream, static_cast<const DevReport*>(d_trep), ntiles, e->d_rep,
+                  e->d_rep_parts, a.disorder);
+    EmpState fin{};
+    hipError_t err = hipGetLastError();
+    if (err == hipSuccess)
+        err = hipMemcpyAsync(e->h_rep, e->d_rep, sizeof(DevReport) + 8, hipMemcpyDeviceToHost,
+                             stream);
+    if (err == hipSuccess)
+        err = hipMemcpyAsync(&fin, d_fin, sizeof(fin), hipMemcpyDeviceToHost, stream);
+    if (err == hipSuccess) err = hipStreamSynchronize(stream);
+    if (err != hipSuccess) {
+        return HBFSIM_CUDA_ERROR;
+    }
+    lease.synced();
+    if (e->h_rep[1].v[0] != 0) {
+        // a record's issue time goes back: served in (issue, position) order;
+        // the engine state is as the run found it
+        lease.release();
         return run_in_issue_order(
             d_rec, false, n, d_comp, d_status, stream,
             [&](const void* sorted, std::uint64_t* comp, std::uint8_t* status) {
@@ -5381,66 +5601,8 @@ int run_empirical(engine* e, const hbf_record32* d_rec, std::size_t n, std::uint
                                      base_ps, stream, out, true);
             });
     }
-    BState init{};
-    {
-        const std::uint64_t packed = e->burst;
-        const std::uint64_t p1 = packed >> 11;
-        init.valid = (packed != 0 && (packed & kRunCap) != 0 && p1 != 0) ? 1u : 0u;
-        init.page = p1 == 0 ? 0 : p1 - 1;
-        init.op = static_cast<std::uint32_t>((packed >> 10) & 1u);
-        init.run = packed & kRunCap;
-    }
-    const std::size_t lds = 8ull * a.r_nfence;
-    const dim3 grid(static_cast<unsigned>(ntiles));
-    (void)hipEventRecord(e->ev[0], stream);
-    hipLaunchKernelGGL(k_emp_burst, grid, dim3(kEmpThreads), lds, stream, a, d_rec, n, base_ps,
-                       d_bt);
-    hipLaunchKernelGGL(k_emp_burst_carry, dim3(1), dim3(kEmpThreads), 0, stream,
-                       static_cast<const Burst*>(d_bt), ntiles, init, seq0, d_in, d_tseq, d_final,
-                       d_fin);
-    (void)hipEventRecord(e->ev[1], stream);
-    hipLaunchKernelGGL(k_emp_map, grid, dim3(kEmpThreads), lds, stream, a, d_rec, n, base_ps,
-                       static_cast<const BState*>(d_in), static_cast<const std::uint64_t*>(d_svc),
-                       c.emp_program_ns * 1000ull, d_maps);
-    hipLaunchKernelGGL(k_emp_tail_carry, dim3(1), dim3(kEmpThreads), 0, stream,
-                       static_cast<const TailMap*>(d_maps), ntiles, tail0, d_tail, d_fin + 1);
-    (void)hipEventRecord(e->ev[2], stream);
-    hipLaunchKernelGGL(k_emp_apply, grid, dim3(kEmpThreads), lds, stream, a, d_rec, n, base_ps,
-                       static_cast<const BState*>(d_in), static_cast<const std::uint64_t*>(d_tseq),
-                       static_cast<const std::uint64_t*>(d_tail),
-                       static_cast<const std::uint64_t*>(d_svc), c.emp_program_ns * 1000ull,
-                       d_comp, d_status, d_trep);
-    (void)hipEventRecord(e->ev[3], stream);
-    launch_report(stream, static_cast<const DevReport*>(d_trep), ntiles, e->d_rep,
-                  e->d_rep_parts, nullptr);
-    BState fin{};
-    std::uint64_t fin2[2] = {0, 0};
-    err = hipGetLastError();
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(e->h_rep, e->d_rep, sizeof(DevReport), hipMemcpyDeviceToHost, stream);
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(&fin, d_final, sizeof(BState), hipMemcpyDeviceToHost, stream);
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(fin2, d_fin, 16, hipMemcpyDeviceToHost, stream);
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(e->d_seq, d_fin, 8, hipMemcpyDeviceToDevice, stream);
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(e->d_cbusy, d_fin + 1, 8, hipMemcpyDeviceToDevice, stream);
-    std::uint64_t tot = 0;
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(&tot, e->d_ctot, 8, hipMemcpyDeviceToHost, stream);
-    if (err == hipSuccess) err = hipStreamSynchronize(stream);
-    if (err == hipSuccess) {
-        tot += e->h_rep->v[R_SERVICE];
-        err = hipMemcpyAsync(e->d_ctot, &tot, 8, hipMemcpyHostToDevice, stream);
-    }
-    if (err == hipSuccess) err = hipStreamSynchronize(stream);
-    release();
-    if (err != hipSuccess) {
-        return HBFSIM_CUDA_ERROR;
-    }
     if (fin.valid) {
-        e->burst = ((fin.page + 1) << 11) | (static_cast<std::uint64_t>(fin.op) << 10) | fin.run;
+        e->burst = (((fin.key >> 1) + 1) << 11) | ((fin.key & 1u) << 10) | fin.run;
     }
     for (int k = 0; k < 3; ++k) {
         float ms = 0.0f;
@@ -5661,7 +5823,9 @@ int engine_create(const engine_config& c, engine** out)
         return HBFSIM_IO_ERROR;
     }
     e->cfg = c;
+    scratch_hold();
     if (hipGetDevice(&e->device) != hipSuccess) {
+        scratch_drop();
         delete e;
         return HBFSIM_CUDA_ERROR;
     }
@@ -5761,6 +5925,7 @@ void engine_destroy(engine* e)
     hfree(e->d_rep);
     hfree(e->d_rep_parts);
     hfree(e->d_disorder);
+    hfree(e->d_emp_svc);
     if (e->h_rep != nullptr) {
         (void)hipHostFree(e->h_rep);
     }
@@ -5770,6 +5935,7 @@ void engine_destroy(engine* e)
         }
     }
     delete e;
+    scratch_drop();
 }
 
 const engine_config& engine_get_config(const engine* e) { return e->cfg; }

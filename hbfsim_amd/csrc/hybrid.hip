@@ -817,6 +817,7 @@ int sampler_create(std::uint32_t warmup, double sample_rate, std::uint64_t seed,
     if (s == nullptr) {
         return HBFSIM_INVALID_ARGUMENT;
     }
+    scratch_hold();
     s->warmup = warmup;
     s->seed = seed;
     s->threshold = sample_rate >= 1.0
@@ -832,8 +833,8 @@ void sampler_destroy(sampler_state* s)
 {
     if (s != nullptr) {
         (void)hipFree(s->seen_class);
-        scratch_trim();
         delete s;
+        scratch_drop();
     }
 }
 

@@ -20,17 +20,22 @@ std::mutex g_mu;
 // never destroyed: engines may outlive this file's static objects
 std::vector<Block>& g_blocks = *new std::vector<Block>;
 
-// Takes the idle blocks of `device` out of the list, oldest first, until at
+std::size_t g_holders = 0;
+
+// Takes the idle blocks of `device` (-1: of every device) out of the list, oldest first, until at
 // most `keep` idle bytes remain; the caller frees them without the lock.
 std::vector<void*> take_idle(int device, std::size_t keep)
 {
     std::size_t idle = 0;
+    const auto mine = [&](const Block& b) {
+        return !b.busy && (device < 0 || b.device == device);
+    };
     for (const Block& b : g_blocks) {
-        idle += b.device == device && !b.busy ? b.bytes : 0;
+        idle += mine(b) ? b.bytes : 0;
     }
     std::vector<void*> out;
     for (std::size_t k = 0; k < g_blocks.size() && idle > keep;) {
-        if (g_blocks[k].device == device && !g_blocks[k].busy) {
+        if (mine(g_blocks[k])) {
             out.push_back(g_blocks[k].ptr);
             idle -= g_blocks[k].bytes;
             g_blocks.erase(g_blocks.begin() + static_cast<std::ptrdiff_t>(k));
@@ -102,7 +107,8 @@ void scratch_give(void* block)
                 g_blocks[k].busy = false;
                 // the block used last is the one kept longest
                 std::rotate(g_blocks.begin() + static_cast<std::ptrdiff_t>(k),
-                            g_blocks.begin() + static_cast<std::ptrdiff_t>(k) + 1, g_blocks.end());
+                            g_blocks.begin() + static_cast<std::ptrdiff_t>(k) + 1,
+                            g_blocks.end());
                 drop = take_idle(g_blocks.back().device, kScratchKeep);
                 break;
             }
@@ -125,6 +131,27 @@ void scratch_trim()
     try {
         std::lock_guard<std::mutex> hold(g_mu);
         drop = take_idle(device, 0);
+    } catch (const std::bad_alloc&) {
+    }
+    for (void* p : drop) {
+        (void)hipFree(p);
+    }
+}
+
+void scratch_hold()
+{
+    std::lock_guard<std::mutex> hold(g_mu);
+    ++g_holders;
+}
+
+void scratch_drop()
+{
+    std::vector<void*> drop;
+    try {
+        std::lock_guard<std::mutex> hold(g_mu);
+        if (--g_holders == 0) {
+            drop = take_idle(-1, 0);
+        }
     } catch (const std::bad_alloc&) {
     }
     for (void* p : drop) {

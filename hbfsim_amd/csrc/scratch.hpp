@@ -5,9 +5,9 @@
 // 2.5 of its 4.0 ms in them.  A call takes one block for all its scratch and
 // gives it back once its stream has been synchronised, so a block never has
 // two users, whatever threads and streams they are on.  The pool keeps at
-// most kScratchKeep bytes of idle blocks per device; scratch_trim() returns
-// them (engines and samplers call it when they are destroyed, and every
-// allocation that fails does before it tries again).
+// most kScratchKeep bytes of idle blocks per device; they are freed when the
+// last engine or sampler is destroyed, and before an allocation that failed
+// is tried again.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -25,6 +25,10 @@ void* scratch_take(std::size_t bytes);
 void scratch_give(void* block);
 // Frees the idle blocks of the current device.
 void scratch_trim();
+// Engines and samplers hold the pool for as long as they live; the last one
+// to drop it frees the idle blocks of every device.
+void scratch_hold();
+void scratch_drop();
 
 // Lays out several arrays in one block, each 256-byte aligned.
 struct ScratchPlan {
