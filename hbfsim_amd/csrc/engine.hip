@@ -3810,6 +3810,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWide ? 4 : 
 {
     extern __shared__ std::uint64_t sm[];
     __shared__ std::uint64_t xp[33];
+    // a stream that went back in time is timed again from a sorted copy:
+    // nothing of this run is kept (8.4M records: 190 us not spent here)
+    if (a.disorder != nullptr && *a.disorder != 0u) {
+        return;
+    }
     if constexpr (kPacked) {
         if (a.tile_split != nullptr && a.tile_split[blockIdx.x] != 0) {
             apply_tile<kRefresh, kHits, kStaged, kPacked, true, kWide>(
@@ -4501,7 +4506,7 @@ __global__ __launch_bounds__(256) void k_window_counts(KArgs a, const hbf_record
 // (a wave scan per 64 records would spend six rounds of 64-bit moves on
 // each), and runs follow from two 32-bit scans over the threads (records so
 // far, and where the current streak started).  6M records: 104 us for the two
-// tile passes (43 + 61, 5.2 TB/s of records read and results written), against
+// tile passes (43 + 61 us, 4.5 and 4.0 TB/s of records and results), against
 // 545 us for three when every pass gathered 16 records per thread at a
 // 512-byte stride, decoded them up to three times and folded the tile report
 // in one thread.
