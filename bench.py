@@ -7,7 +7,7 @@ A step is one pass of the timing engine over one batch of access records
 resident in HBM (one decode step of the workload); engine state carries from
 step to step and each step's issue times start at the previous step's
 makespan.  Prints one JSON line with the modeled accesses/s, the roofline of
-the dominant kernel (HIP-event timed on the engine's stream) and the CPU
+the dominant kernel (timed by the engine from start to start) and the CPU
 oracle's rate on a bounded sample of the same stream, timed on this host.
 """
 from __future__ import annotations
@@ -470,9 +470,9 @@ def sub_line(engine, profile, ranges, batches, records, args, what: str, mode="f
         roof["from_profile"] = roofline_from_profile(kernels_summary, names[dominant],
                                                      kb[names[dominant]] * per_launch)
         if kms[dominant] < 0.1:
-            roof["timing_note"] = ("a kernel of tens of microseconds: the HIP-event interval "
-                                   "around it holds its dispatch too (2.5-5 us more than the "
-                                   "kernel trace's duration on config 0)")
+            roof["timing_note"] = ("a kernel of tens of microseconds: the interval from its "
+                                   "start to the next kernel's holds that one's dispatch too "
+                                   "(a few us more than the kernel trace's duration)")
     if traffic_summary is not None:
         traffic, src = committed_traffic(traffic_summary, names[dominant], int(per_launch))
         roof["traffic"], roof["traffic_source"] = traffic, src

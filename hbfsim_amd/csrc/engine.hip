@@ -151,7 +151,21 @@ struct KArgs {
     // tile holds a split step (the apply pass then takes its split-capable
     // body), else 0; null when the run takes no linear batches
     std::uint8_t* tile_split;
+    // start times of the summary pass, the carry chain and the apply pass
+    // (stamp_start)
+    std::uint64_t* stamp;
 };
+
+// The first workgroup of a run's kernels notes when it starts, by the GPU's
+// constant-rate clock.  (Event records between the kernels gave the same
+// intervals but kept 5-6 us of idle time at each: 17 us of a short run.)
+__device__ __forceinline__ void stamp_start(const KArgs& a, int which)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        a.stamp[which] = static_cast<std::uint64_t>(wall_clock64());
+    }
+}
+
 
 // Record operations: 0 read, 1 write, and 2 refresh of media page `addr`
 // (read out and programmed back), valid only with kMediaFlag.
@@ -1929,6 +1943,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
     const std::size_t tile = blockIdx.x;
     const std::size_t begin = tile * a.tile;
     const std::size_t end = begin + a.tile < n ? begin + a.tile : n;
+    stamp_start(a, 0);
     // set-up loads and the first group of records are in flight together
     const FenceRegs fr = fetch_fences(a, lane);
     const std::uint64_t xv = fetch_xfer(a, lane);
@@ -2407,6 +2422,7 @@ __global__ __launch_bounds__(256) void k_carry_up(KArgs a, std::size_t ntiles, s
 {
     const std::uint32_t rt = a.Rp + a.Rc + 1;
     const std::size_t id = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    stamp_start(a, 1);
     if (id >= ngroups * rt) {
         return;
     }
@@ -2732,6 +2748,7 @@ __global__ __launch_bounds__(kMidBlock) void k_carry_one(
 {
     __shared__ MidShared sh;
     __shared__ std::uint64_t red[kMidBlock / kWave];
+    stamp_start(a, 1);
     const std::uint32_t r = blockIdx.x;
     const std::size_t t0 = static_cast<std::size_t>(threadIdx.x) * span;
     const std::size_t t1 = t0 + span < ntiles ? t0 + span : ntiles;
@@ -3810,6 +3827,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWide ? 4 : 
 {
     extern __shared__ std::uint64_t sm[];
     __shared__ std::uint64_t xp[33];
+    stamp_start(a, 2);
     // a stream that went back in time is timed again from a sorted copy:
     // nothing of this run is kept (8.4M records: 190 us not spent here)
     if (a.disorder != nullptr && *a.disorder != 0u) {
@@ -3829,15 +3847,33 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWide ? 4 : 
                                                                 xp);
 }
 
-// Folds the per-tile report partials into one report (sums, maxima and the
-// 128-bit latency sum).  One block.
-// Report reduction in two launches: blocks fold runs of tile reports into
-// partials, then one block folds the partials.  A block's 256 threads are 16
+// Report reduction: each block folds a run of tile reports; the last block to
+// finish folds their partials and writes the result to pinned host memory
+// (two launches and a copy took 8-16 us).  A block's 256 threads are 16
 // streams x 16 words (the 14 report words, the carry out of the 128-bit
 // latency sum, padding); sums and maxima are exact in any order.
 constexpr int kRepWords = 16;
 constexpr int kRepCarry = 14;
 constexpr int kRepParts = 256;
+constexpr std::size_t kRepRun = 128;  // tile reports per block at least: one round of loads
+
+// The burst state before a tile of the empirical model, and the modeled
+// records before it.
+struct alignas(16) EmpState {
+    std::uint64_t key;
+    std::uint64_t seq;
+    std::uint32_t run, valid;
+    std::uint32_t pad[2];
+};
+
+// What a run leaves for the host, in pinned memory: the last kernel writes it
+// there (a copy command behind the kernels took another 4 us).
+struct HostOut {
+    DevReport rep;
+    std::uint64_t back;      // some record's issue time went back
+    std::uint64_t stamp[4];  // starts of the passes, and of the report
+    EmpState fin;            // the empirical model's burst state after the run
+};
 
 __device__ __forceinline__ void rep_join(int f, std::uint64_t& acc, std::uint64_t& carry,
                                          std::uint64_t v, std::uint64_t vcarry)
@@ -3853,22 +3889,23 @@ __device__ __forceinline__ void rep_join(int f, std::uint64_t& acc, std::uint64_
     }
 }
 
-// in: `count` entries of kIn words (14: tile reports, kRepWords: partials);
-// block b folds entries [b * per, (b + 1) * per).  With kFinal the single
-// block writes the report (carry added into the high latency word), else a
-// kRepWords partial per block.
-template <int kIn, bool kFinal>
-__global__ __launch_bounds__(256) void k_report(const std::uint64_t* in, std::size_t count,
-                                                std::size_t per, std::uint64_t* out,
-                                                std::uint32_t* disorder)
+// Folds entries [lo, hi) of kIn words (14: tile reports, kRepWords: partials)
+// into acc_sh[0] and carry_sh[0].  kShared: the entries were written by other
+// blocks of this launch.
+template <int kIn, bool kShared>
+__device__ __forceinline__ void rep_fold(const std::uint64_t* in, std::size_t lo, std::size_t hi,
+                                         std::uint64_t (*acc_sh)[kRepWords],
+                                         std::uint64_t* carry_sh)
 {
-    __shared__ std::uint64_t acc_sh[16][kRepWords];
-    __shared__ std::uint64_t carry_sh[16];
-    const int t = threadIdx.x;
-    const int f = t % kRepWords;
-    const int stream = t / kRepWords;
-    const std::size_t lo = static_cast<std::size_t>(blockIdx.x) * per;
-    const std::size_t hi = lo + per < count ? lo + per : count;
+    const int f = threadIdx.x % kRepWords;
+    const int stream = threadIdx.x / kRepWords;
+    const auto load = [&](std::size_t w) {
+        if constexpr (kShared) {
+            return __hip_atomic_load(&in[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+            return in[w];
+        }
+    };
     std::uint64_t acc = 0, carry = 0;
     // kBatch entries per stream are loaded before any is joined (one memory
     // round trip per batch, not per entry); entries past `hi` read as 0,
@@ -3879,15 +3916,16 @@ __global__ __launch_bounds__(256) void k_report(const std::uint64_t* in, std::si
 #pragma unroll
         for (int k = 0; k < kBatch; ++k) {
             const std::size_t i = i0 + 16 * static_cast<std::size_t>(k);
-            v[k] = i < hi && f < kIn ? in[i * kIn + f] : 0ull;
+            v[k] = i < hi && f < kIn ? load(i * kIn + f) : 0ull;
             // a partial's carry word travels with its latency word
-            vc[k] = i < hi && kIn == kRepWords && f == R_LAT_LO ? in[i * kIn + kRepCarry] : 0ull;
+            vc[k] = i < hi && kIn == kRepWords && f == R_LAT_LO ? load(i * kIn + kRepCarry) : 0ull;
         }
 #pragma unroll
         for (int k = 0; k < kBatch; ++k) {
             rep_join(f, acc, carry, f == kRepCarry ? 0ull : v[k], vc[k]);
         }
     }
+    __syncthreads();
     acc_sh[stream][f] = acc;
     if (f == R_LAT_LO) {
         carry_sh[stream] = carry;
@@ -3906,26 +3944,59 @@ __global__ __launch_bounds__(256) void k_report(const std::uint64_t* in, std::si
         }
         __syncthreads();
     }
-    if (stream == 0) {
-        if (kFinal) {
-            if (f < 14) {
-                out[f] = f == R_LAT_HI ? acc_sh[0][f] + carry_sh[0] : acc_sh[0][f];
-            } else if (f == 14) {
-                // the run's disorder flag travels with the report, and is
-                // cleared for the next run
-                out[14] = disorder != nullptr ? *disorder : 0u;
-                if (disorder != nullptr) {
-                    *disorder = 0u;
-                }
-            }
-        } else {
-            out[static_cast<std::size_t>(blockIdx.x) * kRepWords + f] =
-                f == kRepCarry ? carry_sh[0] : acc_sh[0][f];
+}
+
+// Block b folds tile reports [b * per, (b + 1) * per); `done` counts the
+// blocks that have (0 between launches).  The disorder flag travels with the
+// report and is cleared for the next run.
+__global__ __launch_bounds__(256) void k_report(const DevReport* tile_rep, std::size_t count,
+                                                std::size_t per, std::uint64_t* parts,
+                                                std::uint32_t* done, std::uint32_t* disorder,
+                                                const std::uint64_t* stamp, HostOut* out)
+{
+    __shared__ std::uint64_t acc_sh[16][kRepWords];
+    __shared__ std::uint64_t carry_sh[16];
+    __shared__ std::uint32_t last;
+    const std::uint64_t start = static_cast<std::uint64_t>(wall_clock64());
+    const int t = threadIdx.x;
+    const std::size_t lo = static_cast<std::size_t>(blockIdx.x) * per;
+    const std::size_t hi = lo + per < count ? lo + per : count;
+    rep_fold<14, false>(reinterpret_cast<const std::uint64_t*>(tile_rep), lo, hi, acc_sh,
+                        carry_sh);
+    if (gridDim.x > 1) {
+        if (t < kRepWords) {
+            parts[static_cast<std::size_t>(blockIdx.x) * kRepWords + t] =
+                t == kRepCarry ? carry_sh[0] : acc_sh[0][t];
+            __threadfence();
         }
+        __syncthreads();
+        if (t == 0) {
+            last = atomicAdd(done, 1u) + 1 == gridDim.x ? 1u : 0u;
+        }
+        __syncthreads();
+        if (last == 0) {
+            return;
+        }
+        __threadfence();
+        rep_fold<kRepWords, true>(parts, 0, gridDim.x, acc_sh, carry_sh);
+        if (t == 0) {
+            *done = 0;
+        }
+    }
+    if (t < 14) {
+        out->rep.v[t] = t == R_LAT_HI ? acc_sh[0][t] + carry_sh[0] : acc_sh[0][t];
+    } else if (t == 14) {
+        out->back = disorder != nullptr ? *disorder : 0u;
+        if (disorder != nullptr) {
+            *disorder = 0u;
+        }
+    } else if (t < 18) {
+        out->stamp[t - 15] = stamp[t - 15];
+    } else if (t == 18) {
+        out->stamp[3] = start;
     }
 }
 
-// Folds `ntiles` tile reports into `rep` (parts: kRepParts * kRepWords words).
 // ---- warp grouping (hbf_device.cu:1223-1231) ----------------------------
 //
 // The lanes of one warp instruction are consecutive records with one nonzero
@@ -4076,24 +4147,15 @@ __global__ __launch_bounds__(256) void k_follow(const hbf_record32* rec, std::si
     }
 }
 
-// The report's word 14 receives *disorder, which is then cleared (both skipped
-// when disorder is null); `rep` holds two DevReports.
+// Folds `ntiles` (at least 1) tile reports into *out; parts: kRepParts *
+// kRepWords words, done: a zero word.  disorder may be null.
 void launch_report(hipStream_t stream, const DevReport* tile_rep, std::size_t ntiles,
-                   DevReport* rep, std::uint64_t* parts, std::uint32_t* disorder)
+                   std::uint64_t* parts, std::uint32_t* done, std::uint32_t* disorder,
+                   const std::uint64_t* stamp, HostOut* out)
 {
-    const std::size_t per = (ntiles + kRepParts - 1) / kRepParts;
-    const std::size_t nparts = per == 0 ? 0 : (ntiles + per - 1) / per;
-    if (nparts == 0) {
-        hipLaunchKernelGGL((k_report<kRepWords, true>), dim3(1), dim3(256), 0, stream, parts,
-                           std::size_t{0}, std::size_t{1}, reinterpret_cast<std::uint64_t*>(rep),
-                           disorder);
-        return;
-    }
-    hipLaunchKernelGGL((k_report<14, false>), dim3(static_cast<unsigned>(nparts)), dim3(256), 0,
-                       stream, reinterpret_cast<const std::uint64_t*>(tile_rep), ntiles, per,
-                       parts, static_cast<std::uint32_t*>(nullptr));
-    hipLaunchKernelGGL((k_report<kRepWords, true>), dim3(1), dim3(256), 0, stream, parts, nparts,
-                       nparts, reinterpret_cast<std::uint64_t*>(rep), disorder);
+    const std::size_t per = std::max(kRepRun, (ntiles + kRepParts - 1) / kRepParts);
+    hipLaunchKernelGGL(k_report, dim3(static_cast<unsigned>((ntiles + per - 1) / per)), dim3(256),
+                       0, stream, tile_rep, ntiles, per, parts, done, disorder, stamp, out);
 }
 
 }  // namespace
@@ -4162,8 +4224,10 @@ struct engine {
     std::uint64_t* d_ptot{nullptr};
     std::uint64_t* d_ctot{nullptr};
     std::uint64_t* d_seq{nullptr};
-    DevReport* d_rep{nullptr};  // two: the report, then the disorder word
-    DevReport* h_rep{nullptr};  // pinned, the same two
+    HostOut* h_out{nullptr};    // pinned; written by a run's last kernel
+    std::uint32_t* d_done{nullptr};   // blocks of the report reduction that are done
+    std::uint64_t* d_stamp{nullptr};  // the passes' start times (KArgs::stamp)
+    double ms_per_tick{0};
     std::uint64_t* d_rep_parts{nullptr};  // report partials
     std::uint32_t* d_disorder{nullptr};  // a run's records went back in time
     // scratch
@@ -4187,7 +4251,6 @@ struct engine {
     std::uint32_t* d_desc_rid{nullptr};  // and their range ids (hybrid runs)
     SplitDesc* d_desc_split{nullptr};    // and split steps' second runs
     std::size_t desc_cap{0};
-    hipEvent_t ev[4]{};
     float last_ms[3]{0, 0, 0};
     std::uint64_t burst{0};
     std::uint64_t* d_emp_svc{nullptr};  // the empirical model's services by run
@@ -4533,14 +4596,6 @@ struct alignas(16) EmpTile {
     std::uint32_t lead_end;    // records up to the first streak's last one
 };
 
-// The burst state before a tile, and the modeled records before it.
-struct alignas(16) EmpState {
-    std::uint64_t key;
-    std::uint64_t seq;
-    std::uint32_t run, valid;
-    std::uint32_t pad[2];
-};
-
 __device__ __forceinline__ TailMap tail_compose(const TailMap& f, const TailMap& s)
 {
     return TailMap{f.A + s.A, umax64(f.B + s.A, s.B)};
@@ -4574,6 +4629,7 @@ void k_emp_tile(KArgs a, const hbf_record32* rec, std::size_t n, std::uint64_t b
                 TailMap* maps, const EmpState* tile_in, const std::uint64_t* tile_tail,
                 std::uint64_t* completion, std::uint8_t* status, DevReport* tile_rep)
 {
+    stamp_start(a, kApply ? 2 : 0);
     extern __shared__ std::uint64_t fence[];
     __shared__ ulonglong2 sh[kEmpSlots];  // issue (then completion), key << 2 | class
     __shared__ std::uint32_t w_count[kEmpWaves], w_start[kEmpWaves], w_lead[kEmpWaves];
@@ -4941,11 +4997,13 @@ constexpr int kEmpChain = 1024;
 
 // One block, a run of tiles per thread: the burst state and sequence before
 // every tile, and after the last (`fin`).
-__global__ __launch_bounds__(kEmpChain) void k_emp_chain(const EmpTile* tiles, std::size_t ntiles,
+__global__ __launch_bounds__(kEmpChain) void k_emp_chain(KArgs a, const EmpTile* tiles, std::size_t ntiles,
                                                          EmpState init, const std::uint64_t* seq0,
-                                                         EmpState* tile_in, EmpState* fin)
+                                                         EmpState* tile_in,
+                                                         std::uint64_t* fin_seq, EmpState* fin)
 {
     __shared__ EmpSpan w_span[kEmpChain / kWave];
+    stamp_start(a, 1);
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const std::size_t per = (ntiles + kEmpChain - 1) / kEmpChain;
     const std::size_t b = threadIdx.x * per;
@@ -4988,6 +5046,7 @@ __global__ __launch_bounds__(kEmpChain) void k_emp_chain(const EmpTile* tiles, s
     }
     if (e == ntiles && b < e) {
         *fin = st;
+        *fin_seq = st.seq;
     }
 }
 
@@ -5050,7 +5109,7 @@ __global__ __launch_bounds__(kEmpThreads) void k_emp_lead(KArgs a, const hbf_rec
 // time, also the engine state after the run: tail, sequence and the service
 // charged (the maps' sums).
 __global__ __launch_bounds__(kEmpChain) void k_emp_tail(const TailMap* maps, std::size_t ntiles,
-                                                        const EmpState* fin,
+                                                        const std::uint64_t* fin_seq,
                                                         const std::uint32_t* disorder,
                                                         std::uint64_t* tile_tail,
                                                         std::uint64_t* cursor, std::uint64_t* seq,
@@ -5090,7 +5149,7 @@ __global__ __launch_bounds__(kEmpChain) void k_emp_tail(const TailMap* maps, std
             all = tail_compose(all, w_map[w]);
         }
         *cursor = umax64(tail0 + all.A, all.B);
-        *seq = fin->seq;
+        *seq = *fin_seq;
         *total += all.A;
     }
 }
@@ -5408,7 +5467,11 @@ void choose_match(KArgs& a)
 // below that, the largest that gives every CU eight tiles, at least 256.
 // (Mid-sized runs of 2^22 to 2^25 records take twice the tiles they would at
 // eight per CU: more waves to cover the per-record passes' latency, at the
-// price of a carry chain of twice the tiles.)
+// price of a carry chain of twice the tiles.)  Runs of fewer than 1,024 such
+// tiles (up to 2^18 records) leave most of the chip idle and take as long as
+// one tile's steps in a row: their tiles go down to 64 records, one step each
+// (4,096 records 87 -> 72 us, 2^16 92 -> 81; at 2^18 records 64-record tiles
+// cost the carry chain more than they save, 105 -> 116).
 std::uint32_t auto_tile(std::size_t n)
 {
     std::uint32_t t = 16384;
@@ -5416,6 +5479,9 @@ std::uint32_t auto_tile(std::size_t n)
         t >>= 1;
     }
     while (t > 256 && (n + t - 1) / t < 2048) {
+        t >>= 1;
+    }
+    while (t > 64 && (n + t - 1) / t < 1024) {
         t >>= 1;
     }
     return t;
@@ -5505,6 +5571,15 @@ std::vector<std::uint64_t> emp_service_table(const engine_config& c)
     return t;
 }
 
+// The passes' times over the run that has just completed, from their stamps.
+void note_times(engine* e)
+{
+    for (int k = 0; k < 3; ++k) {
+        const std::uint64_t from = e->h_out->stamp[k], to = e->h_out->stamp[k + 1];
+        e->last_ms[k] = to > from ? static_cast<float>((to - from) * e->ms_per_tick) : 0.0f;
+    }
+}
+
 int run_empirical(engine* e, const hbf_record32* d_rec, std::size_t n, std::uint64_t* d_comp,
                   std::uint8_t* d_status, std::uint64_t base_ps, hipStream_t stream,
                   hbfsim_amd_report* out, bool in_order)
@@ -5538,7 +5613,7 @@ int run_empirical(engine* e, const hbf_record32* d_rec, std::size_t n, std::uint
     const std::size_t o_maps = plan.add<TailMap>(ntiles);
     const std::size_t o_tail = plan.add<std::uint64_t>(ntiles);
     const std::size_t o_rep = plan.add<DevReport>(ntiles);
-    const std::size_t o_fin = plan.add<EmpState>(1);
+    const std::size_t o_fseq = plan.add<std::uint64_t>(1);
     ScratchLease lease(plan.bytes, stream);
     if (!lease.ok()) {
         return HBFSIM_CUDA_ERROR;
@@ -5548,7 +5623,7 @@ int run_empirical(engine* e, const hbf_record32* d_rec, std::size_t n, std::uint
     auto* d_maps = lease.at<TailMap>(o_maps);
     auto* d_tail = lease.at<std::uint64_t>(o_tail);
     auto* d_trep = lease.at<DevReport>(o_rep);
-    auto* d_fin = lease.at<EmpState>(o_fin);
+    auto* d_fseq = lease.at<std::uint64_t>(o_fseq);  // the sequence after the run
     EmpState init{};
     {
         const std::uint64_t packed = e->burst;
@@ -5561,41 +5636,31 @@ int run_empirical(engine* e, const hbf_record32* d_rec, std::size_t n, std::uint
     const std::size_t lds_apply = lds + (a.hybrid ? 4ull * kEmpSlots : 0ull);
     const std::uint64_t program_ps = c.emp_program_ns * 1000ull;
     const dim3 grid(static_cast<unsigned>(ntiles));
-    (void)hipEventRecord(e->ev[0], stream);
     hipLaunchKernelGGL(k_emp_tile<false>, grid, dim3(kEmpThreads), lds, stream, a, d_rec, n,
                        base_ps, d_svc, program_ps, d_tiles, d_maps,
                        static_cast<const EmpState*>(nullptr),
                        static_cast<const std::uint64_t*>(nullptr),
                        static_cast<std::uint64_t*>(nullptr), static_cast<std::uint8_t*>(nullptr),
                        static_cast<DevReport*>(nullptr));
-    (void)hipEventRecord(e->ev[1], stream);
-    hipLaunchKernelGGL(k_emp_chain, dim3(1), dim3(kEmpChain), 0, stream, d_tiles, ntiles, init,
-                       e->d_seq, d_in, d_fin);
+    hipLaunchKernelGGL(k_emp_chain, dim3(1), dim3(kEmpChain), 0, stream, a, d_tiles, ntiles, init,
+                       e->d_seq, d_in, d_fseq, &e->h_out->fin);
     hipLaunchKernelGGL(k_emp_lead, dim3(static_cast<unsigned>((ntiles + kEmpWaves - 1) / kEmpWaves)),
                        dim3(kEmpThreads), lds, stream, a, d_rec, n, ntiles, base_ps, d_svc,
                        program_ps, d_tiles, d_in, d_maps);
-    hipLaunchKernelGGL(k_emp_tail, dim3(1), dim3(kEmpChain), 0, stream, d_maps, ntiles, d_fin,
+    hipLaunchKernelGGL(k_emp_tail, dim3(1), dim3(kEmpChain), 0, stream, d_maps, ntiles, d_fseq,
                        a.disorder, d_tail, e->d_cbusy, e->d_seq, e->d_ctot);
-    (void)hipEventRecord(e->ev[2], stream);
     hipLaunchKernelGGL(k_emp_tile<true>, grid, dim3(kEmpThreads), lds_apply, stream, a, d_rec, n,
                        base_ps, d_svc, program_ps, static_cast<EmpTile*>(nullptr),
                        static_cast<TailMap*>(nullptr), d_in, d_tail, d_comp, d_status, d_trep);
-    (void)hipEventRecord(e->ev[3], stream);
-    launch_report(stream, static_cast<const DevReport*>(d_trep), ntiles, e->d_rep,
-                  e->d_rep_parts, a.disorder);
-    EmpState fin{};
+    launch_report(stream, d_trep, ntiles, e->d_rep_parts, e->d_done, a.disorder, e->d_stamp,
+                  e->h_out);
     hipError_t err = hipGetLastError();
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(e->h_rep, e->d_rep, sizeof(DevReport) + 8, hipMemcpyDeviceToHost,
-                             stream);
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(&fin, d_fin, sizeof(fin), hipMemcpyDeviceToHost, stream);
     if (err == hipSuccess) err = hipStreamSynchronize(stream);
     if (err != hipSuccess) {
         return HBFSIM_CUDA_ERROR;
     }
     lease.synced();
-    if (e->h_rep[1].v[0] != 0) {
+    if (e->h_out->back != 0) {
         // a record's issue time goes back: served in (issue, position) order;
         // the engine state is as the run found it
         lease.release();
@@ -5606,17 +5671,13 @@ int run_empirical(engine* e, const hbf_record32* d_rec, std::size_t n, std::uint
                                      base_ps, stream, out, true);
             });
     }
+    const EmpState& fin = e->h_out->fin;
     if (fin.valid) {
         e->burst = (((fin.key >> 1) + 1) << 11) | ((fin.key & 1u) << 10) | fin.run;
     }
-    for (int k = 0; k < 3; ++k) {
-        float ms = 0.0f;
-        if (hipEventElapsedTime(&ms, e->ev[k], e->ev[k + 1]) == hipSuccess) {
-            e->last_ms[k] = ms;
-        }
-    }
+    note_times(e);
     if (out != nullptr) {
-        std::memcpy(out, e->h_rep, sizeof(DevReport));
+        std::memcpy(out, &e->h_out->rep, sizeof(DevReport));
     }
     return HBFSIM_OK;
 }
@@ -5884,14 +5945,17 @@ int engine_create(const engine_config& c, engine** out)
     if (err == hipSuccess) err = halloc(e->d_ptot, rp);
     if (err == hipSuccess) err = halloc(e->d_ctot, rc);
     if (err == hipSuccess) err = halloc(e->d_seq, 1);
-    if (err == hipSuccess) err = halloc(e->d_rep, 2);
+    if (err == hipSuccess) err = halloc(e->d_done, 1);
+    if (err == hipSuccess) err = halloc(e->d_stamp, 4);
     if (err == hipSuccess) err = halloc(e->d_rep_parts, kRepParts * kRepWords);
     if (err == hipSuccess) err = halloc(e->d_disorder, 1);
     if (err == hipSuccess)
-        err = hipHostMalloc(reinterpret_cast<void**>(&e->h_rep), 2 * sizeof(DevReport));
-    for (int i = 0; i < 4 && err == hipSuccess; ++i) {
-        err = hipEventCreate(&e->ev[i]);
-    }
+        err = hipHostMalloc(reinterpret_cast<void**>(&e->h_out), sizeof(HostOut));
+    int khz = 0;
+    if (err == hipSuccess)
+        err = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, e->device);
+    e->ms_per_tick = khz > 0 ? 1.0 / khz : 0.0;
+    a.stamp = e->d_stamp;
     if (err != hipSuccess) {
         engine_destroy(e);
         return HBFSIM_CUDA_ERROR;
@@ -5927,17 +5991,13 @@ void engine_destroy(engine* e)
     hfree(e->d_ptot);
     hfree(e->d_ctot);
     hfree(e->d_seq);
-    hfree(e->d_rep);
+    hfree(e->d_done);
+    hfree(e->d_stamp);
     hfree(e->d_rep_parts);
     hfree(e->d_disorder);
     hfree(e->d_emp_svc);
-    if (e->h_rep != nullptr) {
-        (void)hipHostFree(e->h_rep);
-    }
-    for (auto& ev : e->ev) {
-        if (ev != nullptr) {
-            (void)hipEventDestroy(ev);
-        }
+    if (e->h_out != nullptr) {
+        (void)hipHostFree(e->h_out);
     }
     delete e;
     scratch_drop();
@@ -5962,6 +6022,7 @@ int engine_reset(engine* e)
     if (err == hipSuccess) err = hipMemset(e->d_ctot, 0, rc * 8);
     if (err == hipSuccess) err = hipMemset(e->d_seq, 0, 8);
     if (err == hipSuccess) err = hipMemset(e->d_disorder, 0, 4);
+    if (err == hipSuccess) err = hipMemset(e->d_done, 0, 4);
     if (err == hipSuccess) err = hipDeviceSynchronize();
     e->burst = 0;
     return hip_status(err);
@@ -6214,7 +6275,6 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
         }
     }
     const dim3 grid(static_cast<unsigned>(ntiles));
-    (void)hipEventRecord(e->ev[0], stream);
     const std::uint8_t* hits = d_hits;
     if (k2) {
         (void)allow_lds(k_summary<false, true>, lds_a);
@@ -6247,7 +6307,6 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
                            n, base_ps, sc.psum, sc.tmask, sc.csum, sc.tcount,
                            hits, desc);
     }
-    (void)hipEventRecord(e->ev[1], stream);
     {
         const std::size_t ngroups = (ntiles + kGroup - 1) / kGroup;
         const std::size_t rt = static_cast<std::size_t>(a.Rp) + a.Rc + 1;
@@ -6272,7 +6331,6 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
                                sc.gccarry, sc.gseq, sc.pcarry, sc.ccarry, sc.tseq);
         }
     }
-    (void)hipEventRecord(e->ev[2], stream);
     const bool staged = desc != nullptr && staged_steps(a) != 0;
     // the four-wave apply pass: a large stream whose last run on this engine
     // had few page-register hits (mostly general steps), where LDS leaves
@@ -6327,10 +6385,8 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
                            base_ps, sc.pcarry, sc.tmask, sc.ccarry, sc.tseq, d_comp,
                            d_status, sc.tile_rep, hits, desc);
     }
-    // (the apply pass's interval ends with it: the report reduction's two
-    // small launches are no part of it)
-    (void)hipEventRecord(e->ev[3], stream);
-    launch_report(stream, sc.tile_rep, ntiles, e->d_rep, e->d_rep_parts, e->d_disorder);
+    launch_report(stream, sc.tile_rep, ntiles, e->d_rep_parts, e->d_done, e->d_disorder,
+                  e->d_stamp, e->h_out);
     unsigned long long h_frep[8] = {};
     if (grouping) {
         const std::size_t nb = (n + 255) / 256;
@@ -6340,13 +6396,10 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
                            base_ps, d_lead, d_comp, d_status, d_frep);
     }
     err = hipGetLastError();
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(e->h_rep, e->d_rep, sizeof(DevReport) + 8, hipMemcpyDeviceToHost,
-                             stream);
     if (err == hipSuccess && grouping)
         err = hipMemcpyAsync(h_frep, d_frep, sizeof(h_frep), hipMemcpyDeviceToHost, stream);
     if (err == hipSuccess) err = hipStreamSynchronize(stream);
-    const bool went_back = err == hipSuccess && e->h_rep[1].v[0] != 0;
+    const bool went_back = err == hipSuccess && e->h_out->back != 0;
     // two page registers: the tags the run leaves, unless it is timed again
     if (err == hipSuccess && k2 && !went_back) {
         err = hipMemcpyAsync(e->d_ptag, k2_tags.data(), k2_tags.size() * 8, hipMemcpyHostToDevice,
@@ -6373,16 +6426,11 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
                                       out, refresh_records, nullptr, true);
             });
     }
-    e->last_modeled = e->h_rep[0].v[R_MODELED];
-    e->last_hits = e->h_rep[0].v[R_HITS];
-    for (int k = 0; k < 3; ++k) {
-        float ms = 0.0f;
-        if (hipEventElapsedTime(&ms, e->ev[k], e->ev[k + 1]) == hipSuccess) {
-            e->last_ms[k] = ms;
-        }
-    }
+    e->last_modeled = e->h_out->rep.v[R_MODELED];
+    e->last_hits = e->h_out->rep.v[R_HITS];
+    note_times(e);
     if (out != nullptr) {
-        std::memcpy(out, e->h_rep, sizeof(DevReport));
+        std::memcpy(out, &e->h_out->rep, sizeof(DevReport));
         if (grouping) {
             // the joined records: modeled, read or write, their latencies
             out->grouped = h_frep[0];

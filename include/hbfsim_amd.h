@@ -382,9 +382,10 @@ int hbfsim_amd_set_state(hbfsim_context* context, const uint64_t* plane_busy,
                          uint64_t burst_state);
 /* Zeroes engine state, busy totals and the cumulative report. */
 int hbfsim_amd_reset(hbfsim_context* context);
-/* Average device time (ms) of each engine kernel over the last run,
- * measured with HIP events on the run's stream: [0] tile summary, [1] carry
- * chain, [2] apply.  Returns the number of kernels written. */
+/* Device time (ms) of each pass of the last run, from the start of its first
+ * kernel to the start of the next pass's by the GPU's wall clock: [0] tile
+ * summary, [1] carry chain, [2] apply (to the start of the report reduction).
+ * Returns the number of passes written. */
 int hbfsim_amd_last_kernel_ms(const hbfsim_context* context, float* ms,
                               int max_kernels);
 /* Diagnostics, no counterpart in the reference: the waves per SIMD the last
