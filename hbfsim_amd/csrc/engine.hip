@@ -396,6 +396,13 @@ __device__ __forceinline__ std::uint64_t readlane64(std::uint64_t v, int lane)
     return (static_cast<std::uint64_t>(hi) << 32) | lo;
 }
 
+// The lane below's value (0 in lane 0), by a DPP wave shift (wave_shr:1 = 0x138):
+// two VALU moves where a shuffle is two LDS operations.
+__device__ __forceinline__ std::uint64_t prev_lane64(std::uint64_t v)
+{
+    return dpp64<0x138, 0xF>(v);
+}
+
 // find_range_index (hbf_device.cuh:826-841): upper_bound(base) - 1 over the
 // sorted range table.  The top level runs over every `stride`-th base,
 // staged in LDS; the bottom level over at most `stride` bases in memory.
@@ -906,7 +913,8 @@ __device__ __forceinline__ Dec invalid_dec()
 // Transfer time of every lane's access.  When all modeled lanes move the same
 // byte count (the usual case) it is computed once, in scalar registers.
 __device__ __forceinline__ std::uint64_t lane_xfer(const KArgs& a, const std::uint64_t* xp,
-                                                   const Dec& d, bool m, std::uint64_t active)
+                                                   const Dec& d, bool m, std::uint64_t active,
+                                                   bool& uniform)
 {
     const int first = __ffsll(static_cast<long long>(active)) - 1;
     const std::uint32_t lo = static_cast<std::uint32_t>(
@@ -914,7 +922,8 @@ __device__ __forceinline__ std::uint64_t lane_xfer(const KArgs& a, const std::ui
     const std::uint32_t hi = static_cast<std::uint32_t>(__builtin_amdgcn_readlane(
         static_cast<int>(static_cast<std::uint32_t>(d.xbytes >> 32)), first));
     const std::uint64_t xb0 = (static_cast<std::uint64_t>(hi) << 32) | lo;
-    if (__ballot(m && d.xbytes != xb0) == 0) {
+    uniform = __ballot(m && d.xbytes != xb0) == 0;
+    if (uniform) {
         return xfer_ps(a, xb0);
     }
     return m ? xfer_ps_lds(a, xp, d.xbytes) : 0ull;
@@ -935,7 +944,7 @@ __device__ __forceinline__ Narrow narrow_check(const Dec& d, bool m, std::uint64
 {
     const int first = __ffsll(static_cast<long long>(active)) - 1;
     Narrow n;
-    n.origin = shfl64(d.issue, first);
+    n.origin = readlane64(d.issue, first);
     const bool bad = m && (d.issue < n.origin || d.issue - n.origin >= (1ull << 30) ||
                            svc1 >= (1ull << 24) || svc2 >= (1ull << 24));
     n.ok = __ballot(bad) == 0;
@@ -957,10 +966,12 @@ __device__ __forceinline__ bool run_step(const KArgs& a, const Dec& d, std::uint
     }
     const std::uint32_t page0 = static_cast<std::uint32_t>(
         __builtin_amdgcn_readlane(static_cast<int>(static_cast<std::uint32_t>(d.page1)), 0));
+    if (__ballot(static_cast<std::uint32_t>(d.page1) != page0) != 0) {
+        return false;  // (scattered streams leave here)
+    }
     const std::uint64_t bytes0 = readlane64(d.xbytes, 0);
-    const std::uint64_t prev = shfl64(d.issue, lane == 0 ? 0 : lane - 1);
-    const bool bad = static_cast<std::uint32_t>(d.page1) != page0 || (d.bits & 1u) != 0 ||
-                     d.xbytes != bytes0 || d.issue < prev;
+    const std::uint64_t prev = prev_lane64(d.issue);
+    const bool bad = (d.bits & 1u) != 0 || d.xbytes != bytes0 || (lane != 0 && d.issue < prev);
     return __ballot(bad) == 0;
 }
 
@@ -1513,7 +1524,8 @@ __device__ __forceinline__ LinBatchT<kRuns> empty_batch()
 // skipped.
 struct Group {
     int pred, leader, last;
-    bool uniform;  // every active lane has the same key (wave-uniform)
+    bool uniform;         // every active lane has the same key (wave-uniform)
+    std::uint64_t peers;  // the group's lanes (group_by only)
 };
 
 // Lanes whose key equals this lane's key, through a per-wave LDS table of
@@ -1543,7 +1555,8 @@ __device__ __forceinline__ Group group_by(std::uint32_t key, std::uint32_t bits,
                                           std::uint64_t* tab = nullptr)
 {
     const int first = __ffsll(static_cast<long long>(active)) - 1;
-    const std::uint32_t key0 = static_cast<std::uint32_t>(__shfl(static_cast<int>(key), first));
+    const std::uint32_t key0 =
+        static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), first));
     Group g;
     std::uint64_t peers;
     g.uniform = __ballot(m && key == key0) == active;
@@ -1558,7 +1571,81 @@ __device__ __forceinline__ Group group_by(std::uint32_t key, std::uint32_t bits,
     g.pred = (m && below) ? 63 - __clzll(below) : -1;
     g.leader = m ? __ffsll(static_cast<long long>(peers)) - 1 : lane;
     g.last = m ? 63 - __clzll(peers) : lane;
+    g.peers = peers;
     return g;
+}
+
+// General steps whose records all move the same byte count (the usual case).
+// The services of a group of lanes are then counts times constants, so a
+// lane's sums over the group's lanes before or after it are population counts
+// of the group's mask, not scans:
+//   miss, prog   lanes whose record senses (a read that misses) or programs.
+// What is left to scan is a maximum.  (Scans of (A, B) pairs by pointer
+// jumping, six LDS shuffles a round for the two chains, were 40% of the
+// summary pass on random records.)
+struct StepCounts {
+    std::uint64_t miss, prog;
+};
+
+__device__ __forceinline__ StepCounts count_services(bool counts, std::uint32_t bits, bool hit)
+{
+    StepCounts c;
+    c.miss = __ballot(counts && (bits & 1u) == 0 && !hit);
+    c.prog = __ballot(counts && (bits & 2u) != 0);
+    return c;
+}
+
+// Service of the group's lanes in `lanes`.
+__device__ __forceinline__ std::uint64_t count_service(const KArgs& a, const StepCounts& c,
+                                                       std::uint64_t lanes)
+{
+    std::uint64_t s =
+        static_cast<std::uint64_t>(static_cast<std::uint32_t>(__popcll(lanes & c.miss))) *
+        a.read_ps;
+    if (c.prog != 0) {
+        s += static_cast<std::uint64_t>(static_cast<std::uint32_t>(__popcll(lanes & c.prog))) *
+             a.program_ps;
+    }
+    return s;
+}
+
+// Prefix maxima of v1 and v2 along two lane groups, by pointer jumping (a
+// chain that is not wanted is passed pred -1 in every lane).
+__device__ __forceinline__ void group_prefix_max(std::uint32_t& v1, int p1, std::uint32_t& v2,
+                                                 int p2, int lane)
+{
+    for (int s = 0; s < 6; ++s) {
+        const bool any1 = __ballot(p1 >= 0) != 0, any2 = __ballot(p2 >= 0) != 0;
+        if (!any1 && !any2) {
+            break;
+        }
+        if (any1) {
+            const int s1 = p1 < 0 ? lane : p1;
+            const std::uint32_t x =
+                static_cast<std::uint32_t>(__shfl(static_cast<int>(v1), s1));
+            const int q = __shfl(p1, s1);
+            v1 = p1 >= 0 && x > v1 ? x : v1;
+            p1 = p1 >= 0 ? q : p1;
+        }
+        if (any2) {
+            const int s2 = p2 < 0 ? lane : p2;
+            const std::uint32_t x =
+                static_cast<std::uint32_t>(__shfl(static_cast<int>(v2), s2));
+            const int q = __shfl(p2, s2);
+            v2 = p2 >= 0 && x > v2 ? x : v2;
+            p2 = p2 >= 0 ? q : p2;
+        }
+    }
+}
+
+__device__ __forceinline__ void lds_add(std::uint64_t* p, std::uint64_t v)
+{
+    (void)__hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+__device__ __forceinline__ void lds_max(std::uint64_t* p, std::uint64_t v)
+{
+    (void)__hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Plane grouping of a batch of linear steps (lane k: step k, active lanes a
@@ -1586,6 +1673,7 @@ __device__ __forceinline__ Group group_plane_runs(const KArgs& a, std::uint32_t 
     const std::uint64_t upto = lane == 63 ? ~0ull : ((2ull << lane) - 1);
     const std::uint64_t later = heads & ~upto;
     Group g;
+    g.peers = 0;
     g.uniform = heads == 1ull;
     g.pred = (m && !head) ? lane - 1 : -1;
     g.leader = m ? 63 - __clzll(heads & upto) : lane;
@@ -2090,7 +2178,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
             step_records(st, lane, x, y);
             Dec d = valid ? decode<kRefresh>(a, fence, rc, x, y, base_ps, stab) : invalid_dec();
             {
-                const std::uint64_t prev = shfl64(d.issue, lane == 0 ? 0 : lane - 1);
+                const std::uint64_t prev = prev_lane64(d.issue);
                 const bool back = valid && d.issue < (lane == 0 ? last_issue : prev);
                 disorder = disorder || __ballot(back) != 0;
                 const std::uint64_t vmask = __ballot(valid);  // lanes 0 .. k
@@ -2106,7 +2194,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
             if (active == 0) {
                 continue;
             }
-            const std::uint64_t xfer = lane_xfer(a, xp, d, m, active);
+            bool same_x = false;
+            const std::uint64_t xfer = lane_xfer(a, xp, d, m, active, same_x);
             if (!kHits && run_step(a, d, active, lane)) {
                 const std::uint64_t W = run_channel_max(d, xfer, lane);
                 if (lane == 63) {
@@ -2155,6 +2244,43 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
                 prev1 = last_page;
             }
             const bool hit = kHits ? (m && hbit) : (a.slots != 0 && m && prev1 == page1);
+            // the leader's class; with given hits, bit 3 carries its hit
+            const std::uint32_t lbits = kHits && hit ? (d.bits | 8u) : d.bits;
+            if (!kRefresh && same_x) {
+                // Per group, (A, B) becomes (A + S, max(B + S, issue_k + S_k)
+                // over its lanes k), with S the service of all of them and S_k
+                // that of lane k and later: the group's last lane adds S, then
+                // every lane joins its own term, all by LDS atomics (a wave's
+                // LDS operations complete in issue order).
+                const StepCounts sc = count_services(m && !tfirst, d.bits, hit);
+                const std::uint64_t from = ~lanemask_lt(lane);
+                if (tfirst) {
+                    p_f1[pk] = page1;
+                    p_fi[pk] = d.issue;
+                    p_fc[pk] = static_cast<std::uint8_t>(lbits);
+                }
+                if (m && lane == gp.last) {
+                    const std::uint64_t S = count_service(a, sc, gp.peers);
+                    lds_add(&p_rA[pk], S);
+                    lds_add(&p_rB[pk], S);
+                    p_l1[pk] = page1;
+                }
+                if (m && !tfirst) {
+                    lds_max(&p_rB[pk], d.issue + count_service(a, sc, gp.peers & from));
+                }
+                if (m && lane == gc.last) {
+                    const std::uint64_t S =
+                        static_cast<std::uint64_t>(
+                            static_cast<std::uint32_t>(__popcll(gc.peers))) * xfer;
+                    lds_add(&c_A[ckey], S);
+                    lds_add(&c_B[ckey], S);
+                }
+                if (m) {
+                    lds_max(&c_B[ckey], d.issue + static_cast<std::uint64_t>(static_cast<std::uint32_t>(
+                                                      __popcll(gc.peers & from))) * xfer);
+                }
+                continue;
+            }
             const std::uint64_t svc = plane_service(a, d.bits, hit);
             std::uint64_t Ap = 0, Bp = 0;
             if (m && !tfirst) {
@@ -2167,8 +2293,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
             const std::uint32_t l1 =
                 static_cast<std::uint32_t>(__shfl(static_cast<int>(page1), gp.leader));
             const std::uint64_t li = shfl64(d.issue, gp.leader);
-            // the leader's class; with given hits, bit 3 carries its hit
-            const std::uint32_t lbits = kHits && hit ? (d.bits | 8u) : d.bits;
             const std::uint32_t lc =
                 static_cast<std::uint32_t>(__shfl(static_cast<int>(lbits), gp.leader));
             if (m && lane == gp.last) {
@@ -3635,7 +3759,8 @@ __device__ __forceinline__ void apply_tile(
                 std::uint8_t st = static_cast<std::uint8_t>(d.cls);
                 std::uint64_t done = 0;
                 if (!kHits && active != 0 && run_step(a, d, active, lane)) {
-                    const std::uint64_t xfer = lane_xfer(a, xp, d, m, active);
+                    bool same_x;
+                    const std::uint64_t xfer = lane_xfer(a, xp, d, m, active, same_x);
                     const std::uint64_t W = run_channel_max(d, xfer, lane);
                     const std::uint32_t page1 = static_cast<std::uint32_t>(d.page1);
                     const std::uint32_t pkey = d.plane;
@@ -3690,7 +3815,8 @@ __device__ __forceinline__ void apply_tile(
                     t.svc_sum += umax64(svc, xfer);
                     t.seq += 64;
                 } else if (active != 0) {
-                    const std::uint64_t xfer = lane_xfer(a, xp, d, m, active);
+                    bool same_x = false;
+                    const std::uint64_t xfer = lane_xfer(a, xp, d, m, active, same_x);
                     const std::uint32_t page1 = static_cast<std::uint32_t>(d.page1);
                     const std::uint32_t pkey = m ? d.plane : 0u;
                     const std::uint32_t ckey = m ? d.chan : 0u;
@@ -3707,18 +3833,66 @@ __device__ __forceinline__ void apply_tile(
                     }
                     const bool hit = kHits ? (m && hbit) : (a.slots != 0 && m && prev1 == page1);
                     const std::uint64_t svc = plane_service(a, d.bits, hit);
-                    std::uint64_t Ap = m ? svc : 0ull;
-                    std::uint64_t Bp = m ? d.issue + svc : 0ull;
-                    std::uint64_t Ac = m ? xfer : 0ull;
-                    std::uint64_t Bc = m ? d.issue + xfer : 0ull;
-                    if (a.contention) {
-                        scan_pair(gp, Ap, Bp, gc, Ac, Bc, d, m, active, svc, xfer, lane);
+                    std::uint64_t pd, cd;
+                    const StepCounts sc = count_services(m, d.bits, hit);
+                    const std::uint64_t origin = readlane64(
+                        d.issue, __ffsll(static_cast<long long>(active)) - 1);
+                    const std::uint64_t most =
+                        static_cast<std::uint64_t>(static_cast<std::uint32_t>(
+                            __popcll(sc.miss))) * a.read_ps +
+                        static_cast<std::uint64_t>(static_cast<std::uint32_t>(
+                            __popcll(sc.prog))) * a.program_ps;
+                    const bool small =
+                        !kRefresh && same_x && most < (1ull << 30) && xfer < (1ull << 24) &&
+                        __ballot(m && d.issue - origin >= (1ull << 30)) == 0;
+                    if (small) {
+                        // lane i of a group completes at max(busy, max over
+                        // k <= i of (issue_k - E_k)) + E_i + its service, with
+                        // E the service of the group's lanes before: where no
+                        // lane's issue time passes busy + E the maximum is busy,
+                        // else it is a prefix maximum of issue - E, in 32 bits
+                        // from the step's first issue time
+                        const std::uint64_t below = lanemask_lt(lane);
+                        const std::uint32_t Ep = static_cast<std::uint32_t>(
+                            count_service(a, sc, gp.peers & below));
+                        const std::uint32_t x32 = static_cast<std::uint32_t>(xfer);
+                        const std::uint32_t Ec =
+                            x32 * static_cast<std::uint32_t>(__popcll(gc.peers & below));
+                        const bool wp = a.contention != 0 &&
+                                        __ballot(m && d.issue > pbusy + Ep) != 0;
+                        const bool wc = __ballot(m && d.issue > cbusy + Ec) != 0;
+                        std::uint64_t tp = pbusy, tc = cbusy;
+                        if (wp || wc) {
+                            const std::uint32_t rel =
+                                m ? static_cast<std::uint32_t>(d.issue - origin) : 0u;
+                            const std::uint32_t most32 = static_cast<std::uint32_t>(most);
+                            const std::uint32_t c64 = x32 * 64u;
+                            std::uint32_t vp = rel + most32 - Ep, vc = rel + c64 - Ec;
+                            group_prefix_max(vp, wp ? gp.pred : -1, vc, wc ? gc.pred : -1, lane);
+                            // (origin - most can only pass below zero where the
+                            // maximum is another lane's: compare before taking off)
+                            if (wp) {
+                                tp = origin + vp > pbusy + most32 ? origin + vp - most32 : pbusy;
+                            }
+                            if (wc) {
+                                tc = origin + vc > cbusy + c64 ? origin + vc - c64 : cbusy;
+                            }
+                        }
+                        pd = a.contention ? (m ? tp + Ep + svc : 0ull) : d.issue + svc;
+                        cd = m ? tc + Ec + xfer : 0ull;
                     } else {
-                        scan_group(gc, Ac, Bc, lane);
+                        std::uint64_t Ap = m ? svc : 0ull;
+                        std::uint64_t Bp = m ? d.issue + svc : 0ull;
+                        std::uint64_t Ac = m ? xfer : 0ull;
+                        std::uint64_t Bc = m ? d.issue + xfer : 0ull;
+                        if (a.contention) {
+                            scan_pair(gp, Ap, Bp, gc, Ac, Bc, d, m, active, svc, xfer, lane);
+                        } else {
+                            scan_group(gc, Ac, Bc, lane);
+                        }
+                        pd = a.contention ? (m ? umax64(pbusy + Ap, Bp) : 0ull) : d.issue + svc;
+                        cd = m ? umax64(cbusy + Ac, Bc) : 0ull;
                     }
-                    const std::uint64_t pd =
-                        a.contention ? (m ? umax64(pbusy + Ap, Bp) : 0ull) : d.issue + svc;
-                    const std::uint64_t cd = m ? umax64(cbusy + Ac, Bc) : 0ull;
                     if (m && lane == gp.last) {
                         if (a.contention) {
                             p_busy[pkey] = pd;
