@@ -102,6 +102,9 @@ struct KArgs {
     const std::uint32_t* r_meta;  // mode | permissions << 8
     const std::uint32_t* r_id;
     std::uint32_t r_count, r_stride, r_nfence;
+    // the per-record passes hold the whole range table in LDS (RangeView);
+    // set where it fits the table's packed form and costs the passes no waves
+    std::uint32_t r_lds;
     // geometry
     std::uint32_t Rp, Rc;           // planes, channels (resource counts)
     std::uint32_t W, D, P;
@@ -403,16 +406,30 @@ __device__ __forceinline__ std::uint64_t prev_lane64(std::uint64_t v)
     return dpp64<0x138, 0xF>(v);
 }
 
+// The range table as a kernel sees it: the fences in LDS and, where the whole
+// table is held there too (KArgs::r_lds), each range's length | mode << 56 |
+// permissions << 60, its first media page and, in hybrid runs, its id.  A
+// lookup then makes no vector-memory load: those made a step of records spread
+// over several ranges wait for the whole record pipeline.
+struct RangeView {
+    const std::uint64_t* fence;
+    const std::uint64_t* len = nullptr;
+    const std::uint32_t* page0 = nullptr;
+    const std::uint32_t* id = nullptr;
+    __device__ __forceinline__ RangeView(const std::uint64_t* f) : fence(f) {}
+};
+constexpr std::uint64_t kRangeLenMask = (1ull << 56) - 1;
+
 // find_range_index (hbf_device.cuh:826-841): upper_bound(base) - 1 over the
 // sorted range table.  The top level runs over every `stride`-th base,
 // staged in LDS; the bottom level over at most `stride` bases in memory.
-__device__ __forceinline__ std::uint32_t find_range(const KArgs& a, const std::uint64_t* fence,
+__device__ __forceinline__ std::uint32_t find_range(const KArgs& a, const RangeView& rv,
                                                     std::uint64_t addr)
 {
     std::uint32_t lo = 0, hi = a.r_nfence;
     while (lo < hi) {
         const std::uint32_t mid = (lo + hi) >> 1;
-        if (fence[mid] <= addr) {
+        if (rv.fence[mid] <= addr) {
             lo = mid + 1;
         } else {
             hi = mid;
@@ -420,6 +437,9 @@ __device__ __forceinline__ std::uint32_t find_range(const KArgs& a, const std::u
     }
     if (lo == 0) {
         return a.r_count;
+    }
+    if (a.r_lds != 0) {
+        return lo - 1;  // every base is a fence
     }
     const std::uint32_t start = (lo - 1) * a.r_stride;
     std::uint32_t end = start + a.r_stride;
@@ -789,7 +809,7 @@ __device__ __forceinline__ std::uint32_t dec_op(std::uint32_t bits)
 // into); the other streams keep the branch out of the hot loop.  `stab`:
 // the wave's stripe table (fill_stripe_table), when the run keeps one.
 template <bool kRefresh, bool kUniform = false>
-__device__ __forceinline__ Dec decode(const KArgs& a, const std::uint64_t* fence, RangeCache& rc,
+__device__ __forceinline__ Dec decode(const KArgs& a, const RangeView& fence, RangeCache& rc,
                                       const uint4& x, const uint4& y, std::uint64_t base_ps,
                                       const std::uint32_t* stab = nullptr)
 {
@@ -824,6 +844,26 @@ __device__ __forceinline__ Dec decode(const KArgs& a, const std::uint64_t* fence
             // wave-uniform record: keep the range in scalar registers
             idx = static_cast<std::uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(idx)));
         }
+        if (a.r_lds != 0) {
+            const std::uint64_t base = idx == a.r_count ? 0ull : fence.fence[idx];
+            const std::uint64_t lm = idx == a.r_count ? 0ull : fence.len[idx];
+            if (idx == a.r_count || addr - base >= (lm & kRangeLenMask)) {
+                const std::uint32_t succ = idx == a.r_count ? 0u : idx + 1u;
+                d.cls = bytes > 0xffffffffull ||
+                                (succ < a.r_count &&
+                                 overlaps(fence.fence[succ], fence.len[succ] & kRangeLenMask, addr,
+                                          bytes))
+                            ? kClsUnsupported
+                            : kClsBypass;
+                return d;
+            }
+            rc.base = base;
+            rc.end = base + (lm & kRangeLenMask);
+            rc.file_offset = static_cast<std::uint64_t>(fence.page0[idx]) << a.page_shift;
+            rc.meta = static_cast<std::uint32_t>(lm >> 56) & 0xfu;
+            rc.meta |= static_cast<std::uint32_t>(lm >> 60) << 8;
+            rc.id = a.hybrid != 0 ? fence.id[idx] : 0u;
+        } else {
         if (idx == a.r_count || addr < a.r_base[idx] ||
             addr - a.r_base[idx] >= a.r_length[idx]) {
             const std::uint32_t succ = idx == a.r_count ? 0u : idx + 1u;
@@ -842,6 +882,7 @@ __device__ __forceinline__ Dec decode(const KArgs& a, const std::uint64_t* fence
         rc.id = a.r_id[idx];
         if (!kUniform) {
             wait_vector_loads();
+        }
         }
     }
     const std::uint32_t mode = rc.meta & 0xffu;
@@ -1010,13 +1051,13 @@ __device__ __forceinline__ std::uint32_t rl32(std::uint32_t v, int k)
 // The range and page checks of a step whose 64 records already follow
 // record 0 (xu: its address and bytes, yu: its issue time and operation).
 template <bool kRefresh>
-__device__ __forceinline__ bool linear_tail(const KArgs& a, const std::uint64_t* fence,
+__device__ __forceinline__ bool linear_tail(const KArgs& a, const RangeView& fence,
                                             RangeCache& rcu, const uint4& xu, const uint4& yu,
                                             std::uint64_t base_ps, std::uint32_t& page1,
                                             std::uint64_t& issue0, std::uint32_t& bytes0);
 
 template <bool kRefresh>
-__device__ __forceinline__ bool linear_detect(const KArgs& a, const std::uint64_t* fence,
+__device__ __forceinline__ bool linear_detect(const KArgs& a, const RangeView& fence,
                                               RangeCache& rcu, const Step32& st,
                                               std::uint64_t base_ps, bool full, int lane,
                                               std::uint32_t& page1, std::uint64_t& issue0,
@@ -1052,7 +1093,7 @@ __device__ __forceinline__ bool linear_detect(const KArgs& a, const std::uint64_
 
 // A packed step: lane l checks its own record against record 0.
 template <bool kRefresh>
-__device__ __forceinline__ bool linear_detect(const KArgs& a, const std::uint64_t* fence,
+__device__ __forceinline__ bool linear_detect(const KArgs& a, const RangeView& fence,
                                               RangeCache& rcu, const Step16& st,
                                               std::uint64_t base_ps, bool full, int lane,
                                               std::uint32_t& page1, std::uint64_t& issue0,
@@ -1080,7 +1121,7 @@ __device__ __forceinline__ bool linear_detect(const KArgs& a, const std::uint64_
 }
 
 template <bool kRefresh>
-__device__ __forceinline__ bool linear_tail(const KArgs& a, const std::uint64_t* fence,
+__device__ __forceinline__ bool linear_tail(const KArgs& a, const RangeView& fence,
                                             RangeCache& rcu, const uint4& xu, const uint4& yu,
                                             std::uint64_t base_ps, std::uint32_t& page1,
                                             std::uint64_t& issue0, std::uint32_t& bytes0)
@@ -1129,7 +1170,7 @@ struct LinStep {
 // address lies outside the wave-uniform range cache refills it through the
 // full classification (one call site for both runs).
 template <bool kRefresh>
-__device__ __forceinline__ bool linear_detect_split(const KArgs& a, const std::uint64_t* fence,
+__device__ __forceinline__ bool linear_detect_split(const KArgs& a, const RangeView& fence,
                                                     RangeCache& rcu, const Step16& st,
                                                     std::uint64_t base_ps, bool full, int lane,
                                                     LinStep& ls)
@@ -1221,7 +1262,7 @@ __device__ __forceinline__ bool linear_detect_split(const KArgs& a, const std::u
 // The step detection of a record form: packed steps may be split (kSplit);
 // otherwise, and for 32-byte records, steps are whole linear steps or none.
 template <bool kRefresh, bool kSplit>
-__device__ __forceinline__ bool detect_step(const KArgs& a, const std::uint64_t* fence,
+__device__ __forceinline__ bool detect_step(const KArgs& a, const RangeView& fence,
                                             RangeCache& rcu, const Step16& st,
                                             std::uint64_t base_ps, bool full, int lane,
                                             LinStep& ls)
@@ -1239,7 +1280,7 @@ __device__ __forceinline__ bool detect_step(const KArgs& a, const std::uint64_t*
 }
 
 template <bool kRefresh, bool kSplit>
-__device__ __forceinline__ bool detect_step(const KArgs& a, const std::uint64_t* fence,
+__device__ __forceinline__ bool detect_step(const KArgs& a, const RangeView& fence,
                                             RangeCache& rcu, const Step32& st,
                                             std::uint64_t base_ps, bool full, int lane,
                                             LinStep& ls)
@@ -1270,13 +1311,13 @@ struct GroupLin {
 };
 
 template <bool kRefresh, int D>
-__device__ __forceinline__ bool group_tail(const KArgs& a, const std::uint64_t* fence,
+__device__ __forceinline__ bool group_tail(const KArgs& a, const RangeView& fence,
                                            RangeCache& rcu, std::uint64_t base_ps,
                                            const uint4& xu, std::uint32_t op0, std::uint32_t vlo,
                                            std::uint32_t vhi, int lane, GroupLin<D>& gl);
 
 template <bool kRefresh, int D>
-__device__ __forceinline__ bool group_linear(const KArgs& a, const std::uint64_t* fence,
+__device__ __forceinline__ bool group_linear(const KArgs& a, const RangeView& fence,
                                              RangeCache& rcu, const RecordPipeT<D>& pipe,
                                              std::uint64_t base_ps, int lane, GroupLin<D>& gl)
 {
@@ -1319,7 +1360,7 @@ __device__ __forceinline__ bool group_linear(const KArgs& a, const std::uint64_t
 
 // A packed group: lane l checks its own record of every step.
 template <bool kRefresh, int D>
-__device__ __forceinline__ bool group_linear(const KArgs& a, const std::uint64_t* fence,
+__device__ __forceinline__ bool group_linear(const KArgs& a, const RangeView& fence,
                                              RangeCache& rcu, const PackedPipeT<D>& pipe,
                                              std::uint64_t base_ps, int lane, GroupLin<D>& gl)
 {
@@ -1357,7 +1398,7 @@ __device__ __forceinline__ bool group_linear(const KArgs& a, const std::uint64_t
 // vlo, vhi: lane j < D holds step j's issue time), and the group's step
 // values, lane j checking and holding step j.
 template <bool kRefresh, int D>
-__device__ __forceinline__ bool group_tail(const KArgs& a, const std::uint64_t* fence,
+__device__ __forceinline__ bool group_tail(const KArgs& a, const RangeView& fence,
                                            RangeCache& rcu, std::uint64_t base_ps,
                                            const uint4& xu, std::uint32_t op0, std::uint32_t vlo,
                                            std::uint32_t vhi, int lane, GroupLin<D>& gl)
@@ -1733,6 +1774,66 @@ __device__ __forceinline__ std::uint64_t plane_service(const KArgs& a, std::uint
     return (bits & 2u) ? a.program_ps : 0ull;
 }
 
+// The range table in LDS (a.r_lds): at most kLdsRanges ranges, two per lane,
+// loaded and stored in two halves as the fences are.
+constexpr std::uint32_t kLdsRanges = 128;
+constexpr int kRangesPerLane = static_cast<int>(kLdsRanges) / kWave;
+
+struct RangeRegs {
+    std::uint64_t len[kRangesPerLane], off[kRangesPerLane];
+    std::uint32_t meta[kRangesPerLane], id[kRangesPerLane];
+};
+
+__host__ __device__ __forceinline__ std::size_t range_lds_bytes(const KArgs& a)
+{
+    return a.r_lds != 0 ? 8ull * a.r_count + (a.hybrid != 0 ? 8ull : 4ull) * a.r_count : 0ull;
+}
+
+__device__ __forceinline__ RangeRegs fetch_ranges(const KArgs& a, int lane)
+{
+    RangeRegs r{};
+    if (a.r_lds != 0) {
+#pragma unroll
+        for (int k = 0; k < kRangesPerLane; ++k) {
+            const std::uint32_t j = static_cast<std::uint32_t>(k * kWave + lane);
+            if (j < a.r_count) {
+                r.len[k] = a.r_length[j];
+                r.off[k] = a.r_file_offset[j];
+                r.meta[k] = a.r_meta[j];
+                r.id[k] = a.hybrid != 0 ? a.r_id[j] : 0u;
+            }
+        }
+    }
+    return r;
+}
+
+// Writes the table at `at` (8-byte aligned) and completes the view.
+__device__ __forceinline__ void store_ranges(const KArgs& a, const RangeRegs& r, void* at,
+                                             RangeView& rv, int lane)
+{
+    if (a.r_lds == 0) {
+        return;
+    }
+    auto* len = static_cast<std::uint64_t*>(at);
+    auto* page0 = reinterpret_cast<std::uint32_t*>(len + a.r_count);
+    auto* id = page0 + a.r_count;
+    rv.len = len;
+    rv.page0 = page0;
+    rv.id = id;
+#pragma unroll
+    for (int k = 0; k < kRangesPerLane; ++k) {
+        const std::uint32_t j = static_cast<std::uint32_t>(k * kWave + lane);
+        if (j < a.r_count) {
+            len[j] = r.len[k] | (static_cast<std::uint64_t>(r.meta[k] & 0xfu) << 56) |
+                     (static_cast<std::uint64_t>((r.meta[k] >> 8) & 0xfu) << 60);
+            page0[j] = static_cast<std::uint32_t>(r.off[k] >> a.page_shift);
+            if (a.hybrid != 0) {
+                id[j] = r.id[k];
+            }
+        }
+    }
+}
+
 // The range fences (r_nfence <= kMaxFences), a lane's share in registers:
 // fetch_fences issues every load before store_fences writes any of them, so
 // a tile's set-up waits for memory once rather than once per 64 fences.
@@ -1997,6 +2098,10 @@ __host__ __device__ __forceinline__ std::size_t summary_stripe_offset(const KArg
 {
     return summary_match_offset(a) + (a.match_lds ? 8ull * (a.Rp + a.Rc) : 0ull);
 }
+__host__ __device__ __forceinline__ std::size_t summary_range_offset(const KArgs& a)
+{
+    return (summary_stripe_offset(a) + (a.stripe_lds ? 4ull * a.Rp : 0ull) + 7ull) & ~7ull;
+}
 
 // Summary pass.  Per plane the tile keeps: the first record (page, issue,
 // class), the (max,+) map of the records after it, and the last page; per
@@ -2012,8 +2117,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
     extern __shared__ std::uint64_t sm[];
     // per-plane state at slot pslot(plane) of plane_slots(a) entries
     const std::uint32_t rpp = plane_slots(a);
-    std::uint64_t* fence = sm;
-    std::uint64_t* p_fi = fence + a.r_nfence;
+    RangeView fence(sm);
+    std::uint64_t* p_fi = sm + a.r_nfence;
     std::uint64_t* p_rA = p_fi + rpp;
     std::uint64_t* p_rB = p_rA + rpp;
     std::uint64_t* c_A = p_rB + rpp;
@@ -2034,6 +2139,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
     stamp_start(a, 0);
     // set-up loads and the first group of records are in flight together
     const FenceRegs fr = fetch_fences(a, lane);
+    const RangeRegs rr = fetch_ranges(a, lane);
     const std::uint64_t xv = fetch_xfer(a, lane);
     // The record before the tile: every record's issue time must be at least
     // its predecessor's for stream position to be the service order.  Steps
@@ -2058,7 +2164,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
     using Pipe = std::conditional_t<kPacked, PackedPipeT<kDepth>, RecordPipeT<kDepth>>;
     Pipe pipe;
     pipe.issue(rec, begin, end, lane);
-    store_fences(a, fr, fence, lane);
+    store_fences(a, fr, sm, lane);
+    store_ranges(a, rr, reinterpret_cast<unsigned char*>(sm) + summary_range_offset(a), fence,
+                 lane);
     store_xfer(xp, xv, lane);
     for (std::uint32_t r = lane; r < rpp; r += kWave) {
         p_fi[r] = 0;
@@ -3426,6 +3534,10 @@ __host__ __device__ __forceinline__ std::size_t apply_stripe_offset(const KArgs&
 {
     return apply_match_offset(a) + (a.match_lds ? 8ull * (a.Rp + a.Rc) : 0ull);
 }
+__host__ __device__ __forceinline__ std::size_t apply_range_offset(const KArgs& a)
+{
+    return (apply_stripe_offset(a) + (a.stripe_lds ? 4ull * a.Rp : 0ull) + 7ull) & ~7ull;
+}
 
 // A tile's plane carry-ins are packed like its summaries: word w of the
 // mask covers planes [64 w, 64 w + 64), so lane l reads bit l of each word.
@@ -3574,8 +3686,8 @@ __device__ __forceinline__ void apply_tile(
     DevReport* tile_rep, const std::uint8_t* hits, const StepDesc* desc, std::uint64_t* sm,
     std::uint64_t* xp)
 {
-    std::uint64_t* fence = sm;
-    std::uint64_t* p_busy = fence + a.r_nfence;
+    RangeView fence(sm);
+    std::uint64_t* p_busy = sm + a.r_nfence;
     std::uint64_t* c_busy = p_busy + a.Rp;
     std::uint32_t* p_tag = reinterpret_cast<std::uint32_t*>(c_busy + a.Rc);
     const int lane = threadIdx.x;
@@ -3596,6 +3708,7 @@ __device__ __forceinline__ void apply_tile(
     std::uint64_t* mt_c = a.match_lds ? mt_p + a.Rp : nullptr;
     const std::size_t tsteps = (end - begin + kWave - 1) / kWave;
     const FenceRegs fr = fetch_fences(a, lane);
+    const RangeRegs rr = fetch_ranges(a, lane);
     const std::uint64_t xv = fetch_xfer(a, lane);
     constexpr int kDescPerLane = static_cast<int>(kStageSteps) / kWave;
     StepDesc dv[kDescPerLane];
@@ -3609,7 +3722,8 @@ __device__ __forceinline__ void apply_tile(
     }
     load_plane_carry(a, tmask, pcarry, tile, p_busy, p_tag, lane);
     load_chan_carry(a, ccarry, tile, c_busy, lane);
-    store_fences(a, fr, fence, lane);
+    store_fences(a, fr, sm, lane);
+    store_ranges(a, rr, reinterpret_cast<unsigned char*>(sm) + apply_range_offset(a), fence, lane);
     store_xfer(xp, xv, lane);
     if (a.match_lds) {
         for (std::uint32_t r = lane; r < a.Rp + a.Rc; r += kWave) {
@@ -4385,6 +4499,7 @@ struct engine {
     // ranges
     std::vector<range_rec> ranges;
     bool ranges_dirty{true};
+    bool ranges_pack{false};  // the range table fits its packed form in LDS
     std::uint64_t* d_r_base{nullptr};
     std::uint64_t* d_r_length{nullptr};
     std::uint64_t* d_r_offset{nullptr};
@@ -4662,6 +4777,14 @@ int upload_ranges(engine* e, hipStream_t stream)
                                                                   kMaxFences);
     a.r_nfence = count == 0 ? 0u
                             : static_cast<std::uint32_t>((count + a.r_stride - 1) / a.r_stride);
+    // the packed form of the table in LDS (store_ranges)
+    e->ranges_pack = count != 0 && count <= kLdsRanges;
+    for (std::size_t i = 0; i < count; ++i) {
+        e->ranges_pack = e->ranges_pack && length[i] <= kRangeLenMask &&
+                         (offset[i] >> a.page_shift) <= 0xffffffffull &&
+                         (offset[i] & ((1ull << a.page_shift) - 1)) == 0 &&
+                         e->ranges[i].mode <= 0xfu && e->ranges[i].permissions <= 0xfu;
+    }
     e->ranges_dirty = false;
     return HBFSIM_OK;
 }
@@ -5576,15 +5699,9 @@ __global__ __launch_bounds__(64) void k_k2_hits(KArgs a, const hbf_record32* rec
     }
 }
 
-std::size_t lds_summary(const KArgs& a)
-{
-    return summary_stripe_offset(a) + (a.stripe_lds ? 4ull * a.Rp : 0ull);
-}
+std::size_t lds_summary(const KArgs& a) { return summary_range_offset(a) + range_lds_bytes(a); }
 
-std::size_t lds_apply(const KArgs& a)
-{
-    return apply_stripe_offset(a) + (a.stripe_lds ? 4ull * a.Rp : 0ull);
-}
+std::size_t lds_apply(const KArgs& a) { return apply_range_offset(a) + range_lds_bytes(a); }
 
 // The lane-matching tables go where they cost neither per-record pass any
 // waves per CU (gfx950: 160 KB of LDS per CU, four SIMDs; both passes run at
@@ -5610,7 +5727,7 @@ hipError_t allow_lds(F* kernel, std::size_t bytes)
                                static_cast<int>(bytes));
 }
 
-void choose_match(KArgs& a)
+void choose_match(KArgs& a, bool ranges_pack)
 {
     constexpr std::size_t kLdsPerCu = kLdsPerCuBytes;
     constexpr std::size_t kMaxWaves = 4 * kSimdsPerCu;
@@ -5620,6 +5737,14 @@ void choose_match(KArgs& a)
     };
     a.match_lds = 0;
     a.stripe_lds = 0;
+    a.r_lds = 0;
+    if (ranges_pack) {
+        const std::size_t s0 = lds_summary(a), p0 = lds_apply(a);
+        a.r_lds = 1;
+        if (waves(lds_summary(a)) < waves(s0) || waves(lds_apply(a)) < waves(p0)) {
+            a.r_lds = 0;
+        }
+    }
     const std::size_t s0 = lds_summary(a), p0 = lds_apply(a);
     a.match_lds = 1;
     if (waves(lds_summary(a)) < waves(s0) || waves(lds_apply(a)) < waves(p0)) {
@@ -5858,10 +5983,11 @@ int run_empirical(engine* e, const hbf_record32* d_rec, std::size_t n, std::uint
 
 // Per-record page-buffer hits for two registers per plane, and the tags the
 // run leaves behind (host array [2 * planes]).  d_hits: n bytes.
-int k2_hits(engine* e, const KArgs& a, const hbf_record32* d_rec, std::size_t n,
+int k2_hits(engine* e, KArgs a, const hbf_record32* d_rec, std::size_t n,
             std::uint64_t base_ps, std::size_t ntiles, hipStream_t stream, std::uint8_t* d_hits,
             std::vector<std::uint64_t>& tags_out)
 {
+    a.r_lds = 0;  // these passes look ranges up through the fences
     const std::uint32_t rp = a.Rp;
     std::vector<std::uint64_t> tags(2ull * rp);
     hipError_t err = hipMemcpyAsync(tags.data(), e->d_ptag, tags.size() * 8,
@@ -6363,7 +6489,7 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
     if (packed) {
         a.tile_split = sc.tsplit;  // the summary pass marks tiles with split steps
     }
-    choose_match(a);
+    choose_match(a, e->ranges_pack);
     const std::size_t lds_a = lds_summary(a), lds_c = lds_apply(a);
     if (lds_a > kLdsPerBlockBytes || lds_c > kLdsPerBlockBytes) {
         return HBFSIM_UNSUPPORTED;
@@ -6387,8 +6513,10 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
         if (err == hipSuccess) err = hipMemsetAsync(d_frep, 0, 64, stream);
         if (err == hipSuccess) {
             const std::size_t nl = (n + kLeadSpan - 1) / kLeadSpan;
+            KArgs la = a;
+            la.r_lds = 0;  // k_lead looks ranges up through the fences
             hipLaunchKernelGGL(k_lead, dim3(static_cast<unsigned>(nl)), dim3(kWave),
-                               static_cast<std::size_t>(a.r_nfence) * 8, stream, a,
+                               static_cast<std::size_t>(a.r_nfence) * 8, stream, la,
                                static_cast<const hbf_record32*>(d_rec), n, d_lead, d_gerr);
             err = hipGetLastError();
         }
