@@ -92,6 +92,7 @@ struct alignas(16) SplitDesc {
     std::uint32_t pad;
 };
 constexpr std::uint32_t kSplitFlag = 0x80000000u;
+constexpr std::uint8_t kTilePlain = 2;
 
 // Kernel arguments, passed by value.
 struct KArgs {
@@ -105,6 +106,7 @@ struct KArgs {
     // the per-record passes hold the whole range table in LDS (RangeView);
     // set where it fits the table's packed form and costs the passes no waves
     std::uint32_t r_lds;
+    std::uint32_t r_top;  // the largest power of two up to r_count (r_lds only)
     // geometry
     std::uint32_t Rp, Rc;           // planes, channels (resource counts)
     std::uint32_t W, D, P;
@@ -152,8 +154,10 @@ struct KArgs {
     std::uint32_t* disorder;
     // per tile, written by the summary pass of packed records: 1 when the
     // tile holds a split step (the apply pass then takes its split-capable
-    // body), else 0; null when the run takes no linear batches
+    // body), kTilePlain when the scattered-record passes take it, else 0; null
+    // for 32-byte records unless those passes run
     std::uint8_t* tile_split;
+    std::uint32_t mixed;  // the scattered-record passes ran before: skip their tiles
     // start times of the summary pass, the carry chain and the apply pass
     // (stamp_start)
     std::uint64_t* stamp;
@@ -2136,7 +2140,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
     const std::size_t tile = blockIdx.x;
     const std::size_t begin = tile * a.tile;
     const std::size_t end = begin + a.tile < n ? begin + a.tile : n;
-    stamp_start(a, 0);
+    if (a.mixed != 0 && a.tile_split[tile] == kTilePlain) {
+        return;  // k_plain_summary took it
+    }
+    if (a.mixed == 0) {
+        stamp_start(a, 0);
+    }
     // set-up loads and the first group of records are in flight together
     const FenceRegs fr = fetch_fences(a, lane);
     const RangeRegs rr = fetch_ranges(a, lane);
@@ -4115,14 +4124,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWide ? 4 : 
 {
     extern __shared__ std::uint64_t sm[];
     __shared__ std::uint64_t xp[33];
-    stamp_start(a, 2);
+    if (a.mixed == 0) {
+        stamp_start(a, 2);
+    }
     // a stream that went back in time is timed again from a sorted copy:
     // nothing of this run is kept (8.4M records: 190 us not spent here)
     if (a.disorder != nullptr && *a.disorder != 0u) {
         return;
     }
+    const std::uint8_t kind = a.tile_split != nullptr ? a.tile_split[blockIdx.x] : 0;
+    if (kind == kTilePlain) {
+        return;  // k_plain_apply took it
+    }
     if constexpr (kPacked) {
-        if (a.tile_split != nullptr && a.tile_split[blockIdx.x] != 0) {
+        if (kind != 0) {
             apply_tile<kRefresh, kHits, kStaged, kPacked, true, kWide>(
                 a, rec, n, base_ps, pcarry, tmask, ccarry, tile_seq, completion, status, tile_rep,
                 hits, desc, sm, xp);
@@ -4133,6 +4148,575 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWide ? 4 : 
                                                                 ccarry, tile_seq, completion,
                                                                 status, tile_rep, hits, desc, sm,
                                                                 xp);
+}
+
+// ---- scattered records -----------------------------------------------------
+//
+// k_summary and k_apply are built around runs of linear steps; what they hold
+// for those costs a step of scattered records registers, spilled scalars and
+// occupancy.  Streams over geometries of power-of-two axes whose range table
+// fits LDS (plain_run) have two kernels of their own with the same inputs
+// and outputs and none of that: k_plain_summary takes the tiles that do not
+// look like runs of lines and leaves the others to k_summary, and
+// k_plain_apply replays those it took.
+//
+// What bounds them is the number of instructions a step issues (k_summary: 515
+// vector, 256 scalar and 86 branches on records spread over 37 ranges), so a
+// step is decoded without divergence in 32-bit page arithmetic, its groups
+// come from a 32-slot LDS table and a ballot per further key bit, and sums over
+// a group are population counts of its mask (count_services).
+constexpr std::uint32_t kMatchSlots = 32;
+
+// LDS of both kernels, in this order: the range table (bases, lengths), the
+// per-plane and per-channel 64-bit words, the match table, then 32-bit words.
+struct PlainLds {
+    std::uint64_t* fence;
+    std::uint64_t* len;
+    std::uint64_t* w64;       // kernel's own 64-bit state
+    std::uint64_t* tab;       // [kMatchSlots], zero between uses
+    std::uint32_t* page0;
+    std::uint32_t* w32;       // kernel's own 32-bit state
+};
+
+__host__ __device__ __forceinline__ std::size_t plain_lds_bytes(const KArgs& a, std::size_t w64,
+                                                                std::size_t w32)
+{
+    return 8ull * (2ull * a.r_count + w64 + kMatchSlots) + 4ull * (a.r_count + w32);
+}
+
+__host__ __device__ __forceinline__ std::size_t plain_summary_lds(const KArgs& a)
+{
+    const std::size_t rp = plane_slots(a);
+    return plain_lds_bytes(a, 3 * rp + 2ull * a.Rc, 2 * rp) + rp;
+}
+
+__host__ __device__ __forceinline__ std::size_t plain_apply_lds(const KArgs& a)
+{
+    return plain_lds_bytes(a, static_cast<std::size_t>(a.Rp) + a.Rc, a.Rp);
+}
+
+__device__ __forceinline__ PlainLds plain_layout(const KArgs& a, std::uint64_t* sm,
+                                                 std::size_t w64)
+{
+    PlainLds l;
+    l.fence = sm;
+    l.len = l.fence + a.r_count;
+    l.w64 = l.len + a.r_count;
+    l.tab = l.w64 + w64;
+    l.page0 = reinterpret_cast<std::uint32_t*>(l.tab + kMatchSlots);
+    l.w32 = l.page0 + a.r_count;
+    return l;
+}
+
+__device__ __forceinline__ void plain_load(const KArgs& a, const PlainLds& l, int lane)
+{
+#pragma unroll
+    for (int k = 0; k < kRangesPerLane; ++k) {
+        const std::uint32_t j = static_cast<std::uint32_t>(k * kWave + lane);
+        if (j < a.r_count) {
+            l.fence[j] = a.r_base[j];
+            const std::uint32_t meta = a.r_meta[j];
+            l.len[j] = a.r_length[j] | (static_cast<std::uint64_t>((meta >> 8) & 0xfu) << 60);
+            l.page0[j] = static_cast<std::uint32_t>(a.r_file_offset[j] >> a.page_shift);
+        }
+    }
+    if (lane < static_cast<int>(kMatchSlots)) {
+        l.tab[lane] = 0;
+    }
+}
+
+// One record (x: address, bytes; y: issue time, flags), classified as decode()
+// does for reads and writes.
+struct PlainRec {
+    std::uint64_t issue;
+    std::uint32_t cls, bits, page1, plane, chan, bytes;
+};
+
+__device__ __forceinline__ PlainRec plain_record(const KArgs& a, const PlainLds& l,
+                                                 const uint4& x, const uint4& y, bool valid,
+                                                 std::uint64_t base_ps)
+{
+    const std::uint64_t addr = x.x | (static_cast<std::uint64_t>(x.y) << 32);
+    const std::uint32_t bytes = x.z;
+    const bool huge = x.w != 0;  // 2^32 bytes or more
+    const std::uint32_t op = y.z & 0xffu;
+    PlainRec d;
+    d.issue = base_ps + (y.x | (static_cast<std::uint64_t>(y.y) << 32));
+    d.bytes = bytes;
+    std::uint32_t lo = 0;  // ranges whose base is at most addr
+    for (std::uint32_t step = a.r_top; step != 0; step >>= 1) {
+        const std::uint32_t mid = lo + step;
+        const std::uint32_t at = (mid < a.r_count ? mid : a.r_count) - 1;
+        lo = l.fence[at] <= addr && mid <= a.r_count ? mid : lo;
+    }
+    const std::uint32_t idx = lo == 0 ? 0u : lo - 1;
+    const std::uint64_t off = addr - l.fence[idx];
+    const std::uint64_t lm = l.len[idx];
+    const std::uint64_t len = lm & kRangeLenMask;
+    const std::uint32_t page_bytes = 1u << a.page_shift;
+    const std::uint32_t in_page = static_cast<std::uint32_t>(off) & (page_bytes - 1);
+    const bool inside = lo != 0 && off < len;
+    // access_supported and media_descriptor (hbf_device.cuh:843-860): inside
+    // one page and the range, permitted
+    const bool ok = inside && !huge && bytes != 0 && op <= 1 && bytes <= page_bytes - in_page &&
+                    bytes <= len - off &&
+                    ((static_cast<std::uint32_t>(lm >> 60) >> (op & 1u)) & 1u) != 0;
+    d.cls = ok ? kClsModeled : (inside || huge ? kClsUnsupported : kClsBypass);
+    if (__ballot(valid && !inside) != 0 && !inside && lo < a.r_count) {
+        // outside every range: unsupported when the span reaches the next one
+        if (overlaps(l.fence[lo], l.len[lo] & kRangeLenMask, addr, bytes)) {
+            d.cls = kClsUnsupported;
+        }
+    }
+    d.cls = valid ? d.cls : kClsInvalid;
+    const std::uint32_t page = l.page0[idx] + static_cast<std::uint32_t>(off >> a.page_shift);
+    d.page1 = page + 1;
+    d.bits = op;
+    if (op == 1 && (a.every_write != 0 || in_page + bytes == page_bytes)) {
+        d.bits = 3u;
+    }
+    d.plane = 0;
+    d.chan = 0;
+    if (!a.flat) {
+        std::uint32_t c[4];
+#pragma unroll
+        for (int ax = 0; ax < 4; ++ax) {
+            c[ax] = (page >> a.axis_shift[ax]) & (a.axis_size[ax] - 1);
+        }
+        d.chan = c[0];
+        d.plane = ((c[0] * a.W + c[1]) * a.D + c[2]) * a.P + c[3];
+    }
+    return d;
+}
+
+// Lanes of `active` with this lane's key (m: this lane is one of them): the
+// low five key bits through the LDS table, the others by ballots.
+__device__ __forceinline__ std::uint64_t plain_match(const PlainLds& l, std::uint32_t key,
+                                                     std::uint32_t bits, bool m, int lane)
+{
+    std::uint64_t peers = match_lds(l.tab, key & (kMatchSlots - 1), m, lane);
+    for (std::uint32_t b = 5; b < bits; ++b) {
+        const bool bit = ((key >> b) & 1u) != 0;
+        const std::uint64_t ones = __ballot(bit);
+        peers &= bit ? ones : ~ones;
+    }
+    return peers;
+}
+
+// Every lane's transfer time; `same` (wave-uniform): the modeled lanes move
+// the same byte count, whose time is kept from step to step (x_bytes, x_ps).
+__device__ __forceinline__ std::uint64_t plain_xfer(const KArgs& a, const PlainRec& d, bool m,
+                                                    std::uint64_t active, std::uint32_t& x_bytes,
+                                                    std::uint64_t& x_ps, bool& same)
+{
+    if (a.transfer_page != 0) {
+        same = true;
+        if (x_bytes == 0) {
+            x_bytes = 1;
+            x_ps = xfer_ps(a, 1ull << a.page_shift);
+        }
+        return x_ps;
+    }
+    const std::uint32_t b0 = static_cast<std::uint32_t>(__builtin_amdgcn_readlane(
+        static_cast<int>(d.bytes), __ffsll(static_cast<long long>(active)) - 1));
+    same = __ballot(m && d.bytes != b0) == 0;
+    if (same) {
+        if (b0 != x_bytes) {
+            x_bytes = b0;
+            x_ps = xfer_ps(a, b0);
+        }
+        return x_ps;
+    }
+    return m ? a.xfer_q * ((static_cast<std::uint64_t>(d.bytes) * a.xfer_num + a.xfer_den - 1) /
+                           a.xfer_den)
+             : 0ull;
+}
+
+// A step's lanes that continue their neighbour's line at its issue time: what
+// weight and KV streams are made of (k_summary batches them).
+__device__ __forceinline__ std::uint32_t plain_continues(const uint4& x, const uint4& y)
+{
+    const std::uint32_t pa = dpp32<0x138, 0xF>(x.x), pt = dpp32<0x138, 0xF>(y.x);
+    return static_cast<std::uint32_t>(__popcll(__ballot(pa + x.z == x.x && pt == y.x)));
+}
+
+// Steps of mostly continuing lines that make a tile k_summary's: the pass
+// stops at the second one it meets.
+constexpr std::uint32_t kStreamLanes = 32;
+constexpr int kStreamSteps = 2;
+// steps in flight: 4 KiB a wave in either form
+template <bool kPacked>
+constexpr int kPlainPipe = kPacked ? 4 : 2;
+
+// The summary pass of scattered records: one wave per tile, the outputs of
+// k_summary (without step descriptors, which only k_apply reads).  kAll: every
+// tile is taken (short runs, where one launch counts more than a tile's steps).
+template <bool kPacked, bool kAll>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6)))
+void k_plain_summary(KArgs a, const void* rec, std::size_t n, std::uint64_t base_ps,
+                     PlaneSum* psum, MaskWord* tmask, ChanSum* csum, std::uint64_t* tile_count)
+{
+    extern __shared__ std::uint64_t sm[];
+    const int lane = threadIdx.x;
+    const std::size_t tile = blockIdx.x;
+    const std::size_t begin = tile * a.tile;
+    const std::size_t end = begin + a.tile < n ? begin + a.tile : n;
+    stamp_start(a, 0);
+    using Pipe = std::conditional_t<kPacked, PackedPipeT<kPlainPipe<kPacked>>,
+                                    RecordPipeT<kPlainPipe<kPacked>>>;
+    Pipe pipe;
+    pipe.issue(rec, begin, end, lane);
+    std::uint64_t last_issue = base_ps;
+    if (begin > 0) {
+        last_issue = base_ps + (kPacked ? (static_cast<const hbf_record16*>(rec)[begin - 1].issue_op &
+                                           ((1ull << 56) - 1))
+                                        : static_cast<const hbf_record32*>(rec)[begin - 1].issue_ps);
+    }
+    const std::uint32_t rpp = plane_slots(a);
+    const PlainLds l = plain_layout(a, sm, 3ull * rpp + 2ull * a.Rc);
+    std::uint64_t* p_fi = l.w64;
+    std::uint64_t* p_rA = p_fi + rpp;
+    std::uint64_t* p_rB = p_rA + rpp;
+    std::uint64_t* c_A = p_rB + rpp;
+    std::uint64_t* c_B = c_A + a.Rc;
+    std::uint32_t* p_f1 = l.w32;
+    std::uint32_t* p_l1 = p_f1 + rpp;
+    std::uint8_t* p_fc = reinterpret_cast<std::uint8_t*>(p_l1 + rpp);
+    plain_load(a, l, lane);
+    for (std::uint32_t r = lane; r < rpp; r += kWave) {
+        p_rA[r] = 0;
+        p_rB[r] = 0;
+        p_f1[r] = 0;
+        p_l1[r] = 0;
+    }
+    for (std::uint32_t r = lane; r < a.Rc; r += kWave) {
+        c_A[r] = 0;
+        c_B[r] = 0;
+    }
+    __syncthreads();
+    const std::uint64_t lt = lanemask_lt(lane);
+    std::uint64_t modeled = 0, x_ps = 0;
+    std::uint32_t x_bytes = 0;
+    bool disorder = false;
+    int streams = 0;
+    constexpr std::size_t kSpan = static_cast<std::size_t>(kPlainPipe<kPacked>) * kWave;
+    for (std::size_t g = begin; g < end; g += kSpan) {
+        pipe.advance(rec, g + kSpan, end, lane);
+        const std::size_t gend = g + kSpan < end ? g + kSpan : end;
+        for (std::size_t s = g; s < gend; s += kWave) {
+            typename Pipe::Step st;
+            pipe.take(st);
+            uint4 x, y;
+            step_records(st, lane, x, y);
+            const bool valid = s + lane < end;
+            if (!kAll) {
+                streams += plain_continues(x, y) >= kStreamLanes ? 1 : 0;
+                if (streams >= kStreamSteps) {
+                    if (lane == 0) {
+                        a.tile_split[tile] = 0;
+                    }
+                    return;  // k_summary takes the tile
+                }
+            }
+            const PlainRec d = plain_record(a, l, x, y, valid, base_ps);
+            {
+                const std::uint64_t prev = prev_lane64(d.issue);
+                const bool back = valid && d.issue < (lane == 0 ? last_issue : prev);
+                disorder = disorder || __ballot(back) != 0;
+                const std::uint64_t vmask = __ballot(valid);  // lanes 0 .. k
+                last_issue = readlane64(d.issue, 63 - __clzll(static_cast<long long>(vmask)));
+            }
+            const bool m = d.cls == kClsModeled;
+            const std::uint64_t active = __ballot(m);
+            if (active == 0) {
+                continue;
+            }
+            modeled += __popcll(active);
+            bool same = false;
+            const std::uint64_t xfer = plain_xfer(a, d, m, active, x_bytes, x_ps, same);
+            const std::uint64_t pp = plain_match(l, d.plane, a.pbits, m, lane);
+            const std::uint64_t pc = plain_match(l, d.chan, a.cbits, m, lane);
+            const std::uint32_t pk = pslot(d.plane);
+            const std::uint32_t f1 = m ? p_f1[pk] : 0u;
+            const std::uint64_t below = pp & lt;
+            std::uint32_t prev1 = static_cast<std::uint32_t>(__shfl(
+                static_cast<int>(d.page1),
+                m && below != 0 ? 63 - __clzll(static_cast<long long>(below)) : lane));
+            const bool lead = m && below == 0;
+            if (lead) {
+                prev1 = p_l1[pk];
+            }
+            const bool tfirst = lead && f1 == 0;
+            const bool hit = a.slots != 0 && prev1 == d.page1;
+            const StepCounts sc = count_services(m && !tfirst, d.bits, hit);
+            // Per group of lanes on one plane, (A, B) becomes (A + S, max(B +
+            // S, issue_k + S_k) over its lanes k), with S the service of all
+            // of them and S_k that of lane k and later: the group's last lane
+            // adds S, then every lane joins its own term (a wave's LDS
+            // operations complete in issue order).  The tile's first record on
+            // a plane is kept apart, its hit not known yet.
+            const std::uint64_t from = count_service(a, sc, pp & ~lt);
+            if (tfirst) {
+                p_f1[pk] = d.page1;
+                p_fi[pk] = d.issue;
+                p_fc[pk] = static_cast<std::uint8_t>(d.bits);
+            }
+            if (m && (pp >> lane) == 1ull) {
+                const std::uint64_t S = from + count_service(a, sc, below);
+                lds_add(&p_rA[pk], S);
+                lds_add(&p_rB[pk], S);
+                p_l1[pk] = d.page1;
+            }
+            if (m && !tfirst) {
+                lds_max(&p_rB[pk], d.issue + from);
+            }
+            // channels likewise
+            std::uint64_t Sc, after;
+            if (same) {
+                const auto times = [&](std::uint64_t lanes) {
+                    return static_cast<std::uint64_t>(
+                               static_cast<std::uint32_t>(__popcll(lanes))) * xfer;
+                };
+                Sc = times(pc);
+                after = times(pc & ~lt);
+            } else {
+                // different byte counts: sums along the group by pointer jumping
+                Sc = m ? xfer : 0ull;
+                std::uint64_t unused = 0;
+                group_scan(Sc, unused, m && (pc & lt) != 0
+                                           ? 63 - __clzll(static_cast<long long>(pc & lt))
+                                           : -1, lane);
+                const std::uint64_t upto = Sc;
+                Sc = shfl64(Sc, m ? 63 - __clzll(static_cast<long long>(pc)) : lane);
+                after = Sc - upto + xfer;
+            }
+            if (m && (pc >> lane) == 1ull) {
+                lds_add(&c_A[d.chan], Sc);
+                lds_add(&c_B[d.chan], Sc);
+            }
+            if (m) {
+                lds_max(&c_B[d.chan], d.issue + after);
+            }
+        }
+    }
+    if (lane == 0) {
+        if (disorder && a.disorder != nullptr) {
+            *a.disorder = 1u;
+        }
+        a.tile_split[tile] = kTilePlain;
+        tile_count[tile] = modeled;
+    }
+    __syncthreads();
+    // the touched planes' summaries, packed in plane order, as k_summary's
+    PlaneSum* ps = psum + tile * a.Rp;
+    MaskWord* tm = tmask + tile * mask_words(a);
+    std::uint32_t count = 0;
+    for (std::uint32_t r0 = 0; r0 < a.Rp; r0 += kWave) {
+        const std::uint32_t r = r0 + lane;
+        const std::uint32_t k = pslot(r);
+        const bool touched = r < a.Rp && p_f1[k] != 0;
+        const std::uint64_t bits = __ballot(touched);
+        if (lane == 0) {
+            tm[r0 / kWave] = MaskWord{bits, count, 0};
+        }
+        if (touched) {
+            PlaneSum v;
+            v.fpage1 = p_f1[k];
+            v.fissue = p_fi[k];
+            v.rA = p_rA[k];
+            v.rB = p_rB[k];
+            v.lpage1 = p_l1[k];
+            v.fcls = p_fc[k];
+            v.pad = 0;
+            ps[count + __popcll(bits & lt)] = v;
+        }
+        count += static_cast<std::uint32_t>(__popcll(bits));
+    }
+    ChanSum* cs = csum + tile * a.Rc;
+    for (std::uint32_t r = lane; r < a.Rc; r += kWave) {
+        cs[r] = ChanSum{c_A[r], c_B[r]};
+    }
+}
+
+// The apply pass over the tiles k_plain_summary took.
+template <bool kPacked, bool kAll>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5)))
+void k_plain_apply(KArgs a, const void* rec, std::size_t n, std::uint64_t base_ps,
+                   const PlaneCarry* pcarry, const MaskWord* tmask, const std::uint64_t* ccarry,
+                   std::uint64_t* completion, std::uint8_t* status, DevReport* tile_rep)
+{
+    extern __shared__ std::uint64_t sm[];
+    stamp_start(a, 2);
+    if ((a.disorder != nullptr && *a.disorder != 0u) ||
+        (!kAll && a.tile_split[blockIdx.x] != kTilePlain)) {
+        return;
+    }
+    const int lane = threadIdx.x;
+    const std::size_t tile = blockIdx.x;
+    const std::size_t begin = tile * a.tile;
+    const std::size_t end = begin + a.tile < n ? begin + a.tile : n;
+    using Pipe = std::conditional_t<kPacked, PackedPipeT<kPlainPipe<kPacked>>,
+                                    RecordPipeT<kPlainPipe<kPacked>>>;
+    Pipe pipe;
+    pipe.issue(rec, begin, end, lane);
+    const PlainLds l = plain_layout(a, sm, static_cast<std::size_t>(a.Rp) + a.Rc);
+    std::uint64_t* p_busy = l.w64;
+    std::uint64_t* c_busy = p_busy + a.Rp;
+    std::uint32_t* p_tag = l.w32;
+    load_plane_carry(a, tmask, pcarry, tile, p_busy, p_tag, lane);
+    load_chan_carry(a, ccarry, tile, c_busy, lane);
+    plain_load(a, l, lane);
+    __syncthreads();
+    const std::uint64_t lt = lanemask_lt(lane);
+    std::uint64_t x_ps = 0, mk = 0, lat_lo = 0, lat_hi = 0, lat_max = 0, svc_sum = 0;
+    std::uint32_t x_bytes = 0;
+    // wave-uniform counts
+    std::uint32_t n_mod = 0, n_byp = 0, n_uns = 0, n_rd = 0, n_hit = 0, n_prog = 0;
+    constexpr std::size_t kSpan = static_cast<std::size_t>(kPlainPipe<kPacked>) * kWave;
+    for (std::size_t g = begin; g < end; g += kSpan) {
+        pipe.advance(rec, g + kSpan, end, lane);
+        const std::size_t gend = g + kSpan < end ? g + kSpan : end;
+        for (std::size_t s = g; s < gend; s += kWave) {
+            typename Pipe::Step sr;
+            pipe.take(sr);
+            uint4 x, y;
+            step_records(sr, lane, x, y);
+            const std::size_t i = s + lane;
+            const bool valid = i < end;
+            const PlainRec d = plain_record(a, l, x, y, valid, base_ps);
+            const bool m = d.cls == kClsModeled;
+            const std::uint64_t active = __ballot(m);
+            std::uint32_t st = d.cls;
+            std::uint64_t done = d.cls == kClsBypass ? d.issue : ~0ull;
+            if (active != 0) {
+                bool same = false;
+                const std::uint64_t xfer = plain_xfer(a, d, m, active, x_bytes, x_ps, same);
+                const std::uint64_t pp = plain_match(l, d.plane, a.pbits, m, lane);
+                const std::uint64_t pc = plain_match(l, d.chan, a.cbits, m, lane);
+                const std::uint64_t below = pp & lt, cbelow = pc & lt;
+                const int ppred =
+                    m && below != 0 ? 63 - __clzll(static_cast<long long>(below)) : -1;
+                const int cpred =
+                    m && cbelow != 0 ? 63 - __clzll(static_cast<long long>(cbelow)) : -1;
+                const std::uint64_t pbusy = m ? p_busy[d.plane] : 0ull;
+                const std::uint64_t cbusy = m ? c_busy[d.chan] : 0ull;
+                std::uint32_t prev1 = static_cast<std::uint32_t>(
+                    __shfl(static_cast<int>(d.page1), ppred < 0 ? lane : ppred));
+                if (m && ppred < 0) {
+                    prev1 = p_tag[d.plane];
+                }
+                const bool hit = a.slots != 0 && m && prev1 == d.page1;
+                const StepCounts sc = count_services(m, d.bits, hit);
+                const std::uint64_t svc = count_service(a, sc, 1ull << lane);
+                const std::uint64_t origin =
+                    readlane64(d.issue, __ffsll(static_cast<long long>(active)) - 1);
+                const std::uint64_t most =
+                    static_cast<std::uint64_t>(static_cast<std::uint32_t>(
+                        __popcll(sc.miss))) * a.read_ps +
+                    static_cast<std::uint64_t>(static_cast<std::uint32_t>(
+                        __popcll(sc.prog))) * a.program_ps;
+                std::uint64_t pd, cd;
+                if (same && most < (1ull << 30) && xfer < (1ull << 24) &&
+                    __ballot(m && d.issue - origin >= (1ull << 30)) == 0) {
+                    // lane i of a group completes at max(busy, max over k <= i
+                    // of (issue_k - E_k)) + E_i + its service, with E the
+                    // service of the group's lanes before: where no lane's
+                    // issue time passes busy + E the maximum is busy, else it
+                    // is a prefix maximum of issue - E, in 32 bits from the
+                    // step's first issue time
+                    const std::uint32_t Ep =
+                        static_cast<std::uint32_t>(count_service(a, sc, below));
+                    const std::uint32_t x32 = static_cast<std::uint32_t>(xfer);
+                    const std::uint32_t Ec = x32 * static_cast<std::uint32_t>(__popcll(cbelow));
+                    const bool wp = a.contention != 0 &&
+                                    __ballot(m && d.issue > pbusy + Ep) != 0;
+                    const bool wc = __ballot(m && d.issue > cbusy + Ec) != 0;
+                    std::uint64_t tp = pbusy, tc = cbusy;
+                    if (wp || wc) {
+                        const std::uint32_t rel =
+                            m ? static_cast<std::uint32_t>(d.issue - origin) : 0u;
+                        const std::uint32_t most32 = static_cast<std::uint32_t>(most);
+                        const std::uint32_t c64 = x32 * 64u;
+                        std::uint32_t vp = rel + most32 - Ep, vc = rel + c64 - Ec;
+                        group_prefix_max(vp, wp ? ppred : -1, vc, wc ? cpred : -1, lane);
+                        // (issue - E may lie below zero where busy is the
+                        // maximum: compared before the offset is taken off)
+                        if (wp) {
+                            tp = origin + vp > pbusy + most32 ? origin + vp - most32 : pbusy;
+                        }
+                        if (wc) {
+                            tc = origin + vc > cbusy + c64 ? origin + vc - c64 : cbusy;
+                        }
+                    }
+                    pd = a.contention != 0 ? tp + Ep + svc : d.issue + svc;
+                    cd = tc + Ec + xfer;
+                } else {
+                    std::uint64_t Ap = m ? svc : 0ull, Bp = m ? d.issue + svc : 0ull;
+                    std::uint64_t Ac = m ? xfer : 0ull, Bc = m ? d.issue + xfer : 0ull;
+                    if (a.contention != 0) {
+                        group_scan(Ap, Bp, ppred, lane);
+                    }
+                    group_scan(Ac, Bc, cpred, lane);
+                    pd = a.contention != 0 ? umax64(pbusy + Ap, Bp) : d.issue + svc;
+                    cd = umax64(cbusy + Ac, Bc);
+                }
+                if (m && (pp >> lane) == 1ull) {
+                    if (a.contention != 0) {
+                        p_busy[d.plane] = pd;
+                    }
+                    p_tag[d.plane] = d.page1;
+                }
+                if (m && (pc >> lane) == 1ull) {
+                    c_busy[d.chan] = cd;
+                }
+                const bool write = (d.bits & 1u) != 0;
+                n_mod += static_cast<std::uint32_t>(__popcll(active));
+                n_rd += static_cast<std::uint32_t>(__popcll(__ballot(m && !write)));
+                n_hit += static_cast<std::uint32_t>(__popcll(__ballot(hit && !write)));
+                n_prog += static_cast<std::uint32_t>(__popcll(__ballot(m && write && svc != 0)));
+                if (m) {
+                    done = umax64(pd, cd);
+                    st |= write ? (svc != 0 ? 16u : 0u) : (hit ? 4u : 0u);
+                    mk = umax64(mk, done);
+                    const std::uint64_t lat = done - d.issue;
+                    add128(lat_lo, lat_hi, lat);
+                    lat_max = umax64(lat_max, lat);
+                    svc_sum += umax64(svc, xfer);
+                }
+            }
+            const std::uint64_t byp = __ballot(d.cls == kClsBypass);
+            const std::uint64_t uns = __ballot(d.cls == kClsUnsupported);
+            n_byp += static_cast<std::uint32_t>(__popcll(byp));
+            n_uns += static_cast<std::uint32_t>(__popcll(uns));
+            if (valid) {
+                put_done(&completion[i], done);
+                if (status != nullptr) {
+                    status[i] = static_cast<std::uint8_t>(st);
+                }
+            }
+        }
+    }
+    // 128-bit latency sum: the high words, then the low words with carries
+    std::uint64_t hi = wave_sum(lat_hi), carry = 0, lo = lat_lo;
+    for (int o = 32; o > 0; o >>= 1) {
+        const std::uint64_t other = shfl64(lo, lane ^ o);
+        const std::uint64_t oc = shfl64(carry, lane ^ o);
+        const std::uint64_t sum = lo + other;
+        carry = carry + oc + (sum < lo ? 1u : 0u);
+        lo = sum;
+    }
+    hi += carry;
+    const std::uint64_t vals[14] = {end - begin, n_mod, n_byp, n_uns, n_rd,
+                                    n_mod - n_rd, n_hit, n_prog, 0ull, wave_max(mk),
+                                    lo, hi, wave_max(lat_max), wave_sum(svc_sum)};
+    if (lane < 14) {
+        unsigned long long out = 0;
+#pragma unroll
+        for (int k = 0; k < 14; ++k) {
+            out = lane == k ? vals[k] : out;
+        }
+        tile_rep[tile].v[lane] = out;
+    }
 }
 
 // Report reduction: each block folds a run of tile reports; the last block to
@@ -4783,7 +5367,8 @@ int upload_ranges(engine* e, hipStream_t stream)
         e->ranges_pack = e->ranges_pack && length[i] <= kRangeLenMask &&
                          (offset[i] >> a.page_shift) <= 0xffffffffull &&
                          (offset[i] & ((1ull << a.page_shift) - 1)) == 0 &&
-                         e->ranges[i].mode <= 0xfu && e->ranges[i].permissions <= 0xfu;
+                         (e->ranges[i].mode == 1 || e->ranges[i].mode == 2) &&
+                         e->ranges[i].permissions <= 0xfu;
     }
     e->ranges_dirty = false;
     return HBFSIM_OK;
@@ -5727,6 +6312,20 @@ hipError_t allow_lds(F* kernel, std::size_t bytes)
                                static_cast<int>(bytes));
 }
 
+// Whether the scattered-record passes can take a packed run: power-of-two axes
+// (or one plane), the range table in its packed form, no hybrid sampling, and
+// their LDS within what a workgroup gets by default.
+bool plain_run(const KArgs& a, bool ranges_pack)
+{
+    return ranges_pack && a.hybrid == 0 && (a.flat != 0 || a.pow2 != 0) &&
+           plain_summary_lds(a) <= 65536 && plain_apply_lds(a) <= 65536;
+}
+
+// Runs of up to this many records take the scattered-record passes alone,
+// whatever their steps look like: tiles are at most four steps, so that what a
+// run of lines costs there is less than the two launches the mixed form adds.
+constexpr std::size_t kPlainAlone = std::size_t{1} << 18;
+
 void choose_match(KArgs& a, bool ranges_pack)
 {
     constexpr std::size_t kLdsPerCu = kLdsPerCuBytes;
@@ -6578,7 +7177,30 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
     }
     const dim3 grid(static_cast<unsigned>(ntiles));
     const std::uint8_t* hits = d_hits;
-    if (k2) {
+    // Scattered records: their own passes take the tiles that hold no runs of
+    // lines.  An engine whose last run mostly hit its page registers (runs of
+    // lines) does not look for them.
+    const bool plain = !grouping && !k2 && !refresh_records && plain_run(a, e->ranges_pack);
+    const bool plain_alone = plain && n <= kPlainAlone;
+    const bool plain_mixed = plain && !plain_alone &&
+                             (e->last_modeled == 0 || e->last_hits * 8 < e->last_modeled);
+    a.mixed = plain_mixed ? 1u : 0u;
+    if (plain_alone || plain_mixed) {
+        a.tile_split = sc.tsplit;
+        a.r_top = 1;
+        while (a.r_top * 2 <= a.r_count) {
+            a.r_top *= 2;
+        }
+        const auto summary = packed ? (plain_alone ? k_plain_summary<true, true>
+                                                   : k_plain_summary<true, false>)
+                                    : (plain_alone ? k_plain_summary<false, true>
+                                                   : k_plain_summary<false, false>);
+        hipLaunchKernelGGL(summary, grid, dim3(kWave), plain_summary_lds(a), stream, a, d_rec, n,
+                           base_ps, sc.psum, sc.tmask, sc.csum, sc.tcount);
+    }
+    if (plain_alone) {
+        // every tile is summarised
+    } else if (k2) {
         (void)allow_lds(k_summary<false, true>, lds_a);
         hipLaunchKernelGGL((k_summary<false, true>), grid, dim3(kWave), lds_a, stream, a, d_rec,
                            n, base_ps, sc.psum, sc.tmask, sc.csum, sc.tcount,
@@ -6641,7 +7263,18 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
                             kLdsPerCuBytes / lds_c >= 4 * kSimdsPerCu && e->last_modeled != 0 &&
                             e->last_hits * 8 < e->last_modeled;
     e->last_apply_waves = packed && !k2 && !refresh_records ? (wide_apply ? 4 : 3) : 1;
-    if (k2) {
+    if (plain_alone || plain_mixed) {
+        const auto apply = packed ? (plain_alone ? k_plain_apply<true, true>
+                                                 : k_plain_apply<true, false>)
+                                  : (plain_alone ? k_plain_apply<false, true>
+                                                 : k_plain_apply<false, false>);
+        hipLaunchKernelGGL(apply, grid, dim3(kWave), plain_apply_lds(a), stream, a, d_rec, n,
+                           base_ps, sc.pcarry, sc.tmask, sc.ccarry, d_comp, d_status,
+                           sc.tile_rep);
+    }
+    if (plain_alone) {
+        // every tile is replayed
+    } else if (k2) {
         (void)allow_lds(k_apply<false, true>, lds_c);
         hipLaunchKernelGGL((k_apply<false, true>), grid, dim3(kWave), lds_c, stream, a, d_rec, n,
                            base_ps, sc.pcarry, sc.tmask, sc.ccarry, sc.tseq, d_comp,
