@@ -3551,12 +3551,12 @@ __host__ __device__ __forceinline__ std::size_t apply_range_offset(const KArgs& 
 // A tile's plane carry-ins are packed like its summaries: word w of the
 // mask covers planes [64 w, 64 w + 64), so lane l reads bit l of each word.
 // Eight words' carries are in flight before any is written.
+template <int kWords = 8>
 __device__ __forceinline__ void load_plane_carry(const KArgs& a, const MaskWord* tmask,
                                                  const PlaneCarry* pcarry, std::size_t tile,
                                                  std::uint64_t* p_busy, std::uint32_t* p_tag,
                                                  int lane)
 {
-    constexpr int kWords = 8;
     const std::uint32_t words = mask_words(a);
     const MaskWord* tm = tmask + tile * words;
     const PlaneCarry* pc = pcarry + tile * a.Rp;
@@ -4187,7 +4187,7 @@ __host__ __device__ __forceinline__ std::size_t plain_lds_bytes(const KArgs& a, 
 __host__ __device__ __forceinline__ std::size_t plain_summary_lds(const KArgs& a)
 {
     const std::size_t rp = plane_slots(a);
-    return plain_lds_bytes(a, 3 * rp + 2ull * a.Rc, 2 * rp) + rp;
+    return plain_lds_bytes(a, rp + 2ull * a.Rc, 2 * rp) + 2 * rp;
 }
 
 __host__ __device__ __forceinline__ std::size_t plain_apply_lds(const KArgs& a)
@@ -4373,21 +4373,23 @@ void k_plain_summary(KArgs a, const void* rec, std::size_t n, std::uint64_t base
                                         : static_cast<const hbf_record32*>(rec)[begin - 1].issue_ps);
     }
     const std::uint32_t rpp = plane_slots(a);
-    const PlainLds l = plain_layout(a, sm, 3ull * rpp + 2ull * a.Rc);
-    std::uint64_t* p_fi = l.w64;
-    std::uint64_t* p_rA = p_fi + rpp;
-    std::uint64_t* p_rB = p_rA + rpp;
+    const PlainLds l = plain_layout(a, sm, rpp + 2ull * a.Rc);
+    // Per plane 18 bytes: the map's B; its A as counts (senses, programs in
+    // the high half); the last page; and 1 + the tile's first record there, read
+    // again at the end for its page and issue time.  (33 bytes, as k_summary
+    // keeps them, left nine waves per CU at 512 planes instead of fifteen.)
+    std::uint64_t* p_rB = l.w64;
     std::uint64_t* c_A = p_rB + rpp;
     std::uint64_t* c_B = c_A + a.Rc;
-    std::uint32_t* p_f1 = l.w32;
-    std::uint32_t* p_l1 = p_f1 + rpp;
-    std::uint8_t* p_fc = reinterpret_cast<std::uint8_t*>(p_l1 + rpp);
+    std::uint32_t* p_n = l.w32;
+    std::uint32_t* p_l1 = p_n + rpp;
+    std::uint16_t* p_f = reinterpret_cast<std::uint16_t*>(p_l1 + rpp);
     plain_load(a, l, lane);
     for (std::uint32_t r = lane; r < rpp; r += kWave) {
-        p_rA[r] = 0;
         p_rB[r] = 0;
-        p_f1[r] = 0;
+        p_n[r] = 0;
         p_l1[r] = 0;
+        p_f[r] = 0;
     }
     for (std::uint32_t r = lane; r < a.Rc; r += kWave) {
         c_A[r] = 0;
@@ -4437,7 +4439,7 @@ void k_plain_summary(KArgs a, const void* rec, std::size_t n, std::uint64_t base
             const std::uint64_t pp = plain_match(l, d.plane, a.pbits, m, lane);
             const std::uint64_t pc = plain_match(l, d.chan, a.cbits, m, lane);
             const std::uint32_t pk = pslot(d.plane);
-            const std::uint32_t f1 = m ? p_f1[pk] : 0u;
+            const std::uint32_t f1 = m ? p_f[pk] : 0u;
             const std::uint64_t below = pp & lt;
             std::uint32_t prev1 = static_cast<std::uint32_t>(__shfl(
                 static_cast<int>(d.page1),
@@ -4457,14 +4459,14 @@ void k_plain_summary(KArgs a, const void* rec, std::size_t n, std::uint64_t base
             // a plane is kept apart, its hit not known yet.
             const std::uint64_t from = count_service(a, sc, pp & ~lt);
             if (tfirst) {
-                p_f1[pk] = d.page1;
-                p_fi[pk] = d.issue;
-                p_fc[pk] = static_cast<std::uint8_t>(d.bits);
+                p_f[pk] = static_cast<std::uint16_t>(s + lane - begin + 1);
             }
             if (m && (pp >> lane) == 1ull) {
-                const std::uint64_t S = from + count_service(a, sc, below);
-                lds_add(&p_rA[pk], S);
-                lds_add(&p_rB[pk], S);
+                const std::uint32_t senses = static_cast<std::uint32_t>(__popcll(pp & sc.miss));
+                const std::uint32_t programs = static_cast<std::uint32_t>(__popcll(pp & sc.prog));
+                (void)__hip_atomic_fetch_add(&p_n[pk], senses | (programs << 16), __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_WORKGROUP);
+                lds_add(&p_rB[pk], senses * a.read_ps + programs * a.program_ps);
                 p_l1[pk] = d.page1;
             }
             if (m && !tfirst) {
@@ -4514,19 +4516,30 @@ void k_plain_summary(KArgs a, const void* rec, std::size_t n, std::uint64_t base
     for (std::uint32_t r0 = 0; r0 < a.Rp; r0 += kWave) {
         const std::uint32_t r = r0 + lane;
         const std::uint32_t k = pslot(r);
-        const bool touched = r < a.Rp && p_f1[k] != 0;
+        const std::uint32_t f = r < a.Rp ? p_f[k] : 0u;
+        const bool touched = f != 0;
         const std::uint64_t bits = __ballot(touched);
         if (lane == 0) {
             tm[r0 / kWave] = MaskWord{bits, count, 0};
         }
+        uint4 x = make_uint4(0, 0, 0, 0), y = x;
+        if (touched) {
+            const std::size_t i = begin + f - 1;
+            if constexpr (kPacked) {
+                unpack16(static_cast<const uint4*>(rec)[i], x, y);
+            } else {
+                load_record(static_cast<const hbf_record32*>(rec), i, x, y);
+            }
+        }
+        const PlainRec d = plain_record(a, l, x, y, touched, base_ps);
         if (touched) {
             PlaneSum v;
-            v.fpage1 = p_f1[k];
-            v.fissue = p_fi[k];
-            v.rA = p_rA[k];
+            v.fpage1 = d.page1;
+            v.fissue = d.issue;
+            v.rA = (p_n[k] & 0xffffu) * a.read_ps + (p_n[k] >> 16) * a.program_ps;
             v.rB = p_rB[k];
             v.lpage1 = p_l1[k];
-            v.fcls = p_fc[k];
+            v.fcls = d.bits;
             v.pad = 0;
             ps[count + __popcll(bits & lt)] = v;
         }
@@ -4540,7 +4553,7 @@ void k_plain_summary(KArgs a, const void* rec, std::size_t n, std::uint64_t base
 
 // The apply pass over the tiles k_plain_summary took.
 template <bool kPacked, bool kAll>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
 void k_plain_apply(KArgs a, const void* rec, std::size_t n, std::uint64_t base_ps,
                    const PlaneCarry* pcarry, const MaskWord* tmask, const std::uint64_t* ccarry,
                    std::uint64_t* completion, std::uint8_t* status, DevReport* tile_rep)
@@ -4563,7 +4576,7 @@ void k_plain_apply(KArgs a, const void* rec, std::size_t n, std::uint64_t base_p
     std::uint64_t* p_busy = l.w64;
     std::uint64_t* c_busy = p_busy + a.Rp;
     std::uint32_t* p_tag = l.w32;
-    load_plane_carry(a, tmask, pcarry, tile, p_busy, p_tag, lane);
+    load_plane_carry<4>(a, tmask, pcarry, tile, p_busy, p_tag, lane);
     load_chan_carry(a, ccarry, tile, c_busy, lane);
     plain_load(a, l, lane);
     __syncthreads();
@@ -6313,11 +6326,12 @@ hipError_t allow_lds(F* kernel, std::size_t bytes)
 }
 
 // Whether the scattered-record passes can take a packed run: power-of-two axes
-// (or one plane), the range table in its packed form, no hybrid sampling, and
-// their LDS within what a workgroup gets by default.
+// (or one plane), the range table in its packed form, no hybrid sampling,
+// tiles whose counts fit 16 bits, and their LDS within what a workgroup gets by
+// default.
 bool plain_run(const KArgs& a, bool ranges_pack)
 {
-    return ranges_pack && a.hybrid == 0 && (a.flat != 0 || a.pow2 != 0) &&
+    return ranges_pack && a.hybrid == 0 && (a.flat != 0 || a.pow2 != 0) && a.tile < 65536 &&
            plain_summary_lds(a) <= 65536 && plain_apply_lds(a) <= 65536;
 }
 
