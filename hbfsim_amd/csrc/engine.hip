@@ -152,10 +152,10 @@ struct KArgs {
     // and the engine times the stream again from a sorted copy (null: the
     // stream is known to be in issue order)
     std::uint32_t* disorder;
-    // per tile, written by the summary pass of packed records: 1 when the
+    // per tile, written by the summary pass: 1 when the
     // tile holds a split step (the apply pass then takes its split-capable
     // body), kTilePlain when the scattered-record passes take it, else 0; null
-    // for 32-byte records unless those passes run
+    // for streams with refresh records
     std::uint8_t* tile_split;
     std::uint32_t mixed;  // the scattered-record passes ran before: skip their tiles
     // start times of the summary pass, the carry chain and the apply pass
@@ -1165,7 +1165,7 @@ struct LinStep {
     std::uint64_t issue;
 };
 
-// Packed steps: a step whose records all share record 0's byte count, issue
+// A step whose records all share record 0's byte count (b0), issue
 // time and read operation, and whose addresses continue record 0's (one run,
 // split where a page boundary falls inside it) or continue record 0's up to
 // a lane k and lane k's after it (two spans joined).  Each run must lie in
@@ -1174,27 +1174,12 @@ struct LinStep {
 // address lies outside the wave-uniform range cache refills it through the
 // full classification (one call site for both runs).
 template <bool kRefresh>
-__device__ __forceinline__ bool linear_detect_split(const KArgs& a, const RangeView& fence,
-                                                    RangeCache& rcu, const Step16& st,
-                                                    std::uint64_t base_ps, bool full, int lane,
-                                                    LinStep& ls)
+__device__ __forceinline__ bool split_runs(const KArgs& a, const RangeView& fence,
+                                           RangeCache& rcu, std::uint64_t addr,
+                                           std::uint32_t b0, const uint4& yu,
+                                           std::uint64_t base_ps, int lane, LinStep& ls)
 {
-    if (!full) {
-        return false;
-    }
-    const uint4& R = st.R;
-    const uint4 r0 = make_uint4(rfl32(R.x), rfl32(R.y), rfl32(R.z), rfl32(R.w));
-    uint4 xu, yu;
-    unpack16(r0, xu, yu);
-    if (yu.z != 0 || xu.z == 0) {
-        return false;  // reads of at least one byte only
-    }
-    const std::uint32_t b0 = xu.z;
-    if (__ballot((R.y >> 16) != b0 || R.z != r0.z || R.w != r0.w) != 0) {
-        return false;
-    }
-    const std::uint64_t a0 = xu.x | (static_cast<std::uint64_t>(xu.y) << 32);
-    const std::uint64_t addr = R.x | (static_cast<std::uint64_t>(R.y & 0xffffu) << 32);
+    const std::uint64_t a0 = readlane64(addr, 0);
     const std::uint64_t breaks = __ballot(addr != a0 + static_cast<std::uint64_t>(lane) * b0);
     std::uint32_t k = 0;  // the split lane (0: none)
     std::uint64_t a1 = 0;
@@ -1263,32 +1248,78 @@ __device__ __forceinline__ bool linear_detect_split(const KArgs& a, const RangeV
     return true;
 }
 
-// The step detection of a record form: packed steps may be split (kSplit);
-// otherwise, and for 32-byte records, steps are whole linear steps or none.
-template <bool kRefresh, bool kSplit>
+template <bool kRefresh>
+__device__ __forceinline__ bool linear_detect_split(const KArgs& a, const RangeView& fence,
+                                                    RangeCache& rcu, const Step16& st,
+                                                    std::uint64_t base_ps, bool full, int lane,
+                                                    LinStep& ls)
+{
+    if (!full) {
+        return false;
+    }
+    const uint4& R = st.R;
+    const uint4 r0 = make_uint4(rfl32(R.x), rfl32(R.y), rfl32(R.z), rfl32(R.w));
+    uint4 xu, yu;
+    unpack16(r0, xu, yu);
+    if (yu.z != 0 || xu.z == 0) {
+        return false;  // reads of at least one byte only
+    }
+    if (__ballot((R.y >> 16) != xu.z || R.z != r0.z || R.w != r0.w) != 0) {
+        return false;
+    }
+    return split_runs<kRefresh>(a, fence, rcu,
+                                R.x | (static_cast<std::uint64_t>(R.y & 0xffffu) << 32), xu.z, yu,
+                                base_ps, lane, ls);
+}
+
+// 32-byte records: a whole step is found in the halves as they lie; only a
+// step that is none is laid out record-per-lane for its runs.
+template <bool kRefresh>
+__device__ __forceinline__ bool linear_detect_split(const KArgs& a, const RangeView& fence,
+                                                    RangeCache& rcu, const Step32& st,
+                                                    std::uint64_t base_ps, bool full, int lane,
+                                                    LinStep& ls)
+{
+    if (!full) {
+        return false;
+    }
+    const std::uint32_t b0 = rfl32(st.A.z);
+    const uint4 yu = make_uint4(rl32(st.A.x, 1), rl32(st.A.y, 1), rl32(st.A.z, 1), 0);
+    if ((yu.z & 0xffu) != 0 || rfl32(st.A.w) != 0 || b0 == 0) {
+        return false;  // reads of 1 .. 2^32 - 1 bytes only
+    }
+    // every even lane's byte count, every odd lane's issue time and flags
+    const bool odd = (lane & 1) != 0;
+    const bool ok_even = st.A.z == b0 && st.A.w == 0 && st.B.z == b0 && st.B.w == 0;
+    const bool ok_odd = st.A.x == yu.x && st.A.y == yu.y && st.A.z == yu.z && st.B.x == yu.x &&
+                        st.B.y == yu.y && st.B.z == yu.z;
+    if (__ballot(odd ? !ok_odd : !ok_even) != 0) {
+        return false;
+    }
+    const int src = ((2 * lane) & 63) << 2;
+    const auto pick = [&](std::uint32_t u, std::uint32_t v) {
+        const std::uint32_t tu =
+            static_cast<std::uint32_t>(__builtin_amdgcn_ds_bpermute(src, static_cast<int>(u)));
+        const std::uint32_t tv =
+            static_cast<std::uint32_t>(__builtin_amdgcn_ds_bpermute(src, static_cast<int>(v)));
+        return lane < 32 ? tu : tv;
+    };
+    const std::uint64_t addr = pick(st.A.x, st.B.x) |
+                               (static_cast<std::uint64_t>(pick(st.A.y, st.B.y)) << 32);
+    return split_runs<kRefresh>(a, fence, rcu, addr, b0, yu, base_ps, lane, ls);
+}
+
+// The step detection: with kSplit steps may be split; otherwise they are whole
+// linear steps or none.
+template <bool kRefresh, bool kSplit, typename Step>
 __device__ __forceinline__ bool detect_step(const KArgs& a, const RangeView& fence,
-                                            RangeCache& rcu, const Step16& st,
+                                            RangeCache& rcu, const Step& st,
                                             std::uint64_t base_ps, bool full, int lane,
                                             LinStep& ls)
 {
     if constexpr (kSplit) {
         return linear_detect_split<kRefresh>(a, fence, rcu, st, base_ps, full, lane, ls);
     }
-    ls.k = 0;
-    ls.page1b = 0;
-    ls.ridb = 0;
-    const bool lin = linear_detect<kRefresh>(a, fence, rcu, st, base_ps, full, lane, ls.page1,
-                                             ls.issue, ls.bytes);
-    ls.rid = rcu.id;
-    return lin;
-}
-
-template <bool kRefresh, bool kSplit>
-__device__ __forceinline__ bool detect_step(const KArgs& a, const RangeView& fence,
-                                            RangeCache& rcu, const Step32& st,
-                                            std::uint64_t base_ps, bool full, int lane,
-                                            LinStep& ls)
-{
     ls.k = 0;
     ls.page1b = 0;
     ls.ridb = 0;
@@ -1942,10 +1973,24 @@ __device__ __forceinline__ void batch_order(const LinBatchT<kR>& q, int lane, st
 // run that holds the tile's first record on its plane records that record
 // and folds the m - 1 hits after it, map (0, issue) (the identity for m = 1).
 // The channel map of a run is (m x, issue + m x).  kGiven: page-register
-// hits come per record from `hits` (two page registers, whole steps only):
-// a step's first record hits as hits[] says, and a step that is the tile's
-// first record on its plane records that hit in its class (bit 3), as the
+// hits come per record from `hits` (two page registers): a run's first record
+// hits as hits[] says, and a run that holds the tile's first record on its
+// plane records that hit in its class (bit 3), as the
 // per-record path does.
+// Stream position of the first record of lane r's run.
+template <bool kR>
+__device__ __forceinline__ std::size_t run_record(const LinBatchT<kR>& q, int lane)
+{
+    int row = lane;
+    std::uint32_t at = 0;
+    if constexpr (kR) {
+        const std::uint64_t heads = __ballot(lane < q.n && q.lo == 0);
+        row = __popcll(heads & (lanemask_lt(lane) | (1ull << lane))) - 1;
+        at = q.lo;
+    }
+    return q.first + static_cast<std::size_t>(row) * kWave + at;
+}
+
 template <bool kR, bool kGiven = false>
 __device__ __forceinline__ void fold_summary(const KArgs& a, const std::uint64_t* xp,
                                              const LinBatchT<kR>& q, int lane, std::uint64_t* p_fi,
@@ -1956,7 +2001,6 @@ __device__ __forceinline__ void fold_summary(const KArgs& a, const std::uint64_t
                                              std::uint64_t* mt_c,
                                              const std::uint8_t* hits = nullptr)
 {
-    static_assert(!(kR && kGiven), "given hits take whole steps only");
     const StepView v = step_view(a, xp, q, lane);
     const bool m = v.m;
     const std::uint32_t pkey = m ? v.d.plane : 0u;
@@ -1975,7 +2019,8 @@ __device__ __forceinline__ void fold_summary(const KArgs& a, const std::uint64_t
     }
     bool hit0 = prev1 == q.page1;
     if constexpr (kGiven) {
-        hit0 = m && hits[q.first + static_cast<std::size_t>(lane) * kWave] != 0;
+        const std::size_t at = run_record(q, lane);
+        hit0 = m && hits[at] != 0;
     }
     const std::uint64_t ls = hit0 ? 0ull : a.read_ps;
     const std::uint64_t cx = q.len() * v.x;
@@ -2119,6 +2164,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
                                                 const std::uint8_t* hits, StepDesc* desc)
 {
     extern __shared__ std::uint64_t sm[];
+    constexpr bool kRuns = !kRefresh;  // batches hold runs: steps may be split
     // per-plane state at slot pslot(plane) of plane_slots(a) entries
     const std::uint32_t rpp = plane_slots(a);
     RangeView fence(sm);
@@ -2203,11 +2249,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
     __syncthreads();
     RangeCache rc = empty_cache();
     RangeCache rcu = empty_cache();  // wave-uniform copy for linear steps
-    LinBatchT<kPacked> q = empty_batch<kPacked>();
-    LinBatchT<kPacked> dq = empty_batch<kPacked>();  // folded, descriptors not written yet
-    // a batch is folded once it holds kFull runs: packed batches keep two
-    // lanes free for a split step's runs
-    constexpr int kFull = kPacked ? kWave - 1 : kWave;
+    LinBatchT<kRuns> q = empty_batch<kRuns>();
+    LinBatchT<kRuns> dq = empty_batch<kRuns>();  // folded, descriptors not written yet
+    // a batch is folded once it holds kFull runs: two lanes stay free for a
+    // split step's runs
+    constexpr int kFull = kRuns ? kWave - 1 : kWave;
     std::uint64_t modeled = 0;
     std::uint32_t lin_miss = 0;  // steps in a row that were not linear (wave-uniform)
     // descriptors of steps replayed from their records are zeroed up to 64
@@ -2235,7 +2281,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
                 q.push_group(gl, g, rcu.id);
                 if (q.n >= kFull || gend >= end) {
                     batch_order(q, lane, last_issue, disorder);
-                    fold_summary<kPacked, kHits>(a, xp, q, lane, p_fi, p_rA, p_rB, c_A, c_B,
+                    fold_summary<kRuns, kHits>(a, xp, q, lane, p_fi, p_rA, p_rB, c_A, c_B,
                                                  p_f1, p_l1, p_fc, mt_p, mt_c, hits);
                     modeled += static_cast<std::uint64_t>(q.rows) * kWave;
                     dq = q;  // (its descriptors wait for the next group's loads)
@@ -2255,14 +2301,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
                 LinStep ls;
                 bool lin = false;
                 if (lin_miss < kLinGiveUp || (s / kWave) % kLinProbe == 0) {
-                    lin = detect_step<kRefresh, kPacked>(a, fence, rcu, st, base_ps, s + kWave <= end,
+                    lin = detect_step<kRefresh, kRuns>(a, fence, rcu, st, base_ps, s + kWave <= end,
                                                 lane, ls);
                     lin_miss = lin ? 0u : lin_miss + 1u;
                 }
                 if (lin) {
-                    if (ls.k == 0) {
+                    if (!kRuns || ls.k == 0) {
                         q.push(ls.page1, ls.issue, ls.bytes, s, ls.rid);
-                    } else {
+                    } else if constexpr (kRuns) {
                         q.push_split(ls.page1, ls.page1b, ls.k, ls.issue, ls.bytes, s, ls.rid,
                                      ls.ridb);
                         any_split = true;
@@ -2270,7 +2316,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
                 }
                 if (q.n != 0 && (!lin || q.n >= kFull || s + kWave >= end)) {
                     batch_order(q, lane, last_issue, disorder);
-                    fold_summary<kPacked, kHits>(a, xp, q, lane, p_fi, p_rA, p_rB, c_A, c_B,
+                    fold_summary<kRuns, kHits>(a, xp, q, lane, p_fi, p_rA, p_rB, c_A, c_B,
                                                  p_f1, p_l1, p_fc, mt_p, mt_c, hits);
                     modeled += static_cast<std::uint64_t>(q.rows) * kWave;
                     write_descs(desc, a.desc_split, a.desc_rid, dq, lane);  // at most one waits
@@ -2439,7 +2485,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPacked ? (k
     if (disorder && a.disorder != nullptr && lane == 0) {
         *a.disorder = 1u;
     }
-    if (kPacked && a.tile_split != nullptr && lane == 0) {
+    if (kRuns && a.tile_split != nullptr && lane == 0) {
         a.tile_split[tile] = any_split ? 1u : 0u;
     }
     __syncthreads();
@@ -3359,12 +3405,14 @@ __device__ __forceinline__ void fold_apply(const KArgs& a, const std::uint64_t* 
 // (P = lead with contention, else the issue time).  Rows are stored whole:
 // lane j of a row takes the run its record belongs to, found by walking the
 // runs row by row (a row's second run starts at a nonzero lane).
+template <bool kGiven>
 __device__ __forceinline__ void fold_apply_runs(const KArgs& a, const std::uint64_t* xp,
                                                 const LinBatchT<true>& q, int lane,
                                                 std::uint64_t* p_busy, std::uint64_t* c_busy,
                                                 std::uint32_t* p_tag, std::uint64_t* completion,
                                                 std::uint8_t* status, ApplySums& t,
-                                                std::uint64_t* mt_p, std::uint64_t* mt_c)
+                                                std::uint64_t* mt_p, std::uint64_t* mt_c,
+                                                const std::uint8_t* hits)
 {
     const StepView v = step_view(a, xp, q, lane);
     const bool m = v.m;
@@ -3380,7 +3428,11 @@ __device__ __forceinline__ void fold_apply_runs(const KArgs& a, const std::uint6
     if (gp.pred < 0) {
         prev1 = tag;
     }
-    const bool lhit = m && prev1 == q.page1;
+    bool lhit = m && prev1 == q.page1;
+    if constexpr (kGiven) {
+        const std::size_t at = run_record(q, lane);
+        lhit = m && hits[at] != 0;
+    }
     const std::uint64_t ls = lhit ? 0ull : a.read_ps;
     const std::uint64_t rm = m ? q.m : 1u;
     const std::uint64_t x = v.x;
@@ -3671,8 +3723,8 @@ __device__ __forceinline__ void fold_batch(const KArgs& a, const std::uint64_t* 
 {
     if constexpr (kR) {
         if (q.any_split()) {
-            fold_apply_runs(a, xp, q, lane, p_busy, c_busy, p_tag, completion, status, t, mt_p,
-                            mt_c);
+            fold_apply_runs<kGiven>(a, xp, q, lane, p_busy, c_busy, p_tag, completion, status, t,
+                                    mt_p, mt_c, hits);
             q.clear();
             return;
         }
@@ -4136,7 +4188,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWide ? 4 : 
     if (kind == kTilePlain) {
         return;  // k_plain_apply took it
     }
-    if constexpr (kPacked) {
+    if constexpr (!kRefresh) {
         if (kind != 0) {
             apply_tile<kRefresh, kHits, kStaged, kPacked, true, kWide>(
                 a, rec, n, base_ps, pcarry, tmask, ccarry, tile_seq, completion, status, tile_rep,
@@ -6335,9 +6387,9 @@ bool plain_run(const KArgs& a, bool ranges_pack)
            plain_summary_lds(a) <= 65536 && plain_apply_lds(a) <= 65536;
 }
 
-// Runs of up to this many records take the scattered-record passes alone,
-// whatever their steps look like: tiles are at most four steps, so that what a
-// run of lines costs there is less than the two launches the mixed form adds.
+// Runs of up to this many records in tiles of at most four steps take the
+// scattered-record passes alone, whatever their steps look like: what a run of
+// lines costs there is less than the two launches the mixed form adds.
 constexpr std::size_t kPlainAlone = std::size_t{1} << 18;
 
 void choose_match(KArgs& a, bool ranges_pack)
@@ -7099,7 +7151,7 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
                         e->d_gccarry, e->d_gcount, e->d_gseq, e->d_tile_rep, nullptr,
                         e->d_tsplit};
     }
-    if (packed) {
+    if (!refresh_records) {
         a.tile_split = sc.tsplit;  // the summary pass marks tiles with split steps
     }
     choose_match(a, e->ranges_pack);
@@ -7195,12 +7247,11 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
     // lines.  An engine whose last run mostly hit its page registers (runs of
     // lines) does not look for them.
     const bool plain = !grouping && !k2 && !refresh_records && plain_run(a, e->ranges_pack);
-    const bool plain_alone = plain && n <= kPlainAlone;
+    const bool plain_alone = plain && n <= kPlainAlone && a.tile <= 256;
     const bool plain_mixed = plain && !plain_alone &&
                              (e->last_modeled == 0 || e->last_hits * 8 < e->last_modeled);
     a.mixed = plain_mixed ? 1u : 0u;
     if (plain_alone || plain_mixed) {
-        a.tile_split = sc.tsplit;
         a.r_top = 1;
         while (a.r_top * 2 <= a.r_count) {
             a.r_top *= 2;
