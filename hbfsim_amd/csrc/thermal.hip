@@ -717,17 +717,49 @@ MarchLaunch march_launcher(std::uint32_t s, int f = 1)
     }
 }
 
-// The marching stencil takes grids of at least kMarchMinCells cells with up
+// The marching stencil takes grids of at least march_min_cells cells with up
 // to 16 layers at 1-4 sweeps per step, up to 8 layers at 5-8 sweeps, at
-// least two strips wide and eight rows per sweep long, whose rings fit the
+// least two strips wide and eight rows per level long, whose rings fit the
 // workgroup's LDS limit.  Returns the LDS bytes, 0 when it does not apply.
-constexpr std::size_t kMarchMinCells = std::size_t{1} << 21;
+//
+// A grid that tiles hold too takes whichever is faster.  Six steps, tiles
+// against the march: 1 sweep at 200 x 180 x 8 68 -> 39 us, 600 x 500 x 1
+// 59 -> 37; 2 sweeps 79 -> 71 and 63 -> 58; 3 and 4 sweeps win from a
+// million cells (4 sweeps: 1100 x 1000 x 1 150 -> 116, 500 x 500 x 8 365 ->
+// 170) and with few layers lose below (600 x 500 x 1 77 -> 109).  At 5 and
+// more sweeps it is no clear gain (300 x 330 x 6 at 8: 381 and 330 us,
+// 130 x 2100 x 1 107 and 254).
+constexpr std::size_t kMarchMinCells = std::size_t{1} << 21;  // with no tile, or 5-8 sweeps
+
+std::size_t march_min_cells(std::uint32_t sweeps, bool tiled)
+{
+    if (!tiled || sweeps > 4) {
+        return kMarchMinCells;
+    }
+    return std::size_t{1} << (sweeps <= 2 ? 18 : 20);
+}
+
+// Fused passes (two steps per read and write of the grid) against single
+// ones: always at 1-3 sweeps (1000 x 1003 x 8: 145 us fused, 235 single for
+// six steps of 2 sweeps).  At 4 the fused pass's 8 levels cost more in halo
+// and in rows per segment than the traffic they save while temperatures in
+// and out and the power (24 B per cell) stay in the 256 MB of shared cache
+// (1000 x 1003 x 8: 282 single, 326 fused; 500 x 500 x 8 170 and 184); past
+// it the fused pass wins (2000 x 2000 x 8: 941 fused, 1065 single).
+constexpr std::size_t kMarchCacheBytes = std::size_t{256} << 20;
+
+bool march_fused(const hbfsim_amd_thermal_grid& g)
+{
+    return g.sweeps < 4 || 24ull * g.nx * g.ny * g.nz > kMarchCacheBytes;
+}
 
 // f = 2: the fused pass of two steps (2 sweeps levels), under the same rules.
-std::size_t march_lds(const hbfsim_amd_thermal_grid& g, std::size_t lds_limit, int f = 1)
+std::size_t march_lds(const hbfsim_amd_thermal_grid& g, std::size_t lds_limit, bool tiled,
+                      int f = 1)
 {
     const std::size_t cells = static_cast<std::size_t>(g.nx) * g.ny * g.nz;
-    if (march_kernel(g.sweeps, f) == nullptr || g.nz > 16 || cells < kMarchMinCells) {
+    if (march_kernel(g.sweeps, f) == nullptr || g.nz > 16 ||
+        cells < march_min_cells(g.sweeps, tiled)) {
         return 0;
     }
     const std::uint32_t levels = g.sweeps * static_cast<std::uint32_t>(f);
@@ -1196,7 +1228,7 @@ int thermal_create(const hbfsim_amd_thermal_grid& g, thermal** out)
     // steps take LDS tiles or, on large grids, the marching kernel
     std::uint32_t tx, ty;
     choose_tile(g.nx, g.ny, g.nz, g.sweeps, 16, 16, tx, ty);
-    if (tx == 0 && march_lds(g, lds_limit) == 0) {
+    if (tx == 0 && march_lds(g, lds_limit, false) == 0) {
         return HBFSIM_UNSUPPORTED;
     }
     auto* th = new (std::nothrow) thermal;
@@ -1309,10 +1341,10 @@ std::uint32_t tile_blocks(const TArgs& a)
 // scattered pieces of them, which measured faster than equal row counts.
 
 // One pass form (f steps per pass): its launch geometry.
-hipError_t setup_march_form(thermal* th, int f)
+hipError_t setup_march_form(thermal* th, bool tiled, int f)
 {
     const auto& g = th->grid;
-    const std::size_t lds = march_lds(g, th->lds_per_block, f);
+    const std::size_t lds = march_lds(g, th->lds_per_block, tiled, f);
     if (lds == 0) {
         return hipSuccess;
     }
@@ -1332,7 +1364,12 @@ hipError_t setup_march_form(thermal* th, int f)
     const std::uint32_t strips = (g.nx + W - 1) / W;
     const std::uint64_t round = static_cast<std::uint64_t>(per_cu) * th->cus;
     std::uint64_t segs = round / strips;
-    const std::uint64_t max_segs = g.ny / (8ull * levels);  // segments of >= 8 L rows
+    // A segment walks 2 L rows more than it writes; shorter ones still pay
+    // until 2 L written rows, since a grid of one round takes as long as one
+    // segment's walk (six steps of 4 sweeps, segments of >= 8 L rows and of
+    // >= 2 L: 700 x 500 x 8 206 -> 187 us single, 294 -> 204 fused;
+    // 1000 x 1003 x 8 309 -> 282 single)
+    const std::uint64_t max_segs = g.ny / (2ull * levels);
     segs = std::max<std::uint64_t>(1, std::min(segs, max_segs));
     const std::uint32_t seg_len = static_cast<std::uint32_t>((g.ny + segs - 1) / segs);
     segs = (g.ny + seg_len - 1) / seg_len;
@@ -1362,9 +1399,13 @@ hipError_t setup_march(thermal* th)
     if (th->cus <= 0) {
         return hipSuccess;
     }
-    hipError_t err = setup_march_form(th, 1);
+    std::uint32_t tx, ty;
+    (void)choose_step_tile(th->grid, th->lds_per_block, tx, ty);
+    hipError_t err = setup_march_form(th, tx != 0, 1);
     if (err == hipSuccess && th->m_lds[0] != 0) {
-        err = setup_march_form(th, 2);
+        if (march_fused(th->grid)) {
+            err = setup_march_form(th, tx != 0, 2);
+        }
         th->march = err == hipSuccess;
     }
     return err;
@@ -1412,8 +1453,9 @@ int thermal_step(thermal* th, const double* d_power, double* d_temp, std::uint64
         }
     }
     const std::size_t cells = static_cast<std::size_t>(g.nx) * g.ny * g.nz;
-    // Passes: on the marching kernel pairs of steps in fused passes (the
-    // power is the same in both) and the odd step in a single-step one.
+    // Passes: on the marching kernel pairs of steps in fused passes where
+    // they pay (the power is the same in both), the others in single-step
+    // ones.
     const std::uint64_t pairs = th->march && th->m_lds[1] != 0 ? steps / 2 : 0;
     const std::uint64_t launches = steps - pairs;
     // Each pass reads one buffer and writes another.  An even count
