@@ -36,6 +36,7 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <optional>
 #include <type_traits>
 #include <vector>
 
@@ -6110,9 +6111,10 @@ __global__ __launch_bounds__(kEmpChain) void k_emp_tail(const TailMap* maps, std
 //   k_k2_first   per plane, the first record (optionally: whose page differs
 //                from a given one) -- the fill events before both slots hold
 //                a page; only run while some plane has an empty slot;
-//   k_k2_last    per tile and plane, the last page other than slot 1's;
-//   k_k2_up/mid/down  the carry of that page across tiles;
-//   k_k2_hits    one hit byte per record.
+//   k_k2_hits    one hit byte per record, and per tile and plane the first and
+//                the last record on a page other than slot 1's;
+//   k_k2_up/mid/down  the carry of that page across tiles; the last level
+//                settles each first record's hit, which needs the carry.
 struct K2Plane {
     std::uint64_t start3;  // first record index with both slots held
     std::uint64_t miss1, miss2;  // fill events before that (or ~0)
@@ -6185,43 +6187,148 @@ __global__ __launch_bounds__(256) void k_k2_page(KArgs a, const hbf_record32* re
     }
 }
 
-__global__ __launch_bounds__(64) void k_k2_last(KArgs a, const hbf_record32* rec, std::size_t n,
+// A tile's first record on a plane whose page is not slot 1's: its hit byte is
+// settled by k_k2_down.  Valid where tile_last is nonzero.
+struct K2First {
+    std::uint32_t page1;
+    std::uint32_t at;  // index in the tile
+};
+
+// The wave of a tile walks its records once.  Only a tile's first record off
+// slot 1's page on a plane depends on earlier tiles, so all other hits are
+// written here, and the records are read and decoded once instead of by one
+// pass for the carry and one for the hits.  Records arrive through the
+// pipeline of the timing passes (four steps in flight), and steps of one or
+// two linear runs are classified by run: every record of a run after its first
+// hits the page the first one left in a register.
+// The paged-KV step of 73M records with two registers: 2981 -> 2369 us, of
+// which this pass takes 776 (3.1 TB/s).
+__global__ __launch_bounds__(64) void k_k2_hits(KArgs a, const hbf_record32* rec, std::size_t n,
                                                 std::uint64_t base_ps, const K2Plane* kp,
-                                                std::uint32_t* tile_last)
+                                                std::uint32_t* tile_last, K2First* tile_first,
+                                                std::uint8_t* hits)
 {
     extern __shared__ std::uint64_t sm[];
     std::uint64_t* fence = sm;
-    std::uint32_t* t1 = reinterpret_cast<std::uint32_t*>(fence + a.r_nfence);
+    // per 64 planes, those that still fill a slot at or after this tile's start
+    std::uint64_t* late = fence + a.r_nfence;
+    const std::uint32_t words = (a.Rp + kWave - 1) / kWave;
+    std::uint32_t* t1 = reinterpret_cast<std::uint32_t*>(late + words);
     std::uint32_t* last = t1 + a.Rp;
     const int lane = threadIdx.x;
-    load_fences(a, fence, lane);
-    for (std::uint32_t r = lane; r < a.Rp; r += kWave) {
-        t1[r] = kp[r].t1;
-        last[r] = 0;
-    }
-    __syncthreads();
     const std::size_t tile = blockIdx.x;
     const std::size_t begin = tile * a.tile;
     const std::size_t end = begin + a.tile < n ? begin + a.tile : n;
+    RecordPipe pipe;
+    pipe.issue(rec, begin, end, lane);
+    load_fences(a, fence, lane);
+    for (std::uint32_t w = 0; w < words; ++w) {
+        const std::uint32_t r = w * kWave + static_cast<std::uint32_t>(lane);
+        bool l = false;
+        if (r < a.Rp) {
+            t1[r] = kp[r].t1;
+            last[r] = 0;
+            l = kp[r].start3 > begin;
+        }
+        const std::uint64_t m = __ballot(l);
+        if (lane == 0) {
+            late[w] = m;
+        }
+    }
+    __syncthreads();
+    // the hit of a modeled record before both of its plane's slots hold a page
+    const auto filling = [&](std::uint32_t plane, std::size_t i, bool hit) {
+        if (((late[plane / kWave] >> (plane % kWave)) & 1u) != 0) {
+            const K2Plane& k = kp[plane];
+            if (i < k.start3) {
+                hit = i != k.miss1 && i != k.miss2;
+            }
+        }
+        return hit;
+    };
     RangeCache rc = empty_cache();
-    for (std::size_t s = begin; s < end; s += kWave) {
-        const std::size_t i = s + lane;
-        const bool valid = i < end;
-        Dec d = invalid_dec();
-        if (valid) {
+    RangeCache rcu = empty_cache();  // wave-uniform copy for linear steps
+    std::uint32_t lin_miss = 0;
+    constexpr std::size_t kSpan = static_cast<std::size_t>(kPipe) * kWave;
+    for (std::size_t g = begin; g < end; g += kSpan) {
+        pipe.advance(rec, g + kSpan, end, lane);
+        const std::size_t gend = g + kSpan < end ? g + kSpan : end;
+        for (std::size_t s = g; s < gend; s += kWave) {
+            Step32 st;
+            pipe.take(st);
+            const std::size_t i = s + lane;
+            if (lin_miss < kLinGiveUp || (s / kWave) % kLinProbe == 0) {
+                LinStep ls;
+                const bool lin = detect_step<false, true>(a, fence, rcu, st, base_ps,
+                                                          s + kWave <= end, lane, ls);
+                lin_miss = lin ? 0u : lin_miss + 1u;
+                if (lin) {
+                    bool hit = true;
+                    std::uint32_t plane = 0;
+                    for (std::uint32_t part = 0; part < (ls.k != 0 ? 2u : 1u); ++part) {
+                        const std::uint32_t page1 = part == 0 ? ls.page1 : ls.page1b;
+                        const std::uint32_t lo = part == 0 ? 0u : ls.k;
+                        Dec d;
+                        d.plane = 0;
+                        d.chan = 0;
+                        stripe(a, page1 - 1u, d);
+                        if (static_cast<std::uint32_t>(lane) >= lo) {
+                            plane = d.plane;
+                        }
+                        if (page1 == t1[d.plane]) {
+                            continue;  // slot 1's page
+                        }
+                        const std::uint32_t prev1 = last[d.plane];
+                        __syncthreads();  // read before it changes
+                        if (static_cast<std::uint32_t>(lane) == lo) {
+                            hit = prev1 == page1;
+                            last[d.plane] = page1;
+                            if (prev1 == 0) {
+                                tile_first[tile * a.Rp + d.plane] =
+                                    K2First{page1, static_cast<std::uint32_t>(i - begin)};
+                            }
+                        }
+                        __syncthreads();
+                    }
+                    hits[i] = filling(plane, i, hit) ? 1u : 0u;
+                    continue;
+                }
+            }
+            const bool valid = i < end;
             uint4 x, y;
-            load_record(rec, i, x, y);
-            d = decode<false>(a, fence, rc, x, y, base_ps);
-        }
-        const std::uint32_t page1 = static_cast<std::uint32_t>(d.page1);
-        const bool nt = valid && d.cls == kClsModeled && page1 != t1[d.plane];
-        const std::uint64_t active = __ballot(nt);
-        if (active == 0) {
-            continue;
-        }
-        const Group g = group_by(nt ? d.plane : 0u, a.pbits, nt, active, lane);
-        if (nt && lane == g.last) {
-            last[d.plane] = page1;
+            step_records(st, lane, x, y);
+            Dec d = invalid_dec();
+            if (valid) {
+                d = decode<false>(a, fence, rc, x, y, base_ps);
+            }
+            const bool m = valid && d.cls == kClsModeled;
+            const std::uint32_t page1 = static_cast<std::uint32_t>(d.page1);
+            const bool nt = m && page1 != t1[d.plane];
+            const std::uint64_t active = __ballot(nt);
+            bool hit = m && !nt;  // slot 1's page
+            if (active != 0) {
+                const Group gr = group_by(nt ? d.plane : 0u, a.pbits, nt, active, lane);
+                std::uint32_t prev1 = static_cast<std::uint32_t>(
+                    __shfl(static_cast<int>(page1), gr.pred < 0 ? lane : gr.pred));
+                if (gr.pred < 0) {
+                    prev1 = nt ? last[d.plane] : 0u;
+                }
+                __syncthreads();  // every lane has read `last` before it changes
+                if (nt) {
+                    hit = prev1 == page1;
+                    if (prev1 == 0) {
+                        tile_first[tile * a.Rp + d.plane] =
+                            K2First{page1, static_cast<std::uint32_t>(i - begin)};
+                    }
+                    if (lane == gr.last) {
+                        last[d.plane] = page1;
+                    }
+                }
+                __syncthreads();
+            }
+            if (valid) {
+                hits[i] = (m ? filling(d.plane, i, hit) : false) ? 1u : 0u;
+            }
         }
     }
     __syncthreads();
@@ -6267,11 +6374,14 @@ __global__ __launch_bounds__(256) void k_k2_mid(KArgs a, std::size_t ngroups, co
     final_last[r] = v;
 }
 
-// Level 3: the page before each tile.
+// Level 3: the page before each tile, which settles the hit of the tile's first
+// record on a page other than slot 1's (once both slots hold a page).
 __global__ __launch_bounds__(256) void k_k2_down(KArgs a, std::size_t ntiles, std::size_t ngroups,
+                                                 const K2Plane* kp,
                                                  const std::uint32_t* tile_last,
+                                                 const K2First* tile_first,
                                                  const std::uint32_t* group_in,
-                                                 std::uint32_t* tile_in)
+                                                 std::uint8_t* hits)
 {
     const std::size_t t = blockIdx.x * static_cast<std::size_t>(blockDim.x) + threadIdx.x;
     if (t >= ngroups * a.Rp) {
@@ -6279,72 +6389,17 @@ __global__ __launch_bounds__(256) void k_k2_down(KArgs a, std::size_t ntiles, st
     }
     const std::size_t g = t / a.Rp, r = t % a.Rp;
     std::uint32_t v = group_in[g * a.Rp + r];
+    const std::uint64_t start3 = kp[r].start3;
     const std::size_t e = (g + 1) * kGroup < ntiles ? (g + 1) * kGroup : ntiles;
     for (std::size_t k = g * kGroup; k < e; ++k) {
-        tile_in[k * a.Rp + r] = v;
         const std::uint32_t x = tile_last[k * a.Rp + r];
-        v = x != 0 ? x : v;
-    }
-}
-
-__global__ __launch_bounds__(64) void k_k2_hits(KArgs a, const hbf_record32* rec, std::size_t n,
-                                                std::uint64_t base_ps, const K2Plane* kp,
-                                                const std::uint32_t* tile_in, std::uint8_t* hits)
-{
-    extern __shared__ std::uint64_t sm[];
-    std::uint64_t* fence = sm;
-    std::uint32_t* t1 = reinterpret_cast<std::uint32_t*>(fence + a.r_nfence);
-    std::uint32_t* last = t1 + a.Rp;
-    const int lane = threadIdx.x;
-    const std::size_t tile = blockIdx.x;
-    load_fences(a, fence, lane);
-    for (std::uint32_t r = lane; r < a.Rp; r += kWave) {
-        t1[r] = kp[r].t1;
-        last[r] = tile_in[tile * a.Rp + r];
-    }
-    __syncthreads();
-    const std::size_t begin = tile * a.tile;
-    const std::size_t end = begin + a.tile < n ? begin + a.tile : n;
-    RangeCache rc = empty_cache();
-    for (std::size_t s = begin; s < end; s += kWave) {
-        const std::size_t i = s + lane;
-        const bool valid = i < end;
-        Dec d = invalid_dec();
-        if (valid) {
-            uint4 x, y;
-            load_record(rec, i, x, y);
-            d = decode<false>(a, fence, rc, x, y, base_ps);
-        }
-        const bool m = valid && d.cls == kClsModeled;
-        const std::uint32_t page1 = static_cast<std::uint32_t>(d.page1);
-        const std::uint32_t pt1 = m ? t1[d.plane] : 0u;
-        const bool nt = m && page1 != pt1;
-        const std::uint64_t active = __ballot(nt);
-        bool hit = false;
-        if (active != 0) {
-            const Group g = group_by(nt ? d.plane : 0u, a.pbits, nt, active, lane);
-            std::uint32_t prev1 = static_cast<std::uint32_t>(
-                __shfl(static_cast<int>(page1), g.pred < 0 ? lane : g.pred));
-            if (g.pred < 0) {
-                prev1 = nt ? last[d.plane] : 0u;
+        if (x != 0) {
+            const K2First f = tile_first[k * a.Rp + r];
+            const std::size_t i = k * a.tile + f.at;
+            if (i >= start3) {
+                hits[i] = f.page1 == v ? 1u : 0u;
             }
-            hit = nt && prev1 == page1;
-            __syncthreads();  // every lane has read `last` before it changes
-            if (nt && lane == g.last) {
-                last[d.plane] = page1;
-            }
-            __syncthreads();
-        }
-        if (m) {
-            const K2Plane& k = kp[d.plane];
-            if (i < k.start3) {
-                hit = i != k.miss1 && i != k.miss2;
-            } else if (!nt) {
-                hit = true;  // slot 1's page
-            }
-            hits[i] = hit ? 1u : 0u;
-        } else if (valid) {
-            hits[i] = 0;
+            v = x;
         }
     }
 }
@@ -6670,35 +6725,32 @@ int k2_hits(engine* e, KArgs a, const hbf_record32* d_rec, std::size_t n,
         const std::uint64_t t0 = tags[2 * r], t1 = tags[2 * r + 1];
         need_a = need_a || (t0 == 0 && t1 == 0);
     }
-    std::uint32_t* d_want = nullptr;
-    std::uint32_t* d_differ = nullptr;
-    unsigned long long* d_first = nullptr;
-    std::uint32_t* d_page = nullptr;
-    K2Plane* d_kp = nullptr;
     const std::size_t ngroups = (ntiles + kGroup - 1) / kGroup;
-    std::uint32_t* d_tlast = nullptr;
-    std::uint32_t* d_tin = nullptr;
-    std::uint32_t* d_glast = nullptr;
-    std::uint32_t* d_gin = nullptr;
-    std::uint32_t* d_final = nullptr;
-    auto release = [&]() {
-        hfree(d_want); hfree(d_differ); hfree(d_first); hfree(d_page); hfree(d_kp);
-        hfree(d_tlast); hfree(d_tin); hfree(d_glast); hfree(d_gin); hfree(d_final);
-    };
-    err = halloc(d_want, rp);
-    if (err == hipSuccess) err = halloc(d_differ, rp);
-    if (err == hipSuccess) err = halloc(d_first, rp);
-    if (err == hipSuccess) err = halloc(d_page, rp);
-    if (err == hipSuccess) err = halloc(d_kp, rp);
-    if (err == hipSuccess) err = halloc(d_tlast, ntiles * rp);
-    if (err == hipSuccess) err = halloc(d_tin, ntiles * rp);
-    if (err == hipSuccess) err = halloc(d_glast, ngroups * rp);
-    if (err == hipSuccess) err = halloc(d_gin, ngroups * rp);
-    if (err == hipSuccess) err = halloc(d_final, rp);
-    if (err != hipSuccess) {
-        release();
+    ScratchPlan plan;
+    const std::size_t o_want = plan.add<std::uint32_t>(rp);
+    const std::size_t o_differ = plan.add<std::uint32_t>(rp);
+    const std::size_t o_first = plan.add<unsigned long long>(rp);
+    const std::size_t o_page = plan.add<std::uint32_t>(rp);
+    const std::size_t o_kp = plan.add<K2Plane>(rp);
+    const std::size_t o_tlast = plan.add<std::uint32_t>(ntiles * rp);
+    const std::size_t o_tfirst = plan.add<K2First>(ntiles * rp);
+    const std::size_t o_glast = plan.add<std::uint32_t>(ngroups * rp);
+    const std::size_t o_gin = plan.add<std::uint32_t>(ngroups * rp);
+    const std::size_t o_final = plan.add<std::uint32_t>(rp);
+    ScratchLease lease(plan.bytes, stream);
+    if (!lease.ok()) {
         return HBFSIM_CUDA_ERROR;
     }
+    auto* d_want = lease.at<std::uint32_t>(o_want);
+    auto* d_differ = lease.at<std::uint32_t>(o_differ);
+    auto* d_first = lease.at<unsigned long long>(o_first);
+    auto* d_page = lease.at<std::uint32_t>(o_page);
+    auto* d_kp = lease.at<K2Plane>(o_kp);
+    auto* d_tlast = lease.at<std::uint32_t>(o_tlast);
+    auto* d_tfirst = lease.at<K2First>(o_tfirst);
+    auto* d_glast = lease.at<std::uint32_t>(o_glast);
+    auto* d_gin = lease.at<std::uint32_t>(o_gin);
+    auto* d_final = lease.at<std::uint32_t>(o_final);
     const unsigned first_blocks = static_cast<unsigned>((n + kK2Chunk - 1) / kK2Chunk);
     const std::size_t lds_first = 8ull * a.r_nfence + 8ull * rp;
     // pass A: the first record of every plane with both slots empty
@@ -6755,7 +6807,6 @@ int k2_hits(engine* e, KArgs a, const hbf_record32* d_rec, std::size_t n,
         }
     }
     if (err != hipSuccess) {
-        release();
         return HBFSIM_CUDA_ERROR;
     }
     for (std::uint32_t r = 0; r < rp; ++r) {
@@ -6794,30 +6845,28 @@ int k2_hits(engine* e, KArgs a, const hbf_record32* d_rec, std::size_t n,
     }
     err = hipMemcpyAsync(d_kp, kp.data(), rp * sizeof(K2Plane), hipMemcpyHostToDevice, stream);
     if (err != hipSuccess) {
-        release();
         return HBFSIM_CUDA_ERROR;
     }
-    const std::size_t lds = 8ull * a.r_nfence + 8ull * rp;
+    const std::size_t lds = 8ull * (a.r_nfence + (rp + kWave - 1) / kWave) + 8ull * rp;
     const unsigned wide = static_cast<unsigned>((ngroups * rp + 255) / 256);
-    hipLaunchKernelGGL(k_k2_last, dim3(static_cast<unsigned>(ntiles)), dim3(kWave), lds, stream, a,
-                       d_rec, n, base_ps, static_cast<const K2Plane*>(d_kp), d_tlast);
+    hipLaunchKernelGGL(k_k2_hits, dim3(static_cast<unsigned>(ntiles)), dim3(kWave), lds, stream, a,
+                       d_rec, n, base_ps, static_cast<const K2Plane*>(d_kp), d_tlast, d_tfirst,
+                       d_hits);
     hipLaunchKernelGGL(k_k2_up, dim3(wide), dim3(256), 0, stream, a, ntiles, ngroups,
                        static_cast<const std::uint32_t*>(d_tlast), d_glast);
     hipLaunchKernelGGL(k_k2_mid, dim3((rp + 255) / 256), dim3(256), 0, stream, a, ngroups,
                        static_cast<const K2Plane*>(d_kp), static_cast<const std::uint32_t*>(d_glast),
                        d_gin, d_final);
     hipLaunchKernelGGL(k_k2_down, dim3(wide), dim3(256), 0, stream, a, ntiles, ngroups,
-                       static_cast<const std::uint32_t*>(d_tlast),
-                       static_cast<const std::uint32_t*>(d_gin), d_tin);
-    hipLaunchKernelGGL(k_k2_hits, dim3(static_cast<unsigned>(ntiles)), dim3(kWave), lds, stream, a,
-                       d_rec, n, base_ps, static_cast<const K2Plane*>(d_kp),
-                       static_cast<const std::uint32_t*>(d_tin), d_hits);
+                       static_cast<const K2Plane*>(d_kp), static_cast<const std::uint32_t*>(d_tlast),
+                       static_cast<const K2First*>(d_tfirst),
+                       static_cast<const std::uint32_t*>(d_gin), d_hits);
     std::vector<std::uint32_t> fin(rp);
     err = hipGetLastError();
     if (err == hipSuccess)
         err = hipMemcpyAsync(fin.data(), d_final, rp * 4, hipMemcpyDeviceToHost, stream);
     if (err == hipSuccess) err = hipStreamSynchronize(stream);
-    release();
+    lease.synced();
     if (err != hipSuccess) {
         return HBFSIM_CUDA_ERROR;
     }
@@ -7201,16 +7250,18 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
     }
     // two page registers: hits first, from their own scans
     const bool k2 = e->cfg.slots == 2;
+    std::optional<ScratchLease> hit_lease;
     std::uint8_t* d_hits = nullptr;
     std::vector<std::uint64_t> k2_tags;
     if (k2) {
-        if (halloc(d_hits, n) != hipSuccess) {
+        hit_lease.emplace(n, stream);
+        if (!hit_lease->ok()) {
             return HBFSIM_CUDA_ERROR;
         }
+        d_hits = hit_lease->at<std::uint8_t>(0);
         st = k2_hits(e, a, static_cast<const hbf_record32*>(d_rec), n, base_ps, ntiles, stream,
                      d_hits, k2_tags);
         if (st != HBFSIM_OK) {
-            hfree(d_hits);
             return st;
         }
         a.ext_hits = 1;
@@ -7406,7 +7457,10 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
                              stream);
         if (err == hipSuccess) err = hipStreamSynchronize(stream);
     }
-    hfree(d_hits);
+    if (err == hipSuccess && hit_lease) {
+        hit_lease->synced();
+    }
+    hit_lease.reset();
     free_group();
     if (err != hipSuccess) {
         return HBFSIM_CUDA_ERROR;
