@@ -5148,6 +5148,13 @@ struct engine {
     std::vector<range_rec> ranges;
     bool ranges_dirty{true};
     bool ranges_pack{false};  // the range table fits its packed form in LDS
+    // The arrays of one purpose lie in one allocation (an engine's first run
+    // spent most of its time in some thirty small ones).
+    unsigned char* range_block{nullptr};
+    unsigned char* state_block{nullptr};
+    std::size_t state_bytes{0};  // of state_block, that a reset clears
+    unsigned char* tile_block{nullptr};
+    unsigned char* desc_block{nullptr};
     std::uint64_t* d_r_base{nullptr};
     std::uint64_t* d_r_length{nullptr};
     std::uint64_t* d_r_offset{nullptr};
@@ -5292,6 +5299,13 @@ hipError_t halloc(T*& p, std::size_t count)
     return err;
 }
 
+// An array of a block laid out by a ScratchPlan.
+template <typename T>
+void place(T*& p, unsigned char* block, std::size_t at)
+{
+    p = reinterpret_cast<T*>(block + at);
+}
+
 std::uint32_t bits_for(std::uint32_t n)
 {
     std::uint32_t b = 0;
@@ -5314,24 +5328,8 @@ std::uint32_t log2u(std::uint64_t v)
 
 void free_scratch(engine* e)
 {
-    hfree(e->d_psum);
-    hfree(e->d_tmask);
-    hfree(e->d_csum);
-    hfree(e->d_pcarry);
-    hfree(e->d_ccarry);
-    hfree(e->d_tcount);
-    hfree(e->d_tseq);
-    hfree(e->d_gpsum);
-    hfree(e->d_gcsum);
-    hfree(e->d_gpcarry);
-    hfree(e->d_gccarry);
-    hfree(e->d_gcount);
-    hfree(e->d_gseq);
-    hfree(e->d_tile_rep);
-    hfree(e->d_tsplit);
-    hfree(e->d_desc);
-    hfree(e->d_desc_rid);
-    hfree(e->d_desc_split);
+    hfree(e->tile_block);
+    hfree(e->desc_block);
     e->desc_cap = 0;
     e->tile_cap = 0;
 }
@@ -5346,24 +5344,42 @@ int ensure_scratch(engine* e, std::size_t ntiles)
     // do not reallocate (freeing device memory synchronises the device)
     const std::size_t cap = std::max<std::size_t>(ntiles + ntiles / 8, 16);
     const std::size_t rp = e->args.Rp, rc = e->args.Rc;
-    if (halloc(e->d_psum, cap * rp) != hipSuccess ||
-        halloc(e->d_tmask, cap * mask_words(e->args)) != hipSuccess ||
-        halloc(e->d_csum, cap * rc) != hipSuccess ||
-        halloc(e->d_pcarry, cap * rp) != hipSuccess ||
-        halloc(e->d_ccarry, cap * rc) != hipSuccess || halloc(e->d_tcount, cap) != hipSuccess ||
-        halloc(e->d_tseq, cap) != hipSuccess) {
-        free_scratch(e);
-        return HBFSIM_CUDA_ERROR;
-    }
     const std::size_t gcap = (cap + kGroup - 1) / kGroup;
-    if (halloc(e->d_gpsum, gcap * rp) != hipSuccess || halloc(e->d_gcsum, gcap * rc) != hipSuccess ||
-        halloc(e->d_gpcarry, gcap * rp) != hipSuccess ||
-        halloc(e->d_gccarry, gcap * rc) != hipSuccess || halloc(e->d_gcount, gcap) != hipSuccess ||
-        halloc(e->d_gseq, gcap) != hipSuccess || halloc(e->d_tile_rep, cap) != hipSuccess ||
-        halloc(e->d_tsplit, cap) != hipSuccess) {
+    ScratchPlan plan;
+    const std::size_t psum = plan.add<PlaneSum>(cap * rp);
+    const std::size_t tmask = plan.add<MaskWord>(cap * mask_words(e->args));
+    const std::size_t csum = plan.add<ChanSum>(cap * rc);
+    const std::size_t pcarry = plan.add<PlaneCarry>(cap * rp);
+    const std::size_t ccarry = plan.add<std::uint64_t>(cap * rc);
+    const std::size_t tcount = plan.add<std::uint64_t>(cap);
+    const std::size_t tseq = plan.add<std::uint64_t>(cap);
+    const std::size_t gpsum = plan.add<PlaneSum>(gcap * rp);
+    const std::size_t gcsum = plan.add<ChanSum>(gcap * rc);
+    const std::size_t gpcarry = plan.add<PlaneCarry>(gcap * rp);
+    const std::size_t gccarry = plan.add<std::uint64_t>(gcap * rc);
+    const std::size_t gcount = plan.add<std::uint64_t>(gcap);
+    const std::size_t gseq = plan.add<std::uint64_t>(gcap);
+    const std::size_t tile_rep = plan.add<DevReport>(cap);
+    const std::size_t tsplit = plan.add<std::uint8_t>(cap);
+    if (halloc(e->tile_block, plan.bytes) != hipSuccess) {
         free_scratch(e);
         return HBFSIM_CUDA_ERROR;
     }
+    place(e->d_psum, e->tile_block, psum);
+    place(e->d_tmask, e->tile_block, tmask);
+    place(e->d_csum, e->tile_block, csum);
+    place(e->d_pcarry, e->tile_block, pcarry);
+    place(e->d_ccarry, e->tile_block, ccarry);
+    place(e->d_tcount, e->tile_block, tcount);
+    place(e->d_tseq, e->tile_block, tseq);
+    place(e->d_gpsum, e->tile_block, gpsum);
+    place(e->d_gcsum, e->tile_block, gcsum);
+    place(e->d_gpcarry, e->tile_block, gpcarry);
+    place(e->d_gccarry, e->tile_block, gccarry);
+    place(e->d_gcount, e->tile_block, gcount);
+    place(e->d_gseq, e->tile_block, gseq);
+    place(e->d_tile_rep, e->tile_block, tile_rep);
+    place(e->d_tsplit, e->tile_block, tsplit);
     e->tile_cap = cap;
     return HBFSIM_OK;
 }
@@ -5371,18 +5387,23 @@ int ensure_scratch(engine* e, std::size_t ntiles)
 int upload_ranges(engine* e, hipStream_t stream)
 {
     const std::size_t count = e->ranges.size();
-    if (count > e->range_cap || e->d_r_base == nullptr) {
-        hfree(e->d_r_base);
-        hfree(e->d_r_length);
-        hfree(e->d_r_offset);
-        hfree(e->d_r_meta);
-        hfree(e->d_r_id);
+    if (count > e->range_cap || e->range_block == nullptr) {
+        hfree(e->range_block);
         const std::size_t cap = std::max<std::size_t>(count, 64);
-        if (halloc(e->d_r_base, cap) != hipSuccess || halloc(e->d_r_length, cap) != hipSuccess ||
-            halloc(e->d_r_offset, cap) != hipSuccess || halloc(e->d_r_meta, cap) != hipSuccess ||
-            halloc(e->d_r_id, cap) != hipSuccess) {
+        ScratchPlan plan;
+        const std::size_t rbase = plan.add<std::uint64_t>(cap);
+        const std::size_t rlength = plan.add<std::uint64_t>(cap);
+        const std::size_t roffset = plan.add<std::uint64_t>(cap);
+        const std::size_t rmeta = plan.add<std::uint32_t>(cap);
+        const std::size_t rid = plan.add<std::uint32_t>(cap);
+        if (halloc(e->range_block, plan.bytes) != hipSuccess) {
             return HBFSIM_CUDA_ERROR;
         }
+        place(e->d_r_base, e->range_block, rbase);
+        place(e->d_r_length, e->range_block, rlength);
+        place(e->d_r_offset, e->range_block, roffset);
+        place(e->d_r_meta, e->range_block, rmeta);
+        place(e->d_r_id, e->range_block, rid);
         e->range_cap = cap;
     }
     std::vector<std::uint64_t> base(count), length(count), offset(count);
@@ -6963,16 +6984,31 @@ int engine_create(const engine_config& c, engine** out)
     }
     a.tile = c.tile;
     a.media_pages = c.media_pages;
-    hipError_t err = halloc(e->d_pbusy, rp);
-    if (err == hipSuccess) err = halloc(e->d_ptag, 2ull * rp);
-    if (err == hipSuccess) err = halloc(e->d_cbusy, rc);
-    if (err == hipSuccess) err = halloc(e->d_ptot, rp);
-    if (err == hipSuccess) err = halloc(e->d_ctot, rc);
-    if (err == hipSuccess) err = halloc(e->d_seq, 1);
-    if (err == hipSuccess) err = halloc(e->d_done, 1);
-    if (err == hipSuccess) err = halloc(e->d_stamp, 4);
-    if (err == hipSuccess) err = halloc(e->d_rep_parts, kRepParts * kRepWords);
-    if (err == hipSuccess) err = halloc(e->d_disorder, 1);
+    ScratchPlan plan;
+    const std::size_t pbusy = plan.add<std::uint64_t>(rp);
+    const std::size_t ptag = plan.add<std::uint64_t>(2ull * rp);
+    const std::size_t cbusy = plan.add<std::uint64_t>(rc);
+    const std::size_t ptot = plan.add<std::uint64_t>(rp);
+    const std::size_t ctot = plan.add<std::uint64_t>(rc);
+    const std::size_t seq = plan.add<std::uint64_t>(1);
+    const std::size_t done = plan.add<std::uint32_t>(1);
+    const std::size_t disorder = plan.add<std::uint32_t>(1);
+    e->state_bytes = plan.bytes;
+    const std::size_t stamp = plan.add<std::uint64_t>(4);
+    const std::size_t rep_parts = plan.add<std::uint64_t>(kRepParts * kRepWords);
+    hipError_t err = halloc(e->state_block, plan.bytes);
+    if (err == hipSuccess) {
+        place(e->d_pbusy, e->state_block, pbusy);
+        place(e->d_ptag, e->state_block, ptag);
+        place(e->d_cbusy, e->state_block, cbusy);
+        place(e->d_ptot, e->state_block, ptot);
+        place(e->d_ctot, e->state_block, ctot);
+        place(e->d_seq, e->state_block, seq);
+        place(e->d_done, e->state_block, done);
+        place(e->d_stamp, e->state_block, stamp);
+        place(e->d_rep_parts, e->state_block, rep_parts);
+        place(e->d_disorder, e->state_block, disorder);
+    }
     if (err == hipSuccess)
         err = hipHostMalloc(reinterpret_cast<void**>(&e->h_out), sizeof(HostOut));
     int khz = 0;
@@ -7004,21 +7040,8 @@ void engine_destroy(engine* e)
     (void)hipSetDevice(e->device);
     (void)hipDeviceSynchronize();
     free_scratch(e);
-    hfree(e->d_r_base);
-    hfree(e->d_r_length);
-    hfree(e->d_r_offset);
-    hfree(e->d_r_meta);
-    hfree(e->d_r_id);
-    hfree(e->d_pbusy);
-    hfree(e->d_ptag);
-    hfree(e->d_cbusy);
-    hfree(e->d_ptot);
-    hfree(e->d_ctot);
-    hfree(e->d_seq);
-    hfree(e->d_done);
-    hfree(e->d_stamp);
-    hfree(e->d_rep_parts);
-    hfree(e->d_disorder);
+    hfree(e->range_block);
+    hfree(e->state_block);
     hfree(e->d_emp_svc);
     if (e->h_out != nullptr) {
         (void)hipHostFree(e->h_out);
@@ -7038,15 +7061,7 @@ int engine_set_ranges(engine* e, const std::vector<range_rec>& ranges)
 
 int engine_reset(engine* e)
 {
-    const std::size_t rp = e->args.Rp, rc = e->args.Rc;
-    hipError_t err = hipMemset(e->d_pbusy, 0, rp * 8);
-    if (err == hipSuccess) err = hipMemset(e->d_ptag, 0, rp * 16);
-    if (err == hipSuccess) err = hipMemset(e->d_cbusy, 0, rc * 8);
-    if (err == hipSuccess) err = hipMemset(e->d_ptot, 0, rp * 8);
-    if (err == hipSuccess) err = hipMemset(e->d_ctot, 0, rc * 8);
-    if (err == hipSuccess) err = hipMemset(e->d_seq, 0, 8);
-    if (err == hipSuccess) err = hipMemset(e->d_disorder, 0, 4);
-    if (err == hipSuccess) err = hipMemset(e->d_done, 0, 4);
+    hipError_t err = hipMemset(e->state_block, 0, e->state_bytes);
     if (err == hipSuccess) err = hipDeviceSynchronize();
     e->burst = 0;
     return hip_status(err);
@@ -7284,16 +7299,20 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
     } else if ((k2 || a.slots == 1) && !grouping) {
         const std::size_t nsteps = (n + kWave - 1) / kWave;
         if (nsteps > e->desc_cap) {
-            hfree(e->d_desc);
-            hfree(e->d_desc_rid);
-            hfree(e->d_desc_split);
+            hfree(e->desc_block);
             e->desc_cap = 0;
             const std::size_t cap = nsteps + nsteps / 8;  // headroom, as for the tiles
-            if (halloc(e->d_desc, cap) != hipSuccess || halloc(e->d_desc_rid, cap) != hipSuccess ||
-                halloc(e->d_desc_split, cap) != hipSuccess) {
+            ScratchPlan plan;
+            const std::size_t steps = plan.add<StepDesc>(cap);
+            const std::size_t rids = plan.add<std::uint32_t>(cap);
+            const std::size_t splits = plan.add<SplitDesc>(cap);
+            if (halloc(e->desc_block, plan.bytes) != hipSuccess) {
                 free_group();
                 return HBFSIM_CUDA_ERROR;
             }
+            place(e->d_desc, e->desc_block, steps);
+            place(e->d_desc_rid, e->desc_block, rids);
+            place(e->d_desc_split, e->desc_block, splits);
             e->desc_cap = cap;
         }
         desc = e->d_desc;
