@@ -1097,6 +1097,7 @@ int calibrate(const hbfsim_amd_access_class* d_access, const std::uint64_t* d_la
     if (n > 0xffffffffull) {
         return HBFSIM_UNSUPPORTED;
     }
+    const ScratchHold hold;  // outlives every lease of the call
     hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
     const std::uint64_t most = most_slots(n, 0);
     std::uint64_t cap = std::min(first_slots(0), most);

@@ -30,6 +30,16 @@ void scratch_trim();
 void scratch_hold();
 void scratch_drop();
 
+// Holds the pool for the scope of a call that needs no engine or sampler: with
+// none alive its blocks are freed when it returns.
+class ScratchHold {
+public:
+    ScratchHold() { scratch_hold(); }
+    ~ScratchHold() { scratch_drop(); }
+    ScratchHold(const ScratchHold&) = delete;
+    ScratchHold& operator=(const ScratchHold&) = delete;
+};
+
 // Lays out several arrays in one block, each 256-byte aligned.
 struct ScratchPlan {
     std::size_t bytes = 0;
