@@ -465,20 +465,56 @@ __global__ __launch_bounds__(kThreads) void k_bucket_sort(Buckets bk, const std:
     }
 }
 
-template <bool kPacked>
-void launch_partition(const void* rec, std::size_t n, const Buckets& bk, ulonglong2* part,
-                      std::uint64_t* key, hipStream_t stream)
+// Lets a histogram kernel have `bytes` of dynamic LDS: beyond 64 KB, its static arrays
+// included, it has to be allowed the size first (16,384 buckets take 64 KB by themselves).
+template <typename F>
+hipError_t allow_hist(F* kernel, std::size_t bytes)
+{
+    if (bytes <= (std::size_t{32} << 10)) {
+        return hipSuccess;
+    }
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                               hipFuncAttributeMaxDynamicSharedMemorySize,
+                               static_cast<int>(bytes));
+}
+
+// Each kernel takes what the one before it wrote for granted (bucket numbers and places are
+// indices), so nothing is launched after one that was refused.
+template <typename T, bool kPacked>
+hipError_t launch_buckets(const void* rec, std::size_t n, const Buckets& bk, ulonglong2* part,
+                          std::uint64_t* key, std::uint32_t* pos, std::uint32_t* place, T* sorted,
+                          hipStream_t stream)
 {
     const std::size_t lds = (std::size_t{1} << bk.log2) * 4;
     const unsigned chunks = static_cast<unsigned>((n + kChunk - 1) / kChunk);
     const unsigned parts = std::min(blocks_for((n + 7) / 8), kRangeParts);
-    hipLaunchKernelGGL(k_issue_range<kPacked>, dim3(parts), dim3(kThreads), 0, stream, rec, n,
-                       part);
-    hipLaunchKernelGGL(k_bucket_count<kPacked>, dim3(chunks), dim3(kThreads), lds, stream, rec, n,
-                       bk, part, parts);
-    hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(1024), 0, stream, bk, n);
-    hipLaunchKernelGGL(k_bucket_scatter<kPacked>, dim3(chunks), dim3(kThreads), lds, stream, rec,
-                       n, bk, key);
+    hipError_t err = allow_hist(k_bucket_count<kPacked>, lds);
+    if (err == hipSuccess) err = allow_hist(k_bucket_scatter<kPacked>, lds);
+    if (err == hipSuccess) {
+        hipLaunchKernelGGL(k_issue_range<kPacked>, dim3(parts), dim3(kThreads), 0, stream, rec, n,
+                           part);
+        err = hipGetLastError();
+    }
+    if (err == hipSuccess) {
+        hipLaunchKernelGGL(k_bucket_count<kPacked>, dim3(chunks), dim3(kThreads), lds, stream, rec,
+                           n, bk, part, parts);
+        err = hipGetLastError();
+    }
+    if (err == hipSuccess) {
+        hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(1024), 0, stream, bk, n);
+        err = hipGetLastError();
+    }
+    if (err == hipSuccess) {
+        hipLaunchKernelGGL(k_bucket_scatter<kPacked>, dim3(chunks), dim3(kThreads), lds, stream,
+                           rec, n, bk, key);
+        err = hipGetLastError();
+    }
+    if (err == hipSuccess) {
+        hipLaunchKernelGGL(k_bucket_sort<T>, dim3(1u << bk.log2), dim3(kThreads), 0, stream, bk,
+                           key, static_cast<const T*>(rec), pos, place, sorted);
+        err = hipGetLastError();
+    }
+    return err;
 }
 
 // The stable order by radix sort: pos receives the positions.  key_a: n words
@@ -586,21 +622,17 @@ int run_in_issue_order(const void* d_rec, bool packed, std::size_t n, std::uint6
         if (err != hipSuccess) {
             return HBFSIM_CUDA_ERROR;
         }
-        if (packed) {
-            launch_partition<true>(d_rec, n, bk, part, key, stream);
-            hipLaunchKernelGGL(k_bucket_sort<hbf_record16>, dim3(static_cast<unsigned>(buckets)),
-                               dim3(kThreads), 0, stream, bk, key,
-                               static_cast<const hbf_record16*>(d_rec), pos, place,
-                               static_cast<hbf_record16*>(sorted));
+        err = packed ? launch_buckets<hbf_record16, true>(d_rec, n, bk, part, key, pos, place,
+                                                          static_cast<hbf_record16*>(sorted),
+                                                          stream)
+                     : launch_buckets<hbf_record32, false>(d_rec, n, bk, part, key, pos, place,
+                                                           static_cast<hbf_record32*>(sorted),
+                                                           stream);
+        if (err != hipSuccess) {
+            (void)hipGetLastError();
+            overflow = 1;  // a launch was refused: the radix sort takes the stream
+            err = hipSuccess;
         } else {
-            launch_partition<false>(d_rec, n, bk, part, key, stream);
-            hipLaunchKernelGGL(k_bucket_sort<hbf_record32>, dim3(static_cast<unsigned>(buckets)),
-                               dim3(kThreads), 0, stream, bk, key,
-                               static_cast<const hbf_record32*>(d_rec), pos, place,
-                               static_cast<hbf_record32*>(sorted));
-        }
-        err = hipGetLastError();
-        if (err == hipSuccess) {
             err = hipMemcpyAsync(&overflow, bk.overflow, 4, hipMemcpyDeviceToHost, stream);
         }
         if (err == hipSuccess) err = hipStreamSynchronize(stream);
