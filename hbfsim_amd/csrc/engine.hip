@@ -6709,7 +6709,7 @@ int run_empirical(engine* e, const hbf_record32* d_rec, std::size_t n, std::uint
     if (err != hipSuccess) {
         return HBFSIM_CUDA_ERROR;
     }
-    lease.synced();
+    lease.synced(err);
     if (e->h_out->back != 0) {
         // a record's issue time goes back: served in (issue, position) order;
         // the engine state is as the run found it
@@ -6897,7 +6897,7 @@ int k2_hits(engine* e, KArgs a, const hbf_record32* d_rec, std::size_t n,
     if (err == hipSuccess)
         err = hipMemcpyAsync(fin.data(), d_final, rp * 4, hipMemcpyDeviceToHost, stream);
     if (err == hipSuccess) err = hipStreamSynchronize(stream);
-    lease.synced();
+    lease.synced(err);
     if (err != hipSuccess) {
         return HBFSIM_CUDA_ERROR;
     }
@@ -7487,7 +7487,7 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
         if (err == hipSuccess) err = hipStreamSynchronize(stream);
     }
     if (err == hipSuccess && hit_lease) {
-        hit_lease->synced();
+        hit_lease->synced(err);
     }
     hit_lease.reset();
     free_group();

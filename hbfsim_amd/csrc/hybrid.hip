@@ -931,7 +931,7 @@ int sampler_reference(sampler_state* s, const hbfsim_amd_access_class* d_access,
             }
             s->seen = total;
         }
-        lease.synced();
+        lease.synced(err);
         break;
     }
     if (references != nullptr) {
@@ -1077,7 +1077,7 @@ int calibrate_rows(const ClassTable& t, const std::uint64_t* d_latency, std::siz
     if (err != hipSuccess) {
         return HBFSIM_CUDA_ERROR;
     }
-    lease.synced();
+    lease.synced(err);
     return HBFSIM_OK;
 }
 

@@ -674,7 +674,7 @@ int run_in_issue_order(const void* d_rec, bool packed, std::size_t n, std::uint6
     if (err != hipSuccess) {
         return HBFSIM_CUDA_ERROR;
     }
-    lease.synced();
+    lease.synced(err);
     return HBFSIM_OK;
 }
 

@@ -52,8 +52,10 @@ struct ScratchPlan {
     }
 };
 
-// One block for the scope of a call.  Unless synced() was called after the
-// last work queued on the block, the destructor waits for the stream first.
+// One block for the scope of a call.  The destructor waits for the stream
+// first, unless synced() was given a success: the result of a wait made after
+// the last work queued on the block (an error instead of it, also one that
+// kept the wait from being made, leaves the wait to the destructor).
 class ScratchLease {
 public:
     ScratchLease(std::size_t bytes, hipStream_t stream)
@@ -69,7 +71,7 @@ public:
     {
         return reinterpret_cast<T*>(static_cast<unsigned char*>(ptr_) + offset);
     }
-    void synced() { idle_ = true; }
+    void synced(hipError_t waited) { idle_ = waited == hipSuccess; }
     void release()
     {
         if (ptr_ != nullptr) {
