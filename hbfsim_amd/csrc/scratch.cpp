@@ -2,6 +2,7 @@
 #include "scratch.hpp"
 
 #include <algorithm>
+#include <initializer_list>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -22,8 +23,13 @@ std::vector<Block>& g_blocks = *new std::vector<Block>;
 
 std::size_t g_holders = 0;
 
+// An idle block serves requests of at least half its size: a small request must not keep a large
+// block from the next large one.
+constexpr std::size_t kFitMost = 2;
+
 // Takes the idle blocks of `device` (-1: of every device) out of the list, oldest first, until at
-// most `keep` idle bytes remain; the caller frees them without the lock.
+// most `keep` idle bytes remain; the caller frees them without the lock.  A block of more than
+// `keep` could not stay whatever else went, so it goes before any other.
 std::vector<void*> take_idle(int device, std::size_t keep)
 {
     std::size_t idle = 0;
@@ -34,13 +40,16 @@ std::vector<void*> take_idle(int device, std::size_t keep)
         idle += mine(b) ? b.bytes : 0;
     }
     std::vector<void*> out;
-    for (std::size_t k = 0; k < g_blocks.size() && idle > keep;) {
-        if (mine(g_blocks[k])) {
-            out.push_back(g_blocks[k].ptr);
-            idle -= g_blocks[k].bytes;
-            g_blocks.erase(g_blocks.begin() + static_cast<std::ptrdiff_t>(k));
-        } else {
-            ++k;
+    out.reserve(g_blocks.size());  // before any block leaves the list: nothing below throws
+    for (const bool large : {true, false}) {
+        for (std::size_t k = 0; k < g_blocks.size() && idle > keep;) {
+            if (mine(g_blocks[k]) && (!large || g_blocks[k].bytes > keep)) {
+                out.push_back(g_blocks[k].ptr);
+                idle -= g_blocks[k].bytes;
+                g_blocks.erase(g_blocks.begin() + static_cast<std::ptrdiff_t>(k));
+            } else {
+                ++k;
+            }
         }
     }
     return out;
@@ -65,6 +74,7 @@ void* scratch_take(std::size_t bytes)
             Block* best = nullptr;
             for (Block& b : g_blocks) {
                 if (b.device == device && !b.busy && b.bytes >= want &&
+                    b.bytes / kFitMost <= want &&
                     (best == nullptr || b.bytes < best->bytes)) {
                     best = &b;
                 }

@@ -87,3 +87,52 @@ def test_block_goes_back_only_after_a_wait(tmp_path, waited, waits):
         }}
         CHECK(fake.waits == {waits} + 1);
     """)
+
+
+def test_a_block_past_the_limit_leaves_the_others(tmp_path):
+    """A block larger than the pool keeps at all is freed by itself when it comes back; below the
+    limit the oldest idle blocks make room."""
+    run(tmp_path, """
+        void* small[3];
+        for (void*& p : small) { p = scratch_take(8 * MiB); }
+        void* large = scratch_take(kScratchKeep + MiB);
+        for (void* p : small) { scratch_give(p); }
+        CHECK(fake.frees == 0);
+        scratch_give(large);
+        CHECK(fake.frees == 1 && fake.held == 24 * MiB);
+        CHECK(scratch_take(8 * MiB) == small[0]);
+        CHECK(fake.mallocs == 4);
+        scratch_give(small[0]);
+        void* wide = scratch_take(kScratchKeep - 8 * MiB);
+        scratch_give(wide);  // small[0] came back last: it stays with this one
+        CHECK(fake.held == kScratchKeep);
+        CHECK(scratch_take(8 * MiB) == small[0]);
+        scratch_give(small[0]);
+        scratch_drop();  // the last holder
+        CHECK(fake.held == 0);
+    """)
+
+
+def test_a_small_request_leaves_a_large_block(tmp_path):
+    run(tmp_path, """
+        void* large = scratch_take(256 * MiB);
+        scratch_give(large);
+        void* tiny = scratch_take(1000);
+        CHECK(tiny != large && fake.mallocs == 2);
+        void* again = scratch_take(200 * MiB);  // at least half of it
+        CHECK(again == large && fake.mallocs == 2);
+        scratch_give(tiny);
+        scratch_give(again);
+        CHECK(scratch_take(2000) == tiny);
+    """)
+
+
+def test_idle_blocks_go_before_an_allocation_fails(tmp_path):
+    run(tmp_path, """
+        fake.limit = 100 * MiB;
+        void* a = scratch_take(60 * MiB);
+        CHECK(scratch_take(60 * MiB) == nullptr);  // a is in use
+        scratch_give(a);
+        void* b = scratch_take(90 * MiB);  // a is idle, too small, and freed for it
+        CHECK(b != nullptr && fake.frees == 1);
+    """)
