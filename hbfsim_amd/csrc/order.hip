@@ -517,10 +517,9 @@ hipError_t launch_buckets(const void* rec, std::size_t n, const Buckets& bk, ulo
     return err;
 }
 
-// The stable order by radix sort: pos receives the positions.  key_a: n words
-// of scratch.
-int radix_order(const void* rec, bool packed, std::size_t n, std::uint64_t* key_a,
-                std::uint32_t* pos, hipStream_t stream)
+// The stable order by radix sort: pos receives the positions.
+int radix_order(const void* rec, bool packed, std::size_t n, std::uint32_t* pos,
+                hipStream_t stream)
 {
     const unsigned end_bit = packed ? 56u : 64u;
     std::size_t temp_bytes = 0;
@@ -534,13 +533,15 @@ int radix_order(const void* rec, bool packed, std::size_t n, std::uint64_t* key_
         return HBFSIM_CUDA_ERROR;
     }
     ScratchPlan plan;
-    const std::size_t o_key = plan.add<std::uint64_t>(n);
+    const std::size_t o_key_a = plan.add<std::uint64_t>(n);
+    const std::size_t o_key_b = plan.add<std::uint64_t>(n);
     const std::size_t o_pos = plan.add<std::uint32_t>(n);
     const std::size_t o_temp = plan.add<unsigned char>(temp_bytes);
     ScratchLease lease(plan.bytes, stream);
     if (!lease.ok()) {
         return HBFSIM_CUDA_ERROR;
     }
+    auto* key_a = lease.at<std::uint64_t>(o_key_a);
     auto* pos_a = lease.at<std::uint32_t>(o_pos);
     if (packed) {
         hipLaunchKernelGGL(k_issue_keys<true>, dim3(blocks_for(n)), dim3(kThreads), 0, stream, rec,
@@ -552,10 +553,138 @@ int radix_order(const void* rec, bool packed, std::size_t n, std::uint64_t* key_
     err = hipGetLastError();
     if (err == hipSuccess) {
         err = rocprim::radix_sort_pairs(lease.at<unsigned char>(o_temp), temp_bytes, key_a,
-                                        lease.at<std::uint64_t>(o_key), pos_a, pos, n, 0, end_bit,
-                                        stream);
+                                        lease.at<std::uint64_t>(o_key_b), pos_a, pos, n, 0,
+                                        end_bit, stream);
     }
     // (the lease waits for the stream)
+    return err == hipSuccess ? HBFSIM_OK : HBFSIM_CUDA_ERROR;
+}
+
+// Results of the sorted copy back to the records' stream positions.
+hipError_t scatter_back(const std::uint32_t* pos, const std::uint32_t* place, std::size_t n,
+                        const std::uint64_t* scomp, const std::uint8_t* sstatus,
+                        std::uint64_t* comp, std::uint8_t* status, hipStream_t stream)
+{
+    const unsigned eighths = (std::min(blocks_for(n), 8192u) + 7) / 8;  // whole rounds of XCDs
+    hipLaunchKernelGGL(k_scatter, dim3(8 * eighths), dim3(kThreads), 0, stream, pos, place, n,
+                       scomp, sstatus, comp, status);
+    const hipError_t err = hipGetLastError();
+    return err == hipSuccess ? hipStreamSynchronize(stream) : err;
+}
+
+// The run by the bucket sort.  `done` stays false, and nothing has changed, where it does not
+// apply: no memory for all its arrays at once, a launch refused, or buckets that do not fit.
+int run_bucketed(const void* d_rec, bool packed, std::size_t n, std::uint64_t* d_comp,
+                 std::uint8_t* d_status, hipStream_t stream, const sorted_runner& run, bool& done)
+{
+    std::uint32_t log2 = 4;
+    while ((kBucketMean << log2) < n && (std::size_t{1} << log2) < kMaxBuckets) {
+        ++log2;
+    }
+    const std::size_t buckets = std::size_t{1} << log2;
+    const std::size_t rec_bytes = packed ? sizeof(hbf_record16) : sizeof(hbf_record32);
+    ScratchPlan plan;
+    const std::size_t o_words = plan.add<unsigned long long>(3);
+    const std::size_t o_count = plan.add<std::uint32_t>(buckets);
+    const std::size_t o_first = plan.add<std::uint32_t>(buckets + 1);
+    const std::size_t o_part = plan.add<ulonglong2>(kRangeParts);
+    const std::size_t o_pos = plan.add<std::uint32_t>(n);
+    const std::size_t o_place = plan.add<std::uint32_t>(n);
+    const std::size_t o_key = plan.add<std::uint64_t>(n);  // keys, then completions
+    const std::size_t o_rec = plan.add<unsigned char>(n * rec_bytes);
+    const std::size_t o_status = plan.add<std::uint8_t>(d_status != nullptr ? n : 0);
+    ScratchLease lease(plan.bytes, stream);
+    if (!lease.ok()) {
+        return HBFSIM_OK;
+    }
+    auto* words = lease.at<unsigned long long>(o_words);
+    auto* pos = lease.at<std::uint32_t>(o_pos);
+    auto* place = lease.at<std::uint32_t>(o_place);
+    auto* key = lease.at<std::uint64_t>(o_key);
+    void* sorted = lease.at<unsigned char>(o_rec);
+    auto* sstatus = d_status != nullptr ? lease.at<std::uint8_t>(o_status) : nullptr;
+    const Buckets bk{words, lease.at<std::uint32_t>(o_count), lease.at<std::uint32_t>(o_first),
+                     reinterpret_cast<std::uint32_t*>(words + 2), log2};
+    auto* part = lease.at<ulonglong2>(o_part);
+    hipError_t err = hipMemsetAsync(words, 0, o_first - o_words, stream);
+    if (err != hipSuccess) {
+        return HBFSIM_CUDA_ERROR;
+    }
+    err = packed ? launch_buckets<hbf_record16, true>(d_rec, n, bk, part, key, pos, place,
+                                                      static_cast<hbf_record16*>(sorted), stream)
+                 : launch_buckets<hbf_record32, false>(d_rec, n, bk, part, key, pos, place,
+                                                       static_cast<hbf_record32*>(sorted), stream);
+    if (err != hipSuccess) {
+        (void)hipGetLastError();
+        return HBFSIM_OK;
+    }
+    std::uint32_t overflow = 0;
+    err = hipMemcpyAsync(&overflow, bk.overflow, 4, hipMemcpyDeviceToHost, stream);
+    if (err == hipSuccess) err = hipStreamSynchronize(stream);
+    if (err != hipSuccess) {
+        return HBFSIM_CUDA_ERROR;
+    }
+    if (overflow != 0) {
+        lease.synced(err);
+        return HBFSIM_OK;
+    }
+    done = true;
+    const int st = run(sorted, key, sstatus);
+    if (st != HBFSIM_OK) {
+        return st;
+    }
+    err = scatter_back(pos, place, n, key, sstatus, d_comp, d_status, stream);
+    lease.synced(err);
+    return err == hipSuccess ? HBFSIM_OK : HBFSIM_CUDA_ERROR;
+}
+
+// The run by the radix sort.  Its keys (24 bytes a record, and the library's own scratch) are
+// given back before the sorted copy and its results are laid out, so that a run needs the larger
+// of the two and not their sum.
+int run_radix(const void* d_rec, bool packed, std::size_t n, std::uint64_t* d_comp,
+              std::uint8_t* d_status, hipStream_t stream, const sorted_runner& run)
+{
+    ScratchLease order(n * sizeof(std::uint32_t), stream);
+    if (!order.ok()) {
+        return HBFSIM_CUDA_ERROR;
+    }
+    auto* pos = order.at<std::uint32_t>(0);
+    int st = radix_order(d_rec, packed, n, pos, stream);
+    if (st != HBFSIM_OK) {
+        return st;
+    }
+    ScratchPlan plan;
+    const std::size_t rec_bytes = packed ? sizeof(hbf_record16) : sizeof(hbf_record32);
+    const std::size_t o_comp = plan.add<std::uint64_t>(n);
+    const std::size_t o_rec = plan.add<unsigned char>(n * rec_bytes);
+    const std::size_t o_status = plan.add<std::uint8_t>(d_status != nullptr ? n : 0);
+    ScratchLease lease(plan.bytes, stream);
+    if (!lease.ok()) {
+        return HBFSIM_CUDA_ERROR;
+    }
+    auto* scomp = lease.at<std::uint64_t>(o_comp);
+    void* sorted = lease.at<unsigned char>(o_rec);
+    auto* sstatus = d_status != nullptr ? lease.at<std::uint8_t>(o_status) : nullptr;
+    if (packed) {
+        hipLaunchKernelGGL(k_gather_records<hbf_record16>, dim3(blocks_for(n)), dim3(kThreads), 0,
+                           stream, static_cast<const hbf_record16*>(d_rec), pos, n,
+                           static_cast<hbf_record16*>(sorted));
+    } else {
+        hipLaunchKernelGGL(k_gather_records<hbf_record32>, dim3(blocks_for(n)), dim3(kThreads), 0,
+                           stream, static_cast<const hbf_record32*>(d_rec), pos, n,
+                           static_cast<hbf_record32*>(sorted));
+    }
+    if (hipGetLastError() != hipSuccess) {
+        return HBFSIM_CUDA_ERROR;
+    }
+    st = run(sorted, scomp, sstatus);
+    if (st != HBFSIM_OK) {
+        return st;
+    }
+    const hipError_t err =
+        scatter_back(pos, nullptr, n, scomp, sstatus, d_comp, d_status, stream);  // pos is sorted
+    lease.synced(err);
+    order.synced(err);
     return err == hipSuccess ? HBFSIM_OK : HBFSIM_CUDA_ERROR;
 }
 
@@ -585,97 +714,14 @@ int run_in_issue_order(const void* d_rec, bool packed, std::size_t n, std::uint6
         return HBFSIM_UNSUPPORTED;  // positions travel as 32-bit payload
     }
     hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
-    const std::size_t rec_bytes = packed ? sizeof(hbf_record16) : sizeof(hbf_record32);
-    std::uint32_t log2 = 4;
-    while ((kBucketMean << log2) < n && (std::size_t{1} << log2) < kMaxBuckets) {
-        ++log2;
-    }
-    const bool bucketed = n <= kMaxBucketed;
-    const std::size_t buckets = std::size_t{1} << log2;
-    ScratchPlan plan;
-    const std::size_t o_words = plan.add<unsigned long long>(3);
-    const std::size_t o_count = plan.add<std::uint32_t>(buckets);
-    const std::size_t o_first = plan.add<std::uint32_t>(buckets + 1);
-    const std::size_t o_part = plan.add<ulonglong2>(kRangeParts);
-    const std::size_t o_pos = plan.add<std::uint32_t>(n);
-    const std::size_t o_place = plan.add<std::uint32_t>(bucketed ? n : 0);
-    const std::size_t o_key = plan.add<std::uint64_t>(n);  // keys, then completions
-    const std::size_t o_rec = plan.add<unsigned char>(n * rec_bytes);
-    const std::size_t o_status = plan.add<std::uint8_t>(d_status != nullptr ? n : 0);
-    ScratchLease lease(plan.bytes, stream);
-    if (!lease.ok()) {
-        return HBFSIM_CUDA_ERROR;
-    }
-    auto* words = lease.at<unsigned long long>(o_words);
-    auto* pos = lease.at<std::uint32_t>(o_pos);
-    std::uint32_t* place = lease.at<std::uint32_t>(o_place);
-    auto* key = lease.at<std::uint64_t>(o_key);
-    void* sorted = lease.at<unsigned char>(o_rec);
-    auto* sstatus = d_status != nullptr ? lease.at<std::uint8_t>(o_status) : nullptr;
-    hipError_t err = hipSuccess;
-    std::uint32_t overflow = bucketed ? 0u : 1u;
-    if (bucketed) {
-        const Buckets bk{words, lease.at<std::uint32_t>(o_count), lease.at<std::uint32_t>(o_first),
-                         reinterpret_cast<std::uint32_t*>(words + 2), log2};
-        auto* part = lease.at<ulonglong2>(o_part);
-        err = hipMemsetAsync(words, 0, o_first - o_words, stream);
-        if (err != hipSuccess) {
-            return HBFSIM_CUDA_ERROR;
-        }
-        err = packed ? launch_buckets<hbf_record16, true>(d_rec, n, bk, part, key, pos, place,
-                                                          static_cast<hbf_record16*>(sorted),
-                                                          stream)
-                     : launch_buckets<hbf_record32, false>(d_rec, n, bk, part, key, pos, place,
-                                                           static_cast<hbf_record32*>(sorted),
-                                                           stream);
-        if (err != hipSuccess) {
-            (void)hipGetLastError();
-            overflow = 1;  // a launch was refused: the radix sort takes the stream
-            err = hipSuccess;
-        } else {
-            err = hipMemcpyAsync(&overflow, bk.overflow, 4, hipMemcpyDeviceToHost, stream);
-        }
-        if (err == hipSuccess) err = hipStreamSynchronize(stream);
-        if (err != hipSuccess) {
-            return HBFSIM_CUDA_ERROR;
-        }
-    }
-    if (overflow != 0) {
-        place = nullptr;  // pos comes in sorted order
-        const int st = radix_order(d_rec, packed, n, key, pos, stream);
-        if (st != HBFSIM_OK) {
+    if (n <= kMaxBucketed) {
+        bool done = false;
+        const int st = run_bucketed(d_rec, packed, n, d_comp, d_status, stream, run, done);
+        if (done || st != HBFSIM_OK) {
             return st;
         }
-        if (packed) {
-            hipLaunchKernelGGL(k_gather_records<hbf_record16>, dim3(blocks_for(n)), dim3(kThreads),
-                               0, stream, static_cast<const hbf_record16*>(d_rec), pos, n,
-                               static_cast<hbf_record16*>(sorted));
-        } else {
-            hipLaunchKernelGGL(k_gather_records<hbf_record32>, dim3(blocks_for(n)), dim3(kThreads),
-                               0, stream, static_cast<const hbf_record32*>(d_rec), pos, n,
-                               static_cast<hbf_record32*>(sorted));
-        }
-        if (hipGetLastError() != hipSuccess) {
-            return HBFSIM_CUDA_ERROR;
-        }
     }
-    const int st = run(sorted, key, sstatus);
-    if (st != HBFSIM_OK) {
-        return st;
-    }
-    const unsigned eighths = (std::min(blocks_for(n), 8192u) + 7) / 8;  // whole rounds of XCDs
-    hipLaunchKernelGGL(k_scatter, dim3(8 * eighths), dim3(kThreads), 0, stream,
-                       static_cast<const std::uint32_t*>(pos),
-                       static_cast<const std::uint32_t*>(place), n,
-                       static_cast<const std::uint64_t*>(key),
-                       static_cast<const std::uint8_t*>(sstatus), d_comp, d_status);
-    err = hipGetLastError();
-    if (err == hipSuccess) err = hipStreamSynchronize(stream);
-    if (err != hipSuccess) {
-        return HBFSIM_CUDA_ERROR;
-    }
-    lease.synced(err);
-    return HBFSIM_OK;
+    return run_radix(d_rec, packed, n, d_comp, d_status, stream, run);
 }
 
 }  // namespace hbfamd

@@ -56,3 +56,39 @@ def test_large_streams_out_of_order(n, packed):
     assert torch.equal(status[order], sstatus)
     assert report == sreport
     assert all((a == b).all() for a, b in zip(busy, sbusy))
+
+
+@pytest.mark.parametrize("n,skewed", [((1 << 25) + 17, False), ((1 << 25) - 1, True)])
+def test_radix_sort_within_its_memory(n, skewed):
+    """The radix sort of 32-byte records needs 45 bytes of scratch a record, its keys given back
+    before the sorted copy is laid out (69 side by side), whether it takes the stream by its size
+    or after the bucket sort could not (half the records in a thousandth of the span)."""
+    import torch
+    from hbfsim_amd import engine as eng
+    rec = stream(n, n)
+    if skewed:
+        rec[::2, 2] //= 1000
+    rec = rec.contiguous()
+    comp = torch.empty(n, dtype=torch.int64, device="cuda")
+    status = torch.empty(n, dtype=torch.uint8, device="cuda")
+    e = eng.Engine(str(C0))
+    try:
+        e.register(w.RANGE_BASE, LENGTH, 3)
+        order = torch.sort(rec[:, 2], stable=True).indices
+        in_order = rec[order]
+        want = e.run(in_order, comp, status)  # also lays out the engine's own arrays
+        wcomp = torch.empty_like(comp)
+        wcomp[order] = comp
+        del in_order, order
+        e.reset()
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        room = 45 * n + (256 << 20)
+        filler = torch.empty(torch.cuda.mem_get_info()[0] - room, dtype=torch.uint8, device="cuda")
+        got = e.run(rec, comp, status)
+        del filler
+        assert torch.equal(comp, wcomp)
+        assert got == want
+    finally:
+        e.close()
+        torch.cuda.empty_cache()
