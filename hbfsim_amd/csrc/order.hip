@@ -155,6 +155,7 @@ constexpr std::size_t kMaxBucketed = kMaxBuckets * 2048;
 constexpr std::uint32_t kBucketCap = 4096;   // records of a bucket in LDS (32 KiB)
 constexpr int kCapPer = kBucketCap / kThreads;
 constexpr std::uint32_t kSubs = 1024;        // sub-buckets within a bucket
+constexpr std::uint32_t kCrowd = 96;         // records of a sub-bucket told apart by comparing
 constexpr std::size_t kChunk = 8192;         // records per workgroup of the partition
 constexpr unsigned kRangeParts = 2048;       // workgroups of k_issue_range
 
@@ -348,10 +349,36 @@ __global__ __launch_bounds__(kThreads) void k_bucket_scatter(const void* rec, st
     }
 }
 
+// Orders keys[0, 2^m), m >= 6, ascending: a bitonic network over the workgroup.
+__device__ __forceinline__ void sort_keys(std::uint64_t* keys, std::uint32_t size)
+{
+    for (std::uint32_t run = 2; run <= size; run *= 2) {
+        for (std::uint32_t gap = run / 2; gap != 0; gap /= 2) {
+            for (std::uint32_t p = threadIdx.x; p < size / 2; p += kThreads) {
+                const std::uint32_t i = 2 * p - (p & (gap - 1));
+                const std::uint64_t a = keys[i], b = keys[i + gap];
+                if ((a > b) == ((i & run) == 0)) {
+                    keys[i] = b;
+                    keys[i + gap] = a;
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+
 // One workgroup per bucket.  Keys are unique, so a record's place is the
 // number of smaller keys: all of the sub-buckets below its own, and those it
 // finds by comparing within its own (one or two records unless many share an
-// issue time).  pos and place (stream position, sorted position) are written in
+// issue time).  A bucket with more than kCrowd records in one sub-bucket is
+// sorted whole by a network instead, and a place found by bisection: comparing
+// is quadratic in the records that share a time (4M packed records, whole run:
+// 512 at a time 1,393 -> 838 us, 2,000 3,182 -> 878, about 4,000 7,231 ->
+// 1,337; the radix sort alone 3,480, whatever the times).  The line lies
+// above steps of one issue time: 4M lines in steps of 64 take 450 us by
+// comparing and 523 by the network, records at random times of 64 each 781 and
+// 842; at 128 each 909 and 792.
+// pos and place (stream position, sorted position) are written in
 // the order the records came into the bucket, for k_scatter.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void k_bucket_sort(Buckets bk, const std::uint64_t* key,
@@ -391,10 +418,12 @@ __global__ __launch_bounds__(kThreads) void k_bucket_sort(Buckets bk, const std:
     __syncthreads();
     // exclusive scan of the sub-bucket counts, four per thread
     std::uint32_t c[4], own = 0;
+    bool crowd = false;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         c[k] = sub[threadIdx.x * 4 + k];
         own += c[k];
+        crowd = crowd || c[k] > kCrowd;
     }
     std::uint32_t incl = own;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -425,16 +454,36 @@ __global__ __launch_bounds__(kThreads) void k_bucket_sort(Buckets bk, const std:
             keys[sub[mine[k] >> down] + rank[k]] = mine[k];
         }
     }
-    __syncthreads();
+    const bool crowded = __syncthreads_or(crowd ? 1 : 0) != 0;
+    if (crowded) {
+        std::uint32_t size = 64;
+        while (size < count) {
+            size *= 2;
+        }
+        for (std::uint32_t j = count + threadIdx.x; j < size; j += kThreads) {
+            keys[j] = ~0ull;
+        }
+        __syncthreads();
+        sort_keys(keys, size);
+    }
     std::uint32_t to[kCapPer];  // sorted place within the bucket
 #pragma unroll
     for (int k = 0; k < kCapPer; ++k) {
         const std::uint32_t j = k * kThreads + threadIdx.x;
         if (j < count) {
-            const std::uint32_t lo = sub[mine[k] >> down], hi = sub[(mine[k] >> down) + 1];
+            std::uint32_t lo = sub[mine[k] >> down], hi = sub[(mine[k] >> down) + 1];
             to[k] = lo;
-            for (std::uint32_t m = lo; m < hi; ++m) {
-                to[k] += keys[m] < mine[k] ? 1u : 0u;
+            if (crowded) {
+                while (lo < hi) {  // the key's place among the sorted ones
+                    const std::uint32_t m = (lo + hi) / 2;
+                    lo = keys[m] < mine[k] ? m + 1 : lo;
+                    hi = keys[m] < mine[k] ? hi : m;
+                }
+                to[k] = lo;
+            } else {
+                for (std::uint32_t m = lo; m < hi; ++m) {
+                    to[k] += keys[m] < mine[k] ? 1u : 0u;
+                }
             }
             pos[s + j] = static_cast<std::uint32_t>(mine[k]);
             place[s + j] = s + to[k];

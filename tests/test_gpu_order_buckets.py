@@ -52,3 +52,25 @@ def test_bucketed_order(n, shape, packed):
     finally:
         p.close()
         q.close()
+
+
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("per", [12, 48, 64, 95, 96, 97, 98, 120, 1000, 2049, 4095, 4096, 4097])
+def test_many_records_of_one_time(per, packed):
+    """`per` records share each issue time: told apart by comparing up to 96 in a sub-bucket, by
+    the sorting network up to the 4,096 that a bucket holds, by the radix sort beyond."""
+    n = 63 * 4096 + 11
+    rec = stream(n, "spread", per)
+    rec[:, 2] = np.random.default_rng(per).permutation(np.arange(n) // per).astype(np.uint64)
+    rec[:, 2] *= np.uint64(2000 * per)
+    p, q = parity.Pair(C0, RANGES), parity.Pair(C0, RANGES)
+    try:
+        g, c = p.run_packed(rec) if packed else p.run(rec)
+        parity.assert_same(g, c, f"{per} records a time")
+        comp, st, rep = sorted_pair_run(q, rec, packed)
+        np.testing.assert_array_equal(g[0], comp)
+        np.testing.assert_array_equal(g[1], st)
+        assert g[2] == rep
+    finally:
+        p.close()
+        q.close()
