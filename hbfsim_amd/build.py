@@ -21,6 +21,7 @@ SOURCES = [CSRC / "engine.hip", CSRC / "gen.hip", CSRC / "thermal.hip", CSRC / "
            CSRC / "probe.hip", CSRC / "scratch.cpp", CSRC / "api.cpp",
            CSRC / "profile.cpp"]
 HEADERS = [CSRC / "engine.hpp", CSRC / "thermal.hpp", CSRC / "link.hpp", CSRC / "scratch.hpp",
+           CSRC / "class_table.hpp",
            CSRC / "profile.hpp",
            CSRC / "json_min.hpp", ROOT / "include" / "hbfsim_amd.h"]
 

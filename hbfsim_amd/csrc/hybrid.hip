@@ -25,6 +25,7 @@
 #include <cstring>  // rocPRIM's host code uses memset
 #include <rocprim/device/device_radix_sort.hpp>
 
+#include "class_table.hpp"
 #include "engine.hpp"
 #include "scratch.hpp"
 
@@ -112,7 +113,7 @@ struct ClassTable {
     unsigned long long* slot;            // [mask + 1]
     std::uint32_t* first;                // [mask + 1], the caller's use
     std::uint64_t mask;
-    std::uint32_t probes;                // probe limit; 0: none (the largest table)
+    std::uint32_t probes;                // probe limit; 0: none (the largest table, class_table.hpp)
     const hbfsim_amd_access_class* access;
     const hbfsim_amd_access_class* seen;
     std::uint32_t* overflow;             // set when a probe limit was reached
@@ -214,13 +215,14 @@ __global__ __launch_bounds__(kThreads) void k_class_sample(ClassTable t, std::si
 // The classes earlier batches saw (all different) take their slots first.
 __global__ __launch_bounds__(kThreads) void k_seen_insert(ClassTable t, std::size_t seen)
 {
-    const std::size_t k = static_cast<std::size_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (k >= seen) {
-        return;
-    }
-    std::uint64_t found;
-    if (class_slot(t, load_class(t.seen, k, true), kSeen | k, found) == kEmpty) {
-        *t.overflow = 1;
+    const std::size_t stride = static_cast<std::size_t>(gridDim.x) * kThreads;
+    for (std::size_t k = static_cast<std::size_t>(blockIdx.x) * kThreads + threadIdx.x; k < seen;
+         k += stride) {
+        std::uint64_t found;
+        if (class_slot(t, load_class(t.seen, k, true), kSeen | k, found) == kEmpty) {
+            *t.overflow = 1;
+            return;
+        }
     }
 }
 
@@ -230,6 +232,81 @@ __device__ __forceinline__ std::uint64_t wave_sum(std::uint64_t v)
         v += __shfl_down(v, off);
     }
     return v;
+}
+
+// Sum of v over the workgroup, in thread 0.
+__device__ __forceinline__ std::uint64_t block_sum(std::uint64_t v)
+{
+    __shared__ std::uint64_t part[kThreads / 64];
+    v = wave_sum(v);
+    __syncthreads();  // (a sum before this one has been read)
+    if ((threadIdx.x & 63) == 0) {
+        part[threadIdx.x / 64] = v;
+    }
+    __syncthreads();
+    v = 0;
+    for (int w = 0; w < kThreads / 64; ++w) {
+        v += part[w];
+    }
+    return v;
+}
+
+// This workgroup's run of `slots` table slots.
+struct SlotRun {
+    std::uint64_t begin, end;
+};
+
+__device__ __forceinline__ SlotRun slot_run(std::uint64_t slots)
+{
+    const std::uint64_t per =
+        (slots + static_cast<std::uint64_t>(gridDim.x) * kThreads - 1) /
+        (static_cast<std::uint64_t>(gridDim.x) * kThreads) * kThreads;
+    const std::uint64_t b = blockIdx.x * per;
+    return SlotRun{b < slots ? b : slots, b + per < slots ? b + per : slots};
+}
+
+// Numbers the slots that `take` accepts, from *count on, and hands each to
+// `emit`: counted first, so that a workgroup asks for its numbers with one
+// atomic (one per wave took 0.6 ms over 2^23 slots, one per slot 1.6).
+template <typename Take, typename Emit>
+__device__ __forceinline__ void compact_slots(std::uint64_t slots, unsigned long long* count,
+                                              Take take, Emit emit)
+{
+    __shared__ unsigned long long start;
+    __shared__ std::uint32_t w_count[kThreads / 64];
+    const SlotRun run = slot_run(slots);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    std::uint64_t own = 0;
+    for (std::uint64_t s = run.begin + threadIdx.x; s < run.end; s += kThreads) {
+        own += take(s) ? 1u : 0u;
+    }
+    const std::uint64_t total = block_sum(own);
+    if (total == 0) {
+        return;  // (the same in every thread)
+    }
+    if (threadIdx.x == 0) {
+        start = atomicAdd(count, static_cast<unsigned long long>(total));
+    }
+    __syncthreads();
+    std::uint64_t at = start;
+    for (std::uint64_t b = run.begin; b < run.end; b += kThreads) {
+        const std::uint64_t s = b + threadIdx.x;
+        const bool taken = s < run.end && take(s);
+        const std::uint64_t m = __ballot(taken);
+        if (lane == 0) {
+            w_count[wave] = static_cast<std::uint32_t>(__popcll(m));
+        }
+        __syncthreads();
+        std::uint64_t mine = at + __popcll(m & ((1ull << lane) - 1));
+        for (int w = 0; w < kThreads / 64; ++w) {
+            mine += w < wave ? w_count[w] : 0u;
+            at += w_count[w];
+        }
+        if (taken) {
+            emit(s, mine);
+        }
+        __syncthreads();
+    }
 }
 
 // flags[i] = warm-up or hash decision (calibrator.cpp:86-95), counted in
@@ -295,22 +372,28 @@ __global__ __launch_bounds__(kThreads) void k_sampler_pass(
 __global__ __launch_bounds__(kThreads) void k_sampler_first(ClassTable t, std::uint8_t* flags,
                                                             unsigned long long* totals)
 {
-    const std::uint64_t s = static_cast<std::uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    const std::uint32_t i = s <= t.mask ? t.first[s] : kNone;
-    const bool fresh = i != kNone;
-    bool raised = false;
-    if (fresh && flags[i] == 0) {
-        flags[i] = 1;
-        raised = true;
+    const SlotRun run = slot_run(t.mask + 1);
+    std::uint64_t fresh = 0, raised = 0;
+    for (std::uint64_t s = run.begin + threadIdx.x; s < run.end; s += kThreads) {
+        const std::uint32_t i = t.first[s];
+        if (i != kNone) {
+            ++fresh;
+            if (flags[i] == 0) {
+                flags[i] = 1;
+                ++raised;
+            }
+        }
     }
-    const std::uint64_t f = __ballot(fresh), r = __ballot(raised);
-    if ((threadIdx.x & 63) == 0) {
-        if (r != 0) {
-            atomicAdd(&totals[0], static_cast<unsigned long long>(__popcll(r)));
+    fresh = block_sum(fresh);
+    if (fresh == 0) {
+        return;  // (the same in every thread)
+    }
+    raised = block_sum(raised);
+    if (threadIdx.x == 0) {
+        if (raised != 0) {
+            atomicAdd(&totals[0], static_cast<unsigned long long>(raised));
         }
-        if (f != 0) {
-            atomicAdd(&totals[1], static_cast<unsigned long long>(__popcll(f)));
-        }
+        atomicAdd(&totals[1], static_cast<unsigned long long>(fresh));
     }
 }
 
@@ -319,11 +402,11 @@ __global__ __launch_bounds__(kThreads) void k_sampler_grow(ClassTable t,
                                                            hbfsim_amd_access_class* out,
                                                            unsigned long long* at)
 {
-    const std::uint64_t s = static_cast<std::uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    const std::uint32_t i = s <= t.mask ? t.first[s] : kNone;
-    if (i != kNone) {
-        out[atomicAdd(at, 1ull)] = load_class(t.access, i, t.aligned);
-    }
+    compact_slots(
+        t.mask + 1, at, [&](std::uint64_t s) { return t.first[s] != kNone; },
+        [&](std::uint64_t s, std::uint64_t k) {
+            out[k] = load_class(t.access, t.first[s], t.aligned);
+        });
 }
 
 // Calibrator: slot_of[i] = the slot of request i's class; the latencies'
@@ -384,25 +467,13 @@ __global__ __launch_bounds__(kThreads) void k_calib_list(ClassTable t, std::uint
                                                          ulonglong2* keys,
                                                          unsigned long long* count)
 {
-    const std::uint64_t s = static_cast<std::uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    const bool used = s <= t.mask && t.slot[s] != kEmpty;
-    const std::uint64_t m = __ballot(used);
-    if (m == 0) {
-        return;
-    }
-    unsigned long long at = 0;
-    const int lane = threadIdx.x & 63;
-    const int lead = __ffsll(static_cast<unsigned long long>(m)) - 1;
-    if (lane == lead) {
-        at = atomicAdd(count, static_cast<unsigned long long>(__popcll(m)));
-    }
-    at = __shfl(at, lead);
-    if (used) {
-        at += __popcll(m & ((1ull << lane) - 1));
-        list[at] = static_cast<std::uint32_t>(s);
-        const hbfsim_amd_access_class c = load_class(t.access, t.slot[s], t.aligned);
-        keys[at] = make_ulonglong2(class_hi(c), class_lo(c));
-    }
+    compact_slots(
+        t.mask + 1, count, [&](std::uint64_t s) { return t.slot[s] != kEmpty; },
+        [&](std::uint64_t s, std::uint64_t k) {
+            list[k] = static_cast<std::uint32_t>(s);
+            const hbfsim_amd_access_class c = load_class(t.access, t.slot[s], t.aligned);
+            keys[k] = make_ulonglong2(class_hi(c), class_lo(c));
+        });
 }
 
 // Up to this many classes are numbered by counting, for each, the classes
@@ -757,27 +828,6 @@ __global__ __launch_bounds__(kThreads) void k_calib_rows(
     }
 }
 
-// The first table holds 2^16 slots (or four per seen class); one that proves
-// too small is made 16 times larger, up to two slots per class the batch could
-// hold (at most 2^32 slots), where probing has no limit: a free slot remains.
-std::uint64_t first_slots(std::size_t seen)
-{
-    std::uint64_t cap = 1ull << 16;
-    while (cap < 4 * static_cast<std::uint64_t>(seen)) {
-        cap <<= 1;
-    }
-    return std::min<std::uint64_t>(cap, 1ull << 32);
-}
-
-std::uint64_t most_slots(std::size_t n, std::size_t seen)
-{
-    std::uint64_t cap = 1ull << 10;
-    while (cap < 2 * (static_cast<std::uint64_t>(n) + seen)) {
-        cap <<= 1;
-    }
-    return std::min<std::uint64_t>(cap, 1ull << 32);
-}
-
 // The buffers of the table and whatever else the call adds to `plan`.
 struct TablePlan {
     ScratchPlan plan;
@@ -857,9 +907,9 @@ int sampler_reference(sampler_state* s, const hbfsim_amd_access_class* d_access,
     }
     hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
     const std::uint64_t most = most_slots(n, s->seen);
-    std::uint64_t cap = std::min(first_slots(s->seen), most);
+    std::uint64_t cap = first_slots(s->seen, most);
     unsigned long long host[4] = {0, 0, 0, 0};  // references, new classes, overflow, -
-    for (;; cap = std::min(cap * 16, most)) {
+    for (;; cap = next_slots(cap, most)) {
         TablePlan p(cap);
         ScratchLease lease(p.plan.bytes, stream);
         if (!lease.ok()) {
@@ -875,7 +925,7 @@ int sampler_reference(sampler_state* s, const hbfsim_amd_access_class* d_access,
             return HBFSIM_CUDA_ERROR;
         }
         if (s->seen != 0) {
-            hipLaunchKernelGGL(k_seen_insert, dim3(blocks_for(s->seen)), dim3(kThreads), 0, stream,
+            hipLaunchKernelGGL(k_seen_insert, dim3(stride_blocks(s->seen)), dim3(kThreads), 0, stream,
                                t, s->seen);
         }
         if (s->seen == 0 && n >= 4 * kSample) {
@@ -885,7 +935,7 @@ int sampler_reference(sampler_state* s, const hbfsim_amd_access_class* d_access,
         hipLaunchKernelGGL(k_sampler_pass, dim3(stride_blocks(n)), dim3(kThreads), 0, stream, t,
                            d_sequence, first_sequence, n, s->warmup, s->threshold, s->seed,
                            d_flags, words);
-        hipLaunchKernelGGL(k_sampler_first, dim3(blocks_for(cap)), dim3(kThreads), 0, stream, t,
+        hipLaunchKernelGGL(k_sampler_first, dim3(walk_blocks(cap)), dim3(kThreads), 0, stream, t,
                            d_flags, words);
         err = hipGetLastError();
         if (err == hipSuccess) err = hipMemcpyAsync(host, words, sizeof(host),
@@ -922,7 +972,7 @@ int sampler_reference(sampler_state* s, const hbfsim_amd_access_class* d_access,
                 s->seen_cap = room;
             }
             // words[3] counts the classes written from here on
-            hipLaunchKernelGGL(k_sampler_grow, dim3(blocks_for(cap)), dim3(kThreads), 0, stream, t,
+            hipLaunchKernelGGL(k_sampler_grow, dim3(walk_blocks(cap)), dim3(kThreads), 0, stream, t,
                                s->seen_class + s->seen, words + 3);
             err = hipGetLastError();
             if (err == hipSuccess) err = hipStreamSynchronize(stream);
@@ -1099,9 +1149,9 @@ int calibrate(const hbfsim_amd_access_class* d_access, const std::uint64_t* d_la
     }
     const ScratchHold hold;  // outlives every lease of the call
     hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
-    const std::uint64_t most = most_slots(n, 0);
-    std::uint64_t cap = std::min(first_slots(0), most);
-    for (;; cap = std::min(cap * 16, most)) {
+    const std::uint64_t most = most_slots(n, 0, std::uint64_t{1} << 32);
+    std::uint64_t cap = first_slots(0, most);
+    for (;; cap = next_slots(cap, most)) {
         TablePlan p(cap);
         const std::size_t o_slot_of = p.plan.add<std::uint32_t>(n);
         const std::size_t o_list = p.plan.add<std::uint32_t>(std::min<std::uint64_t>(cap, n));
@@ -1131,7 +1181,7 @@ int calibrate(const hbfsim_amd_access_class* d_access, const std::uint64_t* d_la
         hipLaunchKernelGGL(k_calib_classes, dim3(stride_blocks(n)), dim3(kThreads), 0, stream, t,
                            d_latency, n, slot_of, words + 1,
                            reinterpret_cast<std::uint32_t*>(words + 3));
-        hipLaunchKernelGGL(k_calib_list, dim3(blocks_for(cap)), dim3(kThreads), 0, stream, t, list,
+        hipLaunchKernelGGL(k_calib_list, dim3(walk_blocks(cap)), dim3(kThreads), 0, stream, t, list,
                            keys, words);
         err = hipGetLastError();
         if (err == hipSuccess) err = hipMemcpyAsync(host, words, sizeof(host),
