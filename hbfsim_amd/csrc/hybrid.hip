@@ -108,6 +108,7 @@ constexpr std::uint64_t kEmpty = ~0ull;
 constexpr std::uint64_t kSeen = 1ull << 63;
 constexpr std::uint32_t kNone = 0xffffffffu;
 constexpr std::uint32_t kProbes = 64;  // then the table counts as too small
+constexpr std::uint32_t kProbesFree = 16;  // from here on also where another lookup said so
 
 struct ClassTable {
     unsigned long long* slot;            // [mask + 1]
@@ -116,7 +117,8 @@ struct ClassTable {
     std::uint32_t probes;                // probe limit; 0: none (the largest table, class_table.hpp)
     const hbfsim_amd_access_class* access;
     const hbfsim_amd_access_class* seen;
-    std::uint32_t* overflow;             // set when a probe limit was reached
+    std::uint32_t* overflow;             // set when the table is too small; then the classes sampled
+    std::uint32_t sample_limit;          // the most of those (class_table.hpp)
     bool aligned;                        // access lies on 16 bytes (seen always does)
 };
 
@@ -152,8 +154,13 @@ __device__ __forceinline__ std::uint64_t class_slot(const ClassTable& t,
             found = v;
             return s;
         }
-        if (t.probes != 0 && k >= t.probes) {
-            return kEmpty;
+        if (t.probes != 0 && k >= kProbesFree) {
+            // (asked for only here: the one word is slow to read from everywhere,
+            // 170 us for a pass over 4M requests)
+            if (k >= t.probes || __hip_atomic_load(t.overflow, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT) != 0) {
+                return kEmpty;
+            }
         }
         s = (s + 1) & t.mask;
     }
@@ -198,18 +205,32 @@ __device__ __forceinline__ void class_slots(const ClassTable& t, std::size_t i, 
 
 // An empty table would meet every thread of a full launch with a
 // compare-and-swap at once (203 us instead of 61 at 4M requests): a sample of
-// the batch, spread evenly over it, takes its classes' slots first.
-constexpr std::size_t kSample = 16384;
-
+// the batch, spread evenly over it, takes its classes' slots first.  The
+// classes among it say whether the table is worth trying.
 __global__ __launch_bounds__(kThreads) void k_class_sample(ClassTable t, std::size_t n)
 {
     const std::size_t k = static_cast<std::size_t>(blockIdx.x) * kThreads + threadIdx.x;
     const std::size_t i = k * (n / kSample);
+    bool fresh = false;
     if (k < kSample && i < n) {
-        std::uint64_t found;
+        std::uint64_t found = kEmpty;
         // (a probe limit reached here is reached again by the full pass)
-        (void)class_slot(t, load_class(t.access, i, t.aligned), i, found);
+        const std::uint64_t at =
+            class_slot(t, load_class(t.access, i, t.aligned), i, found);
+        fresh = at == kEmpty || found == i;
     }
+    const std::uint64_t m = __ballot(fresh);
+    if ((threadIdx.x & 63) == 0 && m != 0) {
+        atomicAdd(&t.overflow[1], static_cast<std::uint32_t>(__popcll(m)));
+    }
+}
+
+// Whether the sample says that the table is too small: a full pass over it
+// would be thrown away (1M classes in 2^16 slots: 64 probes for each of 4M
+// requests).
+__device__ __forceinline__ bool too_small(const ClassTable& t)
+{
+    return t.overflow[1] > t.sample_limit;
 }
 
 // The classes earlier batches saw (all different) take their slots first.
@@ -321,7 +342,10 @@ __global__ __launch_bounds__(kThreads) void k_sampler_pass(
     __shared__ unsigned long long part[kThreads / 64];
     const std::size_t stride = static_cast<std::size_t>(gridDim.x) * kThreads;
     std::uint64_t count = 0;
-    bool full = false;
+    bool full = too_small(t);  // then the host tries again with a larger table
+    if (full) {
+        *t.overflow = 1;
+    }
     for (std::size_t b = static_cast<std::size_t>(blockIdx.x) * kThreads + threadIdx.x;
          b < n && !full; b += stride * kAtOnce) {
         hbfsim_amd_access_class cs[kAtOnce];
@@ -345,7 +369,7 @@ __global__ __launch_bounds__(kThreads) void k_sampler_pass(
             count += hit ? 1u : 0u;
             if (at[k] == kEmpty) {
                 *t.overflow = 1;
-                full = true;  // the host tries again with a larger table
+                full = true;
             } else if ((found[k] & kSeen) == 0 && i < t.first[at[k]]) {
                 atomicMin(&t.first[at[k]], static_cast<std::uint32_t>(i));
             }
@@ -372,6 +396,9 @@ __global__ __launch_bounds__(kThreads) void k_sampler_pass(
 __global__ __launch_bounds__(kThreads) void k_sampler_first(ClassTable t, std::uint8_t* flags,
                                                             unsigned long long* totals)
 {
+    if (*t.overflow != 0) {
+        return;
+    }
     const SlotRun run = slot_run(t.mask + 1);
     std::uint64_t fresh = 0, raised = 0;
     for (std::uint64_t s = run.begin + threadIdx.x; s < run.end; s += kThreads) {
@@ -420,8 +447,12 @@ __global__ __launch_bounds__(kThreads) void k_calib_classes(ClassTable t,
     __shared__ unsigned long long part[kThreads / 64];
     const std::size_t stride = static_cast<std::size_t>(gridDim.x) * kThreads;
     unsigned long long most = 0;
-    for (std::size_t b = static_cast<std::size_t>(blockIdx.x) * kThreads + threadIdx.x; b < n;
-         b += stride * kAtOnce) {
+    bool full = too_small(t);  // (the next table's pass then checks every latency)
+    if (full) {
+        *t.overflow = 1;
+    }
+    for (std::size_t b = static_cast<std::size_t>(blockIdx.x) * kThreads + threadIdx.x;
+         b < n && !full; b += stride * kAtOnce) {
         hbfsim_amd_access_class cs[kAtOnce];
         std::uint64_t at[kAtOnce], found[kAtOnce], v[kAtOnce];
 #pragma unroll
@@ -439,7 +470,8 @@ __global__ __launch_bounds__(kThreads) void k_calib_classes(ClassTable t,
             }
             most = v[k] > most ? v[k] : most;
             if (at[k] == kEmpty) {
-                *t.overflow = 1;  // (the latencies are checked all the same)
+                *t.overflow = 1;
+                full = true;
             } else {
                 slot_of[b + k * stride] = static_cast<std::uint32_t>(at[k]);
             }
@@ -467,6 +499,9 @@ __global__ __launch_bounds__(kThreads) void k_calib_list(ClassTable t, std::uint
                                                          ulonglong2* keys,
                                                          unsigned long long* count)
 {
+    if (*t.overflow != 0) {
+        return;
+    }
     compact_slots(
         t.mask + 1, count, [&](std::uint64_t s) { return t.slot[s] != kEmpty; },
         [&](std::uint64_t s, std::uint64_t k) {
@@ -638,193 +673,164 @@ __device__ __forceinline__ Pair pair_join(Pair a, Pair b)
     return r;
 }
 
-__device__ __forceinline__ Pair wave_pair(Pair v)
+// Sums over samples of one class: the latencies in 128 bits, and the first two
+// moments of their logarithms about the logarithm of the class's median.  The
+// median lies within one deviation of the mean, so that taking the mean's
+// square off the second moment costs at most one bit, and one pass over the
+// samples gives both statistics.
+struct ClassSum {
+    std::uint64_t lo, hi;
+    Pair m1, m2;
+};
+
+__device__ __forceinline__ ClassSum sum_join(const ClassSum& a, const ClassSum& b)
 {
-    for (int off = 32; off > 0; off >>= 1) {
-        v = pair_join(v, Pair{__shfl_down(v.hi, off), __shfl_down(v.lo, off)});
-    }
-    return Pair{__shfl(v.hi, 0), __shfl(v.lo, 0)};
+    const U128 s = add128(U128{a.lo, a.hi}, U128{b.lo, b.hi});
+    return ClassSum{s.lo, s.hi, pair_join(a.m1, b.m1), pair_join(a.m2, b.m2)};
 }
 
-__device__ __forceinline__ U128 wave_sum128(U128 v)
+// The sum over kLanes neighbouring lanes, in the first of them.
+template <int kLanes>
+__device__ __forceinline__ ClassSum lanes_sum(ClassSum v)
 {
-    for (int off = 32; off > 0; off >>= 1) {
-        v = add128(v, U128{static_cast<std::uint64_t>(__shfl_down(
-                               static_cast<unsigned long long>(v.lo), off)),
-                           static_cast<std::uint64_t>(__shfl_down(
-                               static_cast<unsigned long long>(v.hi), off))});
+    for (int off = kLanes / 2; off > 0; off >>= 1) {
+        ClassSum o;
+        o.lo = __shfl_down(static_cast<unsigned long long>(v.lo), off);
+        o.hi = __shfl_down(static_cast<unsigned long long>(v.hi), off);
+        o.m1 = Pair{__shfl_down(v.m1.hi, off), __shfl_down(v.m1.lo, off)};
+        o.m2 = Pair{__shfl_down(v.m2.hi, off), __shfl_down(v.m2.lo, off)};
+        v = sum_join(v, o);
     }
     return v;
 }
 
-// A class's samples are taken in parts of kPart, one wave each, so that one
-// large class does not hold up the rest (one 256-thread block per class took
-// 248 us at 4M samples of 2,000 classes, its largest holding 90,000).
-constexpr std::uint32_t kPart = 512;
-constexpr int kPerLane = kPart / 64;
-
-// first_part[c] = parts of the classes before c; [classes] = all parts.
-__global__ __launch_bounds__(1024) void k_calib_parts(const std::uint32_t* starts,
-                                                      std::size_t classes, std::size_t n,
-                                                      std::uint32_t* first_part)
-{
-    __shared__ std::uint32_t sh[1024 / 64];
-    __shared__ std::uint32_t total;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    std::uint32_t before = 0;
-    for (std::size_t b = 0; b < classes; b += 1024) {
-        const std::size_t c = b + threadIdx.x;
-        std::uint32_t v = 0;
-        if (c < classes) {
-            const std::size_t e = c + 1 < classes ? starts[c + 1] : n;
-            v = static_cast<std::uint32_t>((e - starts[c] + kPart - 1) / kPart);
-        }
-        std::uint32_t incl = v;
-        for (int off = 1; off < 64; off <<= 1) {
-            const std::uint32_t o = __shfl_up(incl, off);
-            incl += lane >= off ? o : 0u;
-        }
-        if (lane == 63) {
-            sh[wave] = incl;
-        }
-        __syncthreads();
-        std::uint32_t waves = 0;
-        for (int w = 0; w < wave; ++w) {
-            waves += sh[w];
-        }
-        if (c < classes) {
-            first_part[c] = before + waves + incl - v;
-        }
-        if (threadIdx.x == 1023) {
-            total = waves + incl;
-        }
-        __syncthreads();
-        before += total;
+// The sorted samples: `key` holds the latency below `shift` bits and the class
+// number above them; with `cls` it is the latency alone and cls the number.
+template <typename K>
+struct Samples {
+    const K* key;
+    const std::uint32_t* cls;
+    unsigned shift;
+    std::uint64_t mask;
+    const std::uint32_t* starts;  // [classes]
+    std::size_t classes, n;
+    __device__ std::uint64_t latency(std::size_t j) const
+    {
+        return static_cast<std::uint64_t>(key[j]) & mask;
     }
-    if (threadIdx.x == 0) {
-        first_part[classes] = before;
+    __device__ std::size_t number(std::size_t j) const
+    {
+        return cls != nullptr ? cls[j] : static_cast<std::size_t>(key[j] >> shift);
     }
-}
-
-struct PartSum {
-    std::uint64_t lo, hi;  // 128-bit sum of the latencies
-    Pair log_sum;          // sum of their logarithms
-    Pair log_m2;           // squared deviations from the part's own mean
+    __device__ std::size_t end(std::size_t c) const { return c + 1 < classes ? starts[c + 1] : n; }
 };
 
-// One wave per part.  The part's logarithms stay in registers, so that the
-// deviations come from the part's own mean without a second pass; the parts
-// are joined by Chan, Golub and LeVeque's formula.
-template <typename K>
-__global__ __launch_bounds__(kThreads) void k_calib_part(const K* key, std::uint64_t low_mask,
-                                                         const std::uint32_t* starts,
-                                                         const std::uint32_t* first_part,
-                                                         std::size_t classes, std::size_t n,
-                                                         PartSum* parts)
+// This lane's share of samples [b, e): every kLanes-th, kAhead loads at once.
+template <int kLanes, int kAhead, typename K>
+__device__ __forceinline__ void add_samples(ClassSum& a, const Samples<K>& in, std::size_t b,
+                                            std::size_t e, double centre, int lane)
 {
-    const std::uint32_t part = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (part >= first_part[classes]) {
-        return;
-    }
-    std::size_t c = 0, up = classes;  // the last class with first_part[c] <= part
-    while (up - c > 1) {
-        const std::size_t mid = c + (up - c) / 2;
-        if (first_part[mid] <= part) {
-            c = mid;
-        } else {
-            up = mid;
+    for (std::size_t j0 = b + lane; j0 < e; j0 += kLanes * kAhead) {
+        K v[kAhead];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            const std::size_t j = j0 + static_cast<std::size_t>(k) * kLanes;
+            v[k] = in.key[j < e ? j : j0];
         }
-    }
-    const std::size_t s = starts[c] + static_cast<std::size_t>(part - first_part[c]) * kPart;
-    const std::size_t last = c + 1 < classes ? starts[c + 1] : n;
-    const std::size_t e = s + kPart < last ? s + kPart : last;
-    K v[kPerLane];  // all loads before the first logarithm
 #pragma unroll
-    for (int k = 0; k < kPerLane; ++k) {
-        const std::size_t j = s + static_cast<std::size_t>(k) * 64 + lane;
-        v[k] = key[j < e ? j : s];
-    }
-    U128 sum{0, 0};
-    double logs[kPerLane];
-    Pair log_sum{0.0, 0.0};
-#pragma unroll
-    for (int k = 0; k < kPerLane; ++k) {
-        logs[k] = 0.0;
-        if (s + static_cast<std::size_t>(k) * 64 + lane < e) {
-            const std::uint64_t x = static_cast<std::uint64_t>(v[k]) & low_mask;
-            sum = add128(sum, U128{x, 0});
-            logs[k] = log(static_cast<double>(x));
-            log_sum = pair_add(log_sum, logs[k]);
+        for (int k = 0; k < kAhead; ++k) {
+            if (j0 + static_cast<std::size_t>(k) * kLanes < e) {
+                const std::uint64_t x = static_cast<std::uint64_t>(v[k]) & in.mask;
+                const U128 s = add128(U128{a.lo, a.hi}, U128{x, 0});
+                const double d = log(static_cast<double>(x)) - centre;
+                a = ClassSum{s.lo, s.hi, pair_add(a.m1, d), pair_add(a.m2, d * d)};
+            }
         }
-    }
-    sum = wave_sum128(sum);
-    log_sum = wave_pair(log_sum);
-    const double mean = (log_sum.hi + log_sum.lo) / static_cast<double>(e - s);
-    Pair m2{0.0, 0.0};
-#pragma unroll
-    for (int k = 0; k < kPerLane; ++k) {
-        const double d = s + static_cast<std::size_t>(k) * 64 + lane < e ? logs[k] - mean : 0.0;
-        m2 = pair_add(m2, d * d);
-    }
-    m2 = wave_pair(m2);
-    if (lane == 0) {
-        parts[part] = PartSum{sum.lo, sum.hi, log_sum, m2};
     }
 }
 
-// One wave per class: its parts in a fixed tree (the result depends only on
-// the samples), and the estimate of calibrator.cpp:107-136.
 template <typename K>
-__global__ __launch_bounds__(kThreads) void k_calib_rows(
-    ClassTable t, const std::uint32_t* list, const std::uint32_t* number, const K* key,
-    std::uint64_t low_mask, const std::uint32_t* starts, const std::uint32_t* first_part,
-    const PartSum* parts, std::size_t classes, std::size_t n, hbfsim_amd_calibration* rows)
+__device__ __forceinline__ double median_log(const Samples<K>& in, std::size_t c)
 {
-    const std::size_t j = static_cast<std::size_t>(blockIdx.x) * (kThreads / 64) +
-                          (threadIdx.x >> 6);
+    const std::size_t s = in.starts[c];
+    return log(static_cast<double>(in.latency(s + rank_index(in.end(c) - s, 50, 100))));
+}
+
+// Whole runs of kPart sorted samples that lie within one class are summed by a
+// wave each, so that one large class does not hold up the rest (one 256-thread
+// block per class took 248 us at 4M samples of 2,000 classes, its largest
+// holding 90,000).
+constexpr std::uint32_t kPart = 512;
+
+template <typename K>
+__global__ __launch_bounds__(kThreads) void k_calib_part(Samples<K> in, ClassSum* parts)
+{
+    const std::size_t part =
+        static_cast<std::size_t>(blockIdx.x) * (kThreads / 64) + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    if (j >= classes) {
+    const std::size_t b = part * kPart, e = b + kPart;
+    if (e > in.n) {
         return;
     }
-    const std::uint32_t slot = list[j];
-    const std::size_t c = number[slot];
-    const std::size_t s = starts[c];
-    const std::size_t e = c + 1 < classes ? starts[c + 1] : n;
-    const std::uint64_t size = e - s;
-    const std::uint32_t p0 = first_part[c], np = first_part[c + 1] - p0;
-    U128 sum{0, 0};
-    Pair log_sum{0.0, 0.0};
-    for (std::uint32_t p = lane; p < np; p += 64) {
-        sum = add128(sum, U128{parts[p0 + p].lo, parts[p0 + p].hi});
-        log_sum = pair_join(log_sum, parts[p0 + p].log_sum);
+    const std::size_t c = in.number(b);
+    if (in.number(e - 1) != c) {
+        return;
     }
-    sum = wave_sum128(sum);
-    log_sum = wave_pair(log_sum);
-    const double log_mean = (log_sum.hi + log_sum.lo) / static_cast<double>(size);
-    Pair m2{0.0, 0.0};
-    for (std::uint32_t p = lane; p < np; p += 64) {
-        const std::uint64_t left = size - static_cast<std::uint64_t>(p) * kPart;
-        const double m = static_cast<double>(left < kPart ? left : kPart);
-        const Pair l = parts[p0 + p].log_sum;
-        const double d = (l.hi + l.lo) / m - log_mean;
-        m2 = pair_add(pair_join(m2, parts[p0 + p].log_m2), m * d * d);
-    }
-    m2 = wave_pair(m2);
+    ClassSum v{0, 0, {0.0, 0.0}, {0.0, 0.0}};
+    add_samples<64, kPart / 64>(v, in, b, e, median_log(in, c), lane);
+    v = lanes_sum<64>(v);
     if (lane == 0) {
-        const auto at = [&](std::uint64_t k) {
-            return static_cast<std::uint64_t>(key[s + k]) & low_mask;
-        };
-        hbfsim_amd_calibration r;
-        r.access = load_class(t.access, t.slot[slot], t.aligned);
-        r.count = size;
-        r.mean_ns = div128(sum, size);
-        r.p50_ns = at(rank_index(size, 50, 100));
-        r.p95_ns = at(rank_index(size, 95, 100));
-        r.p99_ns = at(rank_index(size, 99, 100));
-        r.log_mean = log_mean;
-        r.log_sigma = sqrt((m2.hi + m2.lo) / static_cast<double>(size));
-        rows[c] = r;
+        parts[part] = v;
+    }
+}
+
+// kLanes lanes per class: its whole parts and the samples on either side of
+// them, in a fixed order (the result depends only on the samples), and the
+// estimate of calibrator.cpp:107-136.
+template <typename K, int kLanes>
+__global__ __launch_bounds__(kThreads) void k_calib_rows(ClassTable t, const std::uint32_t* list,
+                                                         const std::uint32_t* number, Samples<K> in,
+                                                         const ClassSum* parts,
+                                                         hbfsim_amd_calibration* rows)
+{
+    const int lane = threadIdx.x % kLanes;
+    const std::size_t stride = static_cast<std::size_t>(gridDim.x) * (kThreads / kLanes);
+    for (std::size_t j = static_cast<std::size_t>(blockIdx.x) * (kThreads / kLanes) +
+                         threadIdx.x / kLanes;
+         j < in.classes; j += stride) {
+        const std::uint32_t slot = list[j];
+        const std::size_t c = number[slot];
+        const std::size_t s = in.starts[c], e = in.end(c);
+        const std::uint64_t size = e - s;
+        const double centre = median_log(in, c);
+        const std::size_t p0 = (s + kPart - 1) / kPart, p1 = e / kPart;
+        ClassSum v{0, 0, {0.0, 0.0}, {0.0, 0.0}};
+        constexpr int kAhead = kLanes == 64 ? 8 : 2;
+        if (p0 < p1) {
+            for (std::size_t p = p0 + lane; p < p1; p += kLanes) {
+                v = sum_join(v, parts[p]);
+            }
+            add_samples<kLanes, kAhead>(v, in, s, p0 * kPart, centre, lane);
+            add_samples<kLanes, kAhead>(v, in, p1 * kPart, e, centre, lane);
+        } else {
+            add_samples<kLanes, kAhead>(v, in, s, e, centre, lane);
+        }
+        v = lanes_sum<kLanes>(v);
+        if (lane == 0) {
+            const double m1 = (v.m1.hi + v.m1.lo) / static_cast<double>(size);
+            const double m2 = (v.m2.hi + v.m2.lo) / static_cast<double>(size);
+            const double variance = m2 - m1 * m1;
+            hbfsim_amd_calibration r;
+            r.access = load_class(t.access, t.slot[slot], t.aligned);
+            r.count = size;
+            r.mean_ns = div128(U128{v.lo, v.hi}, size);
+            r.p50_ns = in.latency(s + rank_index(size, 50, 100));
+            r.p95_ns = in.latency(s + rank_index(size, 95, 100));
+            r.p99_ns = in.latency(s + rank_index(size, 99, 100));
+            r.log_mean = centre + m1;
+            r.log_sigma = sqrt(variance > 0.0 ? variance : 0.0);
+            rows[c] = r;
+        }
     }
 }
 
@@ -908,8 +914,9 @@ int sampler_reference(sampler_state* s, const hbfsim_amd_access_class* d_access,
     hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
     const std::uint64_t most = most_slots(n, s->seen);
     std::uint64_t cap = first_slots(s->seen, most);
-    unsigned long long host[4] = {0, 0, 0, 0};  // references, new classes, overflow, -
-    for (;; cap = next_slots(cap, most)) {
+    // references, new classes, overflow | classes sampled << 32, -
+    unsigned long long host[4] = {0, 0, 0, 0};
+    for (;; cap = next_slots(cap, most, static_cast<std::uint32_t>(host[2] >> 32))) {
         TablePlan p(cap);
         ScratchLease lease(p.plan.bytes, stream);
         if (!lease.ok()) {
@@ -918,7 +925,8 @@ int sampler_reference(sampler_state* s, const hbfsim_amd_access_class* d_access,
         auto* words = lease.at<unsigned long long>(p.o_words);
         ClassTable t{lease.at<unsigned long long>(p.o_slot), lease.at<std::uint32_t>(p.o_first),
                      cap - 1, cap < most ? kProbes : 0u, d_access, s->seen_class,
-                     reinterpret_cast<std::uint32_t*>(words + 2), aligned16(d_access)};
+                     reinterpret_cast<std::uint32_t*>(words + 2), sample_limit(cap, most),
+                     aligned16(d_access)};
         hipError_t err = hipMemsetAsync(t.slot, 0xff, p.o_words - p.o_slot, stream);
         if (err == hipSuccess) err = hipMemsetAsync(words, 0, sizeof(host), stream);
         if (err != hipSuccess) {
@@ -944,7 +952,7 @@ int sampler_reference(sampler_state* s, const hbfsim_amd_access_class* d_access,
         if (err != hipSuccess) {
             return HBFSIM_CUDA_ERROR;
         }
-        if (host[2] != 0) {
+        if (static_cast<std::uint32_t>(host[2]) != 0) {
             continue;  // the table was too small; the largest never is
         }
         if (host[1] != 0) {
@@ -999,7 +1007,8 @@ namespace {
 template <typename K, bool kWide>
 int calibrate_rows(const ClassTable& t, const std::uint64_t* d_latency, std::size_t n,
                    const std::uint32_t* slot_of, const std::uint32_t* list,
-                   const ulonglong2* keys, std::size_t classes, unsigned shift, hbfsim_amd_calibration* d_rows, hipStream_t stream)
+                   const ulonglong2* keys, std::size_t classes, unsigned shift,
+                   hbfsim_amd_calibration* d_rows, hipStream_t stream)
 {
     const unsigned number_bits = [&] {
         unsigned b = 1;
@@ -1009,7 +1018,7 @@ int calibrate_rows(const ClassTable& t, const std::uint64_t* d_latency, std::siz
         return b;
     }();
     const bool counted = classes <= kCountedClasses;
-    const std::size_t parts = classes + n / kPart;
+    const std::size_t parts = n / kPart;
     std::size_t tb_class = 0, tb_main = 0, tb_second = 0;
     hipError_t err = hipSuccess;
     if (!counted) {
@@ -1045,8 +1054,7 @@ int calibrate_rows(const ClassTable& t, const std::uint64_t* d_latency, std::siz
     }
     ScratchPlan p;
     const std::size_t o_starts = p.add<std::uint32_t>(classes);
-    const std::size_t o_first = p.add<std::uint32_t>(classes + 1);
-    const std::size_t o_parts = p.add<PartSum>(parts);
+    const std::size_t o_parts = p.add<ClassSum>(parts);
     const std::size_t o_a = p.add<K>(n), o_b = p.add<K>(n);
     const std::size_t o_na = p.add<std::uint32_t>(kWide ? n : 0);
     const std::size_t o_nb = p.add<std::uint32_t>(kWide ? n : 0);
@@ -1088,8 +1096,8 @@ int calibrate_rows(const ClassTable& t, const std::uint64_t* d_latency, std::siz
     K* b = lease.at<K>(o_b);
     const K* sorted = b;
     auto* starts = lease.at<std::uint32_t>(o_starts);
-    auto* first_part = lease.at<std::uint32_t>(o_first);
-    auto* psum = lease.at<PartSum>(o_parts);
+    auto* psum = lease.at<ClassSum>(o_parts);
+    const std::uint32_t* cls = nullptr;
     const dim3 wide(stride_blocks(n));
     if constexpr (kWide) {
         auto* na = lease.at<std::uint32_t>(o_na);
@@ -1104,6 +1112,7 @@ int calibrate_rows(const ClassTable& t, const std::uint64_t* d_latency, std::siz
                                             stream);
         }
         sorted = a;
+        cls = na;
         hipLaunchKernelGGL((k_calib_starts<std::uint32_t>), wide, block, 0, stream,
                            static_cast<const std::uint32_t*>(na), n, 0u, starts);
     } else {
@@ -1115,13 +1124,20 @@ int calibrate_rows(const ClassTable& t, const std::uint64_t* d_latency, std::siz
         hipLaunchKernelGGL((k_calib_starts<K>), wide, block, 0, stream, sorted, n, shift, starts);
     }
     const std::uint64_t low_mask = kWide || shift >= 64 ? ~0ull : (1ull << shift) - 1;
-    hipLaunchKernelGGL(k_calib_parts, dim3(1), dim3(1024), 0, stream, starts, classes, n,
-                       first_part);
-    hipLaunchKernelGGL((k_calib_part<K>), dim3(blocks_for(parts * 64)), block, 0, stream, sorted,
-                       low_mask, starts, first_part, classes, n, psum);
-    hipLaunchKernelGGL((k_calib_rows<K>), dim3(blocks_for(classes * 64)), block, 0, stream, t,
-                       list, number, sorted, low_mask, starts, first_part, psum, classes, n,
-                       d_rows);
+    const Samples<K> in{sorted, cls, shift, low_mask, starts, classes, n};
+    if (parts != 0) {
+        hipLaunchKernelGGL((k_calib_part<K>), dim3(blocks_for(parts * 64)), block, 0, stream, in,
+                           psum);
+    }
+    // a wave per class, or eight lanes where classes hold fewer than 32 samples
+    // on average (4M samples of 4M classes: the whole call 19.5 ms with a wave
+    // per class and a scan over the classes' parts, 2.2 ms now; 1M classes 10.0
+    // and 1.4, 2,000 classes 438 and 429 us)
+    const bool few = n / 32 < classes;
+    const dim3 groups(static_cast<unsigned>(std::min<std::size_t>(
+        std::size_t{1} << 20, blocks_for(classes * (few ? 8 : 64)))));
+    hipLaunchKernelGGL((few ? k_calib_rows<K, 8> : k_calib_rows<K, 64>), groups, block, 0, stream,
+                       t, list, number, in, psum, d_rows);
     if (err == hipSuccess) err = hipGetLastError();
     if (err == hipSuccess) err = hipStreamSynchronize(stream);
     if (err != hipSuccess) {
@@ -1151,7 +1167,9 @@ int calibrate(const hbfsim_amd_access_class* d_access, const std::uint64_t* d_la
     hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
     const std::uint64_t most = most_slots(n, 0, std::uint64_t{1} << 32);
     std::uint64_t cap = first_slots(0, most);
-    for (;; cap = next_slots(cap, most)) {
+    // classes, largest latency, overflow | classes sampled << 32, zero latency
+    unsigned long long host[4] = {0, 0, 0, 0};
+    for (;; cap = next_slots(cap, most, static_cast<std::uint32_t>(host[2] >> 32))) {
         TablePlan p(cap);
         const std::size_t o_slot_of = p.plan.add<std::uint32_t>(n);
         const std::size_t o_list = p.plan.add<std::uint32_t>(std::min<std::uint64_t>(cap, n));
@@ -1160,15 +1178,14 @@ int calibrate(const hbfsim_amd_access_class* d_access, const std::uint64_t* d_la
         if (!lease.ok()) {
             return HBFSIM_CUDA_ERROR;
         }
-        // words: classes, largest latency, overflow, zero latency
         auto* words = lease.at<unsigned long long>(p.o_words);
         ClassTable t{lease.at<unsigned long long>(p.o_slot), lease.at<std::uint32_t>(p.o_first),
                      cap - 1, cap < most ? kProbes : 0u, d_access, nullptr,
-                     reinterpret_cast<std::uint32_t*>(words + 2), aligned16(d_access)};
+                     reinterpret_cast<std::uint32_t*>(words + 2), sample_limit(cap, most),
+                     aligned16(d_access)};
         auto* slot_of = lease.at<std::uint32_t>(o_slot_of);
         auto* list = lease.at<std::uint32_t>(o_list);
         auto* keys = lease.at<ulonglong2>(o_keys);
-        unsigned long long host[4] = {0, 0, 0, 0};
         hipError_t err = hipMemsetAsync(t.slot, 0xff, p.o_first - p.o_slot, stream);
         if (err == hipSuccess) err = hipMemsetAsync(words, 0, sizeof(host), stream);
         if (err != hipSuccess) {
@@ -1193,7 +1210,7 @@ int calibrate(const hbfsim_amd_access_class* d_access, const std::uint64_t* d_la
         if (host[3] != 0) {
             return HBFSIM_INVALID_ARGUMENT;  // Calibrator::observe: latency_ns must be positive
         }
-        if (host[2] != 0) {
+        if (static_cast<std::uint32_t>(host[2]) != 0) {
             continue;  // the table was too small; the largest never is
         }
         const std::size_t classes = host[0];

@@ -25,11 +25,14 @@ int main()
         for (std::size_t seen : held) {
             const std::uint64_t most = most_slots(n, seen);
             CHECK(most >= 2 * (n + seen) && (most & (most - 1)) == 0);
-            std::uint64_t cap = first_slots(seen, most);
-            int steps = 0;
-            for (; cap != most; cap = next_slots(cap, most)) {
-                CHECK((cap & (cap - 1)) == 0 && cap > seen);
-                CHECK(++steps < 10);
+            for (std::uint32_t sampled : {0u, 16384u}) {
+                std::uint64_t cap = first_slots(seen, most);
+                int steps = 0;
+                for (; cap != most; cap = next_slots(cap, most, sampled)) {
+                    CHECK((cap & (cap - 1)) == 0 && cap > seen);
+                    CHECK(++steps < 10);
+                }
+                CHECK(sample_limit(cap, most) >= kSample);  // the last table is always tried
             }
             CHECK(std::uint64_t{walk_blocks(most)} * 256 < 1ull << 32);
             CHECK(walk_blocks(most) != 0);
