@@ -1067,6 +1067,8 @@ int calibrate_rows(const ClassTable& t, const std::uint64_t* d_latency, std::siz
     if (!lease.ok()) {
         return HBFSIM_CUDA_ERROR;
     }
+    // Sorted class numbers are indices to what follows: nothing is launched after
+    // a sort that failed (the lease then waits for what was).
     void* temp = lease.at<unsigned char>(o_temp);
     std::uint32_t* number = t.first;  // [slots]
     const dim3 block(kThreads);
@@ -1082,12 +1084,15 @@ int calibrate_rows(const ClassTable& t, const std::uint64_t* d_latency, std::siz
                            stream, keys, static_cast<const std::uint32_t*>(nullptr), classes, ka,
                            ia);
         err = rocprim::radix_sort_pairs(temp, tb_class, ka, kb, ia, ib, classes, 0, 64, stream);
-        if (err == hipSuccess) {
-            hipLaunchKernelGGL((k_calib_class_keys<true>), dim3(blocks_for(classes)), block, 0,
-                               stream, keys, static_cast<const std::uint32_t*>(ib), classes, ka,
-                               static_cast<std::uint32_t*>(nullptr));
-            err = rocprim::radix_sort_pairs(temp, tb_class, ka, kb, ib, ia, classes, 0, 64,
-                                            stream);
+        if (err != hipSuccess) {
+            return HBFSIM_CUDA_ERROR;
+        }
+        hipLaunchKernelGGL((k_calib_class_keys<true>), dim3(blocks_for(classes)), block, 0, stream,
+                           keys, static_cast<const std::uint32_t*>(ib), classes, ka,
+                           static_cast<std::uint32_t*>(nullptr));
+        err = rocprim::radix_sort_pairs(temp, tb_class, ka, kb, ib, ia, classes, 0, 64, stream);
+        if (err != hipSuccess) {
+            return HBFSIM_CUDA_ERROR;
         }
         hipLaunchKernelGGL(k_calib_renumber, dim3(blocks_for(classes)), block, 0, stream, list,
                            static_cast<const std::uint32_t*>(ia), classes, number);
@@ -1103,13 +1108,13 @@ int calibrate_rows(const ClassTable& t, const std::uint64_t* d_latency, std::siz
         auto* na = lease.at<std::uint32_t>(o_na);
         auto* nb = lease.at<std::uint32_t>(o_nb);
         hipLaunchKernelGGL(k_calib_numbers, wide, block, 0, stream, slot_of, number, n, na);
-        if (err == hipSuccess) {
-            err = rocprim::radix_sort_pairs(temp, tb_main, d_latency, b, na, nb, n, 0, shift,
-                                            stream);
-        }
+        err = rocprim::radix_sort_pairs(temp, tb_main, d_latency, b, na, nb, n, 0, shift, stream);
         if (err == hipSuccess) {
             err = rocprim::radix_sort_pairs(temp, tb_second, nb, na, b, a, n, 0, number_bits,
                                             stream);
+        }
+        if (err != hipSuccess) {
+            return HBFSIM_CUDA_ERROR;
         }
         sorted = a;
         cls = na;
@@ -1118,8 +1123,9 @@ int calibrate_rows(const ClassTable& t, const std::uint64_t* d_latency, std::siz
     } else {
         hipLaunchKernelGGL((k_calib_keys<K>), wide, block, 0, stream, slot_of, number, d_latency,
                            n, shift, a);
-        if (err == hipSuccess) {
-            err = rocprim::radix_sort_keys(temp, tb_main, a, b, n, 0, shift + number_bits, stream);
+        err = rocprim::radix_sort_keys(temp, tb_main, a, b, n, 0, shift + number_bits, stream);
+        if (err != hipSuccess) {
+            return HBFSIM_CUDA_ERROR;
         }
         hipLaunchKernelGGL((k_calib_starts<K>), wide, block, 0, stream, sorted, n, shift, starts);
     }
@@ -1138,7 +1144,7 @@ int calibrate_rows(const ClassTable& t, const std::uint64_t* d_latency, std::siz
         std::size_t{1} << 20, blocks_for(classes * (few ? 8 : 64)))));
     hipLaunchKernelGGL((few ? k_calib_rows<K, 8> : k_calib_rows<K, 64>), groups, block, 0, stream,
                        t, list, number, in, psum, d_rows);
-    if (err == hipSuccess) err = hipGetLastError();
+    err = hipGetLastError();
     if (err == hipSuccess) err = hipStreamSynchronize(stream);
     if (err != hipSuccess) {
         return HBFSIM_CUDA_ERROR;
