@@ -935,6 +935,17 @@ HBF_API int hbfsim_amd_last_apply_waves(const hbfsim_context* c)
     return hbfamd::engine_last_apply_waves(c->eng);
 }
 
+HBF_API int hbfsim_amd_last_tiles(hbfsim_context* c, uint64_t* batched, uint64_t* scattered)
+{
+    if (c == nullptr || batched == nullptr || scattered == nullptr) {
+        return HBFSIM_INVALID_ARGUMENT;
+    }
+    std::lock_guard<std::mutex> lock(c->mu);
+    *batched = 0;
+    *scattered = 0;
+    return c->eng == nullptr ? HBFSIM_OK : hbfamd::engine_last_tiles(c->eng, batched, scattered);
+}
+
 HBF_API int hbfsim_amd_lookup_range(hbfsim_context* c, uint64_t address, uint32_t bytes,
                                     uint32_t* kind, hbfsim_amd_range* out, uint32_t* count)
 {

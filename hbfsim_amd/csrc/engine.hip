@@ -5204,6 +5204,10 @@ struct engine {
     std::uint64_t last_modeled{0};
     std::uint64_t last_hits{0};
     int last_apply_waves{0};  // waves per SIMD the last run's apply pass was built for
+    // the last run's tiles, and which passes were launched over them (with both,
+    // d_tsplit says which took a tile; a run that reuses d_tsplit sets these too)
+    enum class Passes { none, batched, scattered, both } last_passes{Passes::none};
+    std::size_t last_tiles{0};
 };
 
 // Where one run of the main pipeline keeps its per-tile and per-group
@@ -7181,6 +7185,7 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
         return HBFSIM_UNSUPPORTED;
     }
     hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
+    e->last_passes = engine::Passes::none;
     if (hipSetDevice(e->device) != hipSuccess) {
         return HBFSIM_CUDA_ERROR;
     }
@@ -7511,6 +7516,12 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
     }
     e->last_modeled = e->h_out->rep.v[R_MODELED];
     e->last_hits = e->h_out->rep.v[R_HITS];
+    if (ext_scratch == nullptr) {
+        e->last_tiles = ntiles;
+        e->last_passes = plain_alone   ? engine::Passes::scattered
+                         : plain_mixed ? engine::Passes::both
+                                       : engine::Passes::batched;
+    }
     note_times(e);
     if (out != nullptr) {
         std::memcpy(out, &e->h_out->rep, sizeof(DevReport));
@@ -7642,6 +7653,27 @@ int engine_last_apply_waves(const engine* e)
     return e->last_apply_waves;
 }
 
+int engine_last_tiles(const engine* e, std::uint64_t* batched, std::uint64_t* scattered)
+{
+    *batched = e->last_passes == engine::Passes::batched ? e->last_tiles : 0;
+    *scattered = e->last_passes == engine::Passes::scattered ? e->last_tiles : 0;
+    if (e->last_passes != engine::Passes::both) {
+        return HBFSIM_OK;
+    }
+    try {
+        std::vector<std::uint8_t> kind(e->last_tiles);
+        if (hipSetDevice(e->device) != hipSuccess ||
+            hipMemcpy(kind.data(), e->d_tsplit, kind.size(), hipMemcpyDeviceToHost) !=
+                hipSuccess) {
+            return HBFSIM_CUDA_ERROR;
+        }
+        *scattered = static_cast<std::uint64_t>(std::count(kind.begin(), kind.end(), kTilePlain));
+        *batched = kind.size() - *scattered;
+    } catch (const std::bad_alloc&) {
+        return HBFSIM_CUDA_ERROR;
+    }
+    return HBFSIM_OK;
+}
 
 int engine_window_counts(engine* e, const hbf_record32* d_rec, std::size_t n,
                          std::uint64_t window_ps, std::uint64_t windows, std::uint32_t* d_counts,

@@ -255,6 +255,14 @@ class Engine:
         form for large streams of general steps; results do not depend on it)."""
         return int(self._lib.hbfsim_amd_last_apply_waves(self._ctx))
 
+    def last_tiles(self) -> tuple[int, int]:
+        """Tiles of the last run that the batched passes took, and that the
+        scattered-record passes took."""
+        batched, scattered = ctypes.c_uint64(), ctypes.c_uint64()
+        nat.check(self._lib.hbfsim_amd_last_tiles(self._ctx, ctypes.byref(batched),
+                                                  ctypes.byref(scattered)), "last tiles")
+        return int(batched.value), int(scattered.value)
+
     def run_coupled(self, thermal: "Thermal", options: dict, records: Any, completion: Any,
                     temperature: Any, age_ps: np.ndarray, stream: Any = None) -> tuple[dict, dict]:
         """Thermal-coupled run (hbfsim_amd_run_coupled): returns the coupled

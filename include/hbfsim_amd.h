@@ -396,6 +396,13 @@ int hbfsim_amd_last_kernel_ms(const hbfsim_context* context, float* ms,
  * records), 0 before any run and after an empirical-model run (no apply
  * pass).  Results do not depend on the form. */
 int hbfsim_amd_last_apply_waves(const hbfsim_context* context);
+/* Diagnostics likewise: how many tiles of the last run the batched passes
+ * took (k_summary, k_apply: runs of lines, refresh records, grouping, two page
+ * registers) and how many the scattered-record passes (k_plain_summary,
+ * k_plain_apply).  Both 0 before any run, after an empirical-model run, after
+ * one that failed and after one through the entry point that allocates
+ * nothing. */
+int hbfsim_amd_last_tiles(hbfsim_context* context, uint64_t* batched, uint64_t* scattered);
 
 /* One registered range as the registry holds it (SharedRangeRecord,
  * hbf_device.cuh:105-117). */

@@ -72,6 +72,12 @@ class Pair:
                                             self.ostate)
         return (gcomp, gst, grep), (ocomp, ost, orep)
 
+    def check_batched(self, all_tiles=False):
+        """The last run's tiles went mostly (or all) to the batched passes."""
+        batched, scattered = self.engine.last_tiles()
+        assert batched > scattered, f"{batched} tiles batched, {scattered} scattered"
+        assert scattered == 0 or not all_tiles, f"{scattered} tiles scattered"
+
     def check_state(self):
         gp, gc = self.engine.busy_totals()
         np.testing.assert_array_equal(gp, self.ostate.plane_busy_total, "plane busy totals")

@@ -24,6 +24,11 @@ TILE = 256  # records per tile
 FEW = 3 * 4 * 256  # tiles in one round of three-wave slots
 
 
+# 128 ranges more than these tables hold: the scattered-record passes take no
+# tile, and general steps go through the batched passes
+MANY = [(0x7A00_0000_0000 + k * (1 << 20), 1 << 16, 1) for k in range(128)]
+
+
 def mixed(n, seed, side):
     """n records: random general steps with linear, grouped and split steps
     in between, in issue order."""
@@ -36,9 +41,10 @@ def mixed(n, seed, side):
 
 
 @pytest.mark.parametrize("tiles", [FEW, FEW + 1], ids=["few-tiles form", "four-wave form"])
-def test_summary_forms_at_the_tile_boundary(tiles):
+@pytest.mark.parametrize("more", [[], MANY], ids=["", "many ranges"])
+def test_summary_forms_at_the_tile_boundary(tiles, more):
     side = ranges_for()
-    ranges = [(workloads.RANGE_BASE, 1 << 30, 3)] + side
+    ranges = [(workloads.RANGE_BASE, 1 << 30, 3)] + side + more
     rec = mixed(tiles * TILE, 40 + tiles % 2, side)
     assert len(rec) == tiles * TILE
     p = parity.Pair(C0, ranges, tile_records=TILE)
@@ -47,22 +53,27 @@ def test_summary_forms_at_the_tile_boundary(tiles):
         for k in range(2):  # the second run starts from the first one's state
             g, c = p.run_packed(rec, base_ps=base)
             parity.assert_same(g, c, f"{tiles} tiles, run {k}")
+            if more:
+                p.check_batched(all_tiles=True)
             base = int(g[2]["makespan_ps"])
         p.check_state()
     finally:
         p.close()
 
 
-def test_summary_lds_bound_form_with_general_steps():
+@pytest.mark.parametrize("more", [[], MANY], ids=["", "many ranges"])
+def test_summary_lds_bound_form_with_general_steps(more):
     """Config 2's 512-plane geometry: the LDS-bound summary form, without the
     stripe table, on the same kind of mixed stream."""
     side = ranges_for()
-    ranges = [(workloads.RANGE_BASE, 1 << 30, 3)] + side
+    ranges = [(workloads.RANGE_BASE, 1 << 30, 3)] + side + more
     rec = mixed(600 * TILE, 51, side)
     p = parity.Pair(C2, ranges, tile_records=TILE)
     try:
         g, c = p.run_packed(rec)
         parity.assert_same(g, c, "config 2 geometry, mixed stream")
+        if more:
+            p.check_batched(all_tiles=True)
         p.check_state()
     finally:
         p.close()

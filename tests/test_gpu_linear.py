@@ -99,7 +99,8 @@ def linear_stream(seed, steps, ranges, kinds=None):
 @pytest.mark.parametrize("profile", [C0, C2], ids=["c0", "c2"])
 @pytest.mark.parametrize("options", [
     dict(), dict(plane_contention=0), dict(transfer_page=1), dict(tile_records=64 * 64),
-    dict(tile_records=64 * 70),
+    dict(tile_records=64 * 70), dict(plane_contention=0, tile_records=64 * 70),
+    dict(transfer_page=1, tile_records=64 * 70), dict(tile_records=64 * 8),
 ])
 def test_linear_batches_bit_exact(profile, options):
     ranges = ranges_for()
@@ -108,6 +109,8 @@ def test_linear_batches_bit_exact(profile, options):
     try:
         (_, _, grep), _ = check(p, rec, f"linear batches {profile.name} {options}")
         assert grep["page_hits"] > 0 and grep["bypass"] > 0 and grep["unsupported"] > 0
+        if "tile_records" in options:  # (short tiles of short runs take the scattered passes)
+            p.check_batched()
         p.check_state()
     finally:
         p.close()
@@ -152,13 +155,16 @@ def test_linear_batch_lengths(n_linear):
         p = parity.Pair(C2, ranges, tile_records=tile)
         try:
             check(p, stream, f"{n_linear} linear steps, tile {tile}")
+            if (tile or 0) >= 64 * 8:
+                p.check_batched()
             p.check_state()
         finally:
             p.close()
 
 
+@pytest.mark.parametrize("tile", [None, 64 * 64])
 @pytest.mark.parametrize("wide", ["issue", "sense", "transfer"])
-def test_linear_wide_times_take_64_bit_scans(tmp_path, wide):
+def test_linear_wide_times_take_64_bit_scans(tmp_path, wide, tile):
     """Values past the 32-bit relative scans inside one batch: issue gaps
     beyond 2^30 ps between steps, a sense time of 4e7 ps (> 2^24), or a
     transfer quantum that makes a step's channel time 2^26 ps."""
@@ -176,21 +182,24 @@ def test_linear_wide_times_take_64_bit_scans(tmp_path, wide):
         profile.write_text(json.dumps(prof))
     else:
         opts = dict(xfer_quantum_ps=1 << 20)
-    p = parity.Pair(profile, ranges, **opts)
+    p = parity.Pair(profile, ranges, tile_records=tile, **opts)
     try:
         check(p, rec, f"wide linear steps ({wide})")
+        if tile is not None:
+            p.check_batched(all_tiles=True)
         p.check_state()
     finally:
         p.close()
 
 
-def test_linear_split_runs_resume():
+@pytest.mark.parametrize("tile", [None, 64 * 24])
+def test_linear_split_runs_resume(tile):
     """A stream cut inside batches: the carried state after each run must let
     the next run continue exactly."""
     ranges = ranges_for()
     rec = linear_stream(17, 900, ranges)
-    whole = parity.Pair(C2, ranges)
-    split = parity.Pair(C2, ranges)
+    whole = parity.Pair(C2, ranges, tile_records=tile)
+    split = parity.Pair(C2, ranges, tile_records=tile)
     try:
         (gw, _, _), _ = check(whole, rec, "whole")
         parts = []
@@ -244,7 +253,9 @@ def contiguous_stream(seed, runs, ranges):
 
 
 @pytest.mark.parametrize("options", [dict(), dict(plane_contention=0), dict(transfer_page=1),
-                                     dict(tile_records=64 * 24)])
+                                     dict(tile_records=64 * 24),
+                                     dict(plane_contention=0, tile_records=64 * 24),
+                                     dict(transfer_page=1, tile_records=64 * 24)])
 def test_linear_groups_bit_exact(options):
     ranges = ranges_for()
     rec = contiguous_stream(23, 400, ranges)
@@ -253,6 +264,8 @@ def test_linear_groups_bit_exact(options):
         try:
             (_, _, grep), _ = check(p, rec, f"linear groups {profile.name} {options}")
             assert grep["page_hits"] > 0
+            if "tile_records" in options:
+                p.check_batched()
             p.check_state()
         finally:
             p.close()
@@ -276,10 +289,11 @@ def striding_stream(pages, b, seed, reps=2):
     return np.concatenate(out)
 
 
+@pytest.mark.parametrize("tile", [None, 64 * 64])
 @pytest.mark.parametrize("profile,planes", [(C0, 64), (C2, 512)], ids=["c0", "c2"])
 @pytest.mark.parametrize("shape", ["stride1", "span_below", "span_equal", "stride_over",
                                    "pairs"])
-def test_linear_batches_rising_pages_across_one_stripe_period(profile, planes, shape):
+def test_linear_batches_rising_pages_across_one_stripe_period(profile, planes, shape, tile):
     """Batches whose pages rise from step to step: within one striping period
     (span below the plane count) the runs of equal page are the plane groups;
     from a span of one period on, two pages of a batch may share a plane and
@@ -298,10 +312,12 @@ def test_linear_batches_rising_pages_across_one_stripe_period(profile, planes, s
     assert pages == sorted(pages)
     ranges = [(BASE, 1200 * PAGE, 1)]
     rec = striding_stream(pages, 128 if shape == "pairs" else 256, len(pages) + planes)
-    p = parity.Pair(profile, ranges)
+    p = parity.Pair(profile, ranges, tile_records=tile)
     try:
         (_, _, grep), _ = check(p, rec, f"rising pages {shape} on {planes} planes")
         assert grep["modeled"] == len(rec)
+        if tile is not None:
+            p.check_batched(all_tiles=True)
         p.check_state()
     finally:
         p.close()

@@ -27,7 +27,9 @@ def check_packed(pair, rec, what, base_ps=0):
 
 @pytest.mark.parametrize("profile", [C0, C2], ids=["c0", "c2"])
 @pytest.mark.parametrize("options", [dict(), dict(plane_contention=0), dict(transfer_page=1),
-                                     dict(tile_records=64 * 24), dict(tile_records=64 * 300)])
+                                     dict(tile_records=64 * 24), dict(tile_records=64 * 300),
+                                     dict(plane_contention=0, tile_records=64 * 24),
+                                     dict(transfer_page=1, tile_records=64 * 24)])
 def test_packed_linear_and_general_paths(profile, options):
     ranges = ranges_for()
     rec = chain_clocks(linear_stream(3, 800, ranges), contiguous_stream(4, 200, ranges))
@@ -35,6 +37,8 @@ def test_packed_linear_and_general_paths(profile, options):
     try:
         (_, _, grep), _ = check_packed(p, rec, f"packed {profile.name} {options}")
         assert grep["page_hits"] > 0 and grep["bypass"] > 0 and grep["unsupported"] > 0
+        if "tile_records" in options:  # (short tiles of short runs take the scattered passes)
+            p.check_batched()
         p.check_state()
     finally:
         p.close()
@@ -58,7 +62,8 @@ def test_packed_config0_stream_and_split_runs():
         split.close()
 
 
-def test_packed_rising_pages_and_edge_fields():
+@pytest.mark.parametrize("tile", [None, 64 * 64])
+def test_packed_rising_pages_and_edge_fields(tile):
     """Batches across one striping period, and records at the packed form's
     edges: byte counts up to 65535, addresses near 2^48, issue times near
     2^56 ps (bypass records outside every range still pass through)."""
@@ -69,9 +74,11 @@ def test_packed_rising_pages_and_edge_fields():
     edge[:, 1] = 8
     edge[:64, 1] = 65535
     edge[:, 2] = np.uint64((1 << 56) - 10_000_000)
-    p = parity.Pair(C2, ranges)
+    p = parity.Pair(C2, ranges, tile_records=tile)
     try:
         check_packed(p, np.concatenate([rec, edge]), "rising pages and edges")
+        if tile is not None:
+            p.check_batched(all_tiles=True)
         p.check_state()
     finally:
         p.close()

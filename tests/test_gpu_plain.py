@@ -110,3 +110,34 @@ def test_tiles_of_lines_between_scattered_ones():
         parts.append(r)
     check(np.concatenate(parts), ranges, C0)
     check(np.concatenate(parts), ranges, C0, tile_records=4096)
+
+
+def test_which_passes_took_the_tiles():
+    """The tile counts by pass: a short run, one of mostly scattered tiles, hybrid mode and the
+    state before a run."""
+    ranges = ranges_of(3)
+    p = parity.Pair(C0, ranges)
+    try:
+        assert p.engine.last_tiles() == (0, 0)
+        p.run_packed(scattered(4099, ranges, 1))
+        batched, taken = p.engine.last_tiles()
+        assert batched == 0 and taken == -(-4099 // 64)
+    finally:
+        p.close()
+    p = parity.Pair(C0, ranges)  # (no run before it that mostly hit its registers)
+    try:
+        n = (1 << 18) + 4096
+        rec = scattered(n, ranges, 2)
+        rec[:65536] = lines(65536, ranges, 3)
+        rec[65536:, 2] += np.uint64(int(rec[65535, 2]))
+        p.run_packed(rec)
+        batched, taken = p.engine.last_tiles()
+        assert batched + taken == -(-n // 256) and batched == 65536 // 256
+    finally:
+        p.close()
+    p = parity.Pair(C0, ranges_of(129))
+    try:
+        p.run_packed(scattered(4099, ranges, 1))
+        assert p.engine.last_tiles() == (-(-4099 // 64), 0)
+    finally:
+        p.close()

@@ -12,6 +12,7 @@ import json
 import pytest
 
 import parity
+from test_gpu_forms import MANY
 from test_gpu_linear import chain_clocks, contiguous_stream, linear_stream, ranges_for
 from test_gpu_parity import C0
 from test_gpu_split import split_stream
@@ -22,7 +23,8 @@ pytestmark = pytest.mark.gpu
 BIG = 1 << 24
 
 
-def test_wide_apply_takes_over_on_general_streams():
+@pytest.mark.parametrize("more", [[], MANY], ids=["", "many ranges"])
+def test_wide_apply_takes_over_on_general_streams(more):
     first = workloads.config0(n=BIG, seed=21, write_fraction_per_mille=50)
     second = workloads.config0(n=BIG, seed=22, write_fraction_per_mille=50)
     side = ranges_for()
@@ -33,7 +35,8 @@ def test_wide_apply_takes_over_on_general_streams():
     linear = chain_clocks(linear_stream(8, 4000, side), contiguous_stream(9, 400, side))
     # tiles of 4,096 records: the large runs have more tiles than one round of
     # three-wave slots, so their summary pass is the four-wave form too
-    p = parity.Pair(C0, first.ranges + side, tile_records=4096)
+    # (with many ranges the general steps are the batched passes' too)
+    p = parity.Pair(C0, first.ranges + side + more, tile_records=4096)
     try:
         # no earlier run: the three-wave form
         g, c = p.run_packed(first.records)
@@ -43,6 +46,8 @@ def test_wide_apply_takes_over_on_general_streams():
         # the previous run was general: the four-wave form, mixed steps too
         g, c = p.run_packed(mixed, base_ps=int(g[2]["makespan_ps"]))
         parity.assert_same(g, c, "mixed run, four-wave apply")
+        if more:
+            p.check_batched(all_tiles=True)
         assert p.engine.apply_waves() == 4
         p.check_state()
         # a small run keeps the three-wave form whatever came before
