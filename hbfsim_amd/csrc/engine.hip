@@ -6482,6 +6482,20 @@ bool plain_run(const KArgs& a, bool ranges_pack)
 // lines costs there is less than the two launches the mixed form adds.
 constexpr std::size_t kPlainAlone = std::size_t{1} << 18;
 
+// Whether the scattered-record passes, where they can take a run, take all its
+// tiles: short runs, and runs without page registers, whose lines the batched
+// passes would take record by record as well (they batch what hits a
+// register), at more instructions a step: 67M 32-byte lines 2,512 us with the
+// tiles of lines left to them, 2,415 alone (2,466 before there were two pairs
+// of passes), packed 2,321 and 2,115.  Flat geometry has one plane: group_by
+// sees at once that a step has one group, where the match table takes its 64
+// lanes in turn, so tiles of lines stay with the batched passes (packed 1,422
+// us with them, 1,875 without).
+bool plain_takes_all(const KArgs& a, std::size_t n)
+{
+    return (n <= kPlainAlone && a.tile <= 256) || (a.slots == 0 && a.flat == 0);
+}
+
 void choose_match(KArgs& a, bool ranges_pack)
 {
     constexpr std::size_t kLdsPerCu = kLdsPerCuBytes;
@@ -7332,7 +7346,7 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
     // lines.  An engine whose last run mostly hit its page registers (runs of
     // lines) does not look for them.
     const bool plain = !grouping && !k2 && !refresh_records && plain_run(a, e->ranges_pack);
-    const bool plain_alone = plain && n <= kPlainAlone && a.tile <= 256;
+    const bool plain_alone = plain && plain_takes_all(a, n);
     const bool plain_mixed = plain && !plain_alone &&
                              (e->last_modeled == 0 || e->last_hits * 8 < e->last_modeled);
     a.mixed = plain_mixed ? 1u : 0u;

@@ -141,3 +141,27 @@ def test_which_passes_took_the_tiles():
         assert p.engine.last_tiles() == (-(-4099 // 64), 0)
     finally:
         p.close()
+
+
+@pytest.mark.parametrize("options", [dict(), dict(plane_contention=0), dict(transfer_page=1),
+                                     dict(flat_geometry=1)])
+def test_without_page_registers(options):
+    """Runs of more than 2^18 records without page registers go to the scattered-record passes
+    whole, lines too; with flat geometry the tiles of lines stay with the batched ones."""
+    ranges = ranges_of(4)
+    n = (1 << 18) + 4097
+    rec = scattered(n, ranges, 5)
+    rec[:131_072] = lines(131_072, ranges, 6)
+    rec[131_072:, 2] += np.uint64(int(rec[131_071, 2]))
+    for packed in (True, False):
+        p = parity.Pair(C0, ranges, page_buffers=0, **options)
+        try:
+            for k in range(2):
+                g, c = (p.run_packed if packed else p.run)(rec, k * 10**10)
+                parity.assert_same(g, c, f"packed={packed} {options} run {k}")
+                batched, taken = p.engine.last_tiles()
+                assert batched + taken == -(-n // 256)
+                assert batched == (131_072 // 256 if "flat_geometry" in options else 0)
+            p.check_state()
+        finally:
+            p.close()
