@@ -39,14 +39,15 @@ THERMAL_FLOPS_PER_CELL_SWEEP = 14
 RECORD_BYTES = {"packed": 16, "32": 32}
 
 
-def kernel_bytes(records: str, apply_rereads: bool = False) -> dict:
-    """Algorithmic bytes per access of the two per-record kernels.  The apply
+def kernel_bytes(records: str, passes: list[str], apply_rereads: bool = False) -> dict:
+    """Algorithmic bytes per access of the two per-record kernels, the first
+    and the last of `passes`.  The apply
     pass writes the 8-B completion; it re-reads the record too where steps
     are replayed from their records (streams without linear steps, such as
     random ones), and replays linear steps from the summary pass's step
     descriptors otherwise."""
-    return {"k_summary": RECORD_BYTES[records],
-            "k_apply": 8 + (RECORD_BYTES[records] if apply_rereads else 0)}
+    return {passes[0]: RECORD_BYTES[records],
+            passes[2]: 8 + (RECORD_BYTES[records] if apply_rereads else 0)}
 
 
 def profile_kernel_us(summary: str, kernel: str) -> float | None:
@@ -448,10 +449,10 @@ def sub_line(engine, profile, ranges, batches, records, args, what: str, mode="f
     its own roofline for the dominant per-record kernel, the same roofline
     recomputed from the committed kernel summary it cites, and the HBM
     traffic of that summary's counter companion."""
-    value, dt, kms, streamed, apply_waves = time_steps(engine, profile, ranges, batches, records,
-                                                       args, mode)
-    names = ["k_summary", "k_carry", "k_apply"]
-    kb = kernel_bytes(records, apply_rereads)
+    value, dt, kms, streamed, ran = time_steps(engine, profile, ranges, batches, records, args,
+                                               mode)
+    names = ran["passes"]
+    kb = kernel_bytes(records, names, apply_rereads)
     dominant = 0 if kms[0] >= kms[2] else 2
     per_launch = streamed / args.steps
     achieved = kb[names[dominant]] * per_launch / (kms[dominant] / 1e3) / 1e9
@@ -462,8 +463,9 @@ def sub_line(engine, profile, ranges, batches, records, args, what: str, mode="f
             "achieved": achieved, "peak": PEAK_HBM_GBPS, "unit": "GB/s",
             "frac": achieved / PEAK_HBM_GBPS,
             "kernel_ms": {nm: float(v) for nm, v in zip(names, kms)},
-            "apply_bytes_per_access": kb["k_apply"],
-            "apply_waves_per_simd": apply_waves,
+            "apply_bytes_per_access": kb[names[2]],
+            "apply_waves_per_simd": ran["apply_waves"],
+            "tiles": ran["tiles"],
             "algorithmic_bytes_per_access": algo,
             "pipeline_frac": value * algo / 1e9 / PEAK_HBM_GBPS}
     if kernels_summary is not None:
@@ -811,19 +813,19 @@ def main() -> None:
             records = "32"
     desc = dict(desc, records=("packed 16-byte records (hbf_record16)" if records == "packed"
                                else "32-byte records (hbf_record32)"))
-    value, dt, avg_ms, accesses, _ = time_steps(engine, profile, ranges, timed, records, args)
+    value, dt, avg_ms, accesses, ran = time_steps(engine, profile, ranges, timed, records, args)
     other = None
     if records == "packed" and not args.no_compare:
         # the same steps from 32-byte records, for comparison (its own roofline)
-        v32, dt32, ms32, _, _ = time_steps(engine, profile, ranges, batches, "32", args)
+        v32, dt32, ms32, _, ran32 = time_steps(engine, profile, ranges, batches, "32", args)
         other = {"records": "32-byte records (hbf_record32)", "value": v32,
                  "ms_per_step": dt32 / args.steps * 1e3, "algorithmic_bytes_per_access": 40,
                  "pipeline_frac": v32 * 40 / 1e9 / PEAK_HBM_GBPS,
                  "kernel_ms": {nm: float(v) for nm, v in
-                               zip(["k_summary", "k_carry", "k_apply"], ms32)}}
+                               zip(ran32["passes"], ms32)}}
     algo = RECORD_BYTES[records] + 8
-    kb = kernel_bytes(records)
-    names = ["k_summary", "k_carry", "k_apply"]
+    names = ran["passes"]
+    kb = kernel_bytes(records, names)
     # the dominant per-record kernel (the carry chain works per tile and resource)
     dominant = 0 if avg_ms[0] >= avg_ms[2] else 2
     per_launch = accesses / args.steps
@@ -869,10 +871,10 @@ def main() -> None:
         # each against the ceiling of its own access pattern
         out["roofline"]["measured_read_gbps"] = probe["read_gbps"]
         out["roofline"]["frac_of_measured_read"] = (
-            kb["k_summary"] * per_launch / (avg_ms[0] / 1e3) / 1e9 / probe["read_gbps"])
+            kb[names[0]] * per_launch / (avg_ms[0] / 1e3) / 1e9 / probe["read_gbps"])
         out["roofline"]["measured_write_gbps"] = probe["write_gbps"]
         out["roofline"]["k_apply_frac_of_measured_write"] = (
-            kb["k_apply"] * per_launch / (avg_ms[2] / 1e3) / 1e9 / probe["write_gbps"])
+            kb[names[2]] * per_launch / (avg_ms[2] / 1e3) / 1e9 / probe["write_gbps"])
         log("general path: random stream")
         out["general"] = bench_general(engine, args)
         log("hybrid mode")
@@ -920,8 +922,9 @@ def main() -> None:
 def time_steps(engine, profile, ranges, batches, records, args, mode="fast"):
     """Warm-up steps, then exactly `args.steps` timed steps of one engine
     (bracketed by device synchronisation); returns (modeled accesses/s,
-    seconds, average per-kernel ms, records streamed, waves per SIMD of the
-    last step's apply kernel)."""
+    seconds, average per-kernel ms, records streamed, and what the last step
+    ran: its tiles by pass, the passes that took most of them, and the waves
+    per SIMD its apply kernel was built for)."""
     import torch
     e = engine.Engine(str(profile), mode=mode)
     for base, length, perms in ranges:
@@ -948,11 +951,16 @@ def time_steps(engine, profile, ranges, batches, records, args, mode="fast"):
         kernel_ms += np.array(e.kernel_ms()[:3])
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
-    # the apply kernel's form in the last timed step (waves per SIMD it was built for)
-    apply_waves = e.apply_waves()
+    batched, scattered = e.last_tiles()
+    ran = {"tiles": {"batched": batched, "scattered": scattered},
+           "passes": (["k_plain_summary", "k_carry", "k_plain_apply"] if scattered > batched
+                      else ["k_summary", "k_carry", "k_apply"]),
+           # (apply_waves() speaks of k_apply where that was launched; k_plain_apply
+           # is built for four)
+           "apply_waves": 4 if scattered > batched else e.apply_waves()}
     e.close()
     # the metric counts modeled accesses; the kernels stream every record
-    return modeled / dt, dt, kernel_ms / args.steps, records_seen, apply_waves
+    return modeled / dt, dt, kernel_ms / args.steps, records_seen, ran
 
 
 if __name__ == "__main__":

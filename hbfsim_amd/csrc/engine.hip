@@ -7426,7 +7426,10 @@ int engine_run_any(engine* e, const void* d_rec, bool packed, std::size_t n,
     const bool wide_apply = packed && n >= kWideApplyRecords &&
                             kLdsPerCuBytes / lds_c >= 4 * kSimdsPerCu && e->last_modeled != 0 &&
                             e->last_hits * 8 < e->last_modeled;
-    e->last_apply_waves = packed && !k2 && !refresh_records ? (wide_apply ? 4 : 3) : 1;
+    // (k_plain_apply is built for four waves in either record form)
+    e->last_apply_waves = plain_alone                             ? 4
+                          : packed && !k2 && !refresh_records ? (wide_apply ? 4 : 3)
+                                                              : 1;
     if (plain_alone || plain_mixed) {
         const auto apply = packed ? (plain_alone ? k_plain_apply<true, true>
                                                  : k_plain_apply<true, false>)

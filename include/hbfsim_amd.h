@@ -389,12 +389,14 @@ int hbfsim_amd_reset(hbfsim_context* context);
 int hbfsim_amd_last_kernel_ms(const hbfsim_context* context, float* ms,
                               int max_kernels);
 /* Diagnostics, no counterpart in the reference: the waves per SIMD the last
- * run's apply kernel was built for (4: the form for large streams of general
- * steps, taken when the engine's previous run of at least 2^24 records had
- * fewer page-register hits than an eighth of its modeled records; 3: packed
- * records otherwise; 1: 32-byte records, two page registers or refresh
- * records), 0 before any run and after an empirical-model run (no apply
- * pass).  Results do not depend on the form. */
+ * run's apply kernel was built for: of the batched apply pass where it was
+ * launched (4: the form for large streams of general steps, taken when the
+ * engine's previous run of at least 2^24 records had fewer page-register hits
+ * than an eighth of its modeled records; 3: packed records otherwise; 1:
+ * 32-byte records, two page registers or refresh records), else 4, the
+ * scattered-record pass's (hbfsim_amd_last_tiles says which took the tiles);
+ * 0 before any run and after an empirical-model run (no apply pass).  Results
+ * do not depend on the form. */
 int hbfsim_amd_last_apply_waves(const hbfsim_context* context);
 /* Diagnostics likewise: how many tiles of the last run the batched passes
  * took (k_summary, k_apply: runs of lines, refresh records, grouping, two page

@@ -122,6 +122,7 @@ def test_which_passes_took_the_tiles():
         p.run_packed(scattered(4099, ranges, 1))
         batched, taken = p.engine.last_tiles()
         assert batched == 0 and taken == -(-4099 // 64)
+        assert p.engine.apply_waves() == 4  # k_plain_apply's
     finally:
         p.close()
     p = parity.Pair(C0, ranges)  # (no run before it that mostly hit its registers)
