@@ -722,22 +722,32 @@ MarchLaunch march_launcher(std::uint32_t s, int f = 1)
 // least two strips wide and eight rows per level long, whose rings fit the
 // workgroup's LDS limit.  Returns the LDS bytes, 0 when it does not apply.
 //
-// A grid that tiles hold too takes whichever is faster.  Six steps, tiles
-// against the march: 1 sweep at 200 x 180 x 8 68 -> 39 us, 600 x 500 x 1
-// 59 -> 37; 2 sweeps 79 -> 71 and 63 -> 58; 3 and 4 sweeps win from a
-// million cells (4 sweeps: 1100 x 1000 x 1 150 -> 116, 500 x 500 x 8 365 ->
-// 170) and with few layers lose below (600 x 500 x 1 77 -> 109).  At 5 and
-// more sweeps it is no clear gain (300 x 330 x 6 at 8: 381 and 330 us,
-// 130 x 2100 x 1 107 and 254).
+// A grid that tiles hold too takes whichever is faster (us, tiles and march).
+// 1 sweep, 12 steps: 512 x 512 x 1 81 and 64, 200 x 180 x 8 114 and 72.
+// 2 sweeps, 12 steps: with four to eight layers the march is as fast or faster
+// (260 x 260 x 4 103 and 113, 200 x 180 x 8 137 and 133, 130 x 520 x 4 124 and
+// 102), with fewer or more only from about 330,000 cells (130 x 2100 x 1 89 and
+// 106, 128 x 128 x 16 130 and 159; 600 x 600 x 1 even, 140 x 160 x 16 220 and
+// 161).  3 and 4 sweeps win from a million cells (6 steps of 4: 1024 x 1030 x 1
+// 151 and 132, 300 x 330 x 12 280 and 162) and with few layers lose below (600
+// x 500 x 1 77 and 109).  At 5 and more sweeps it is no clear gain (300 x 330 x
+// 6 at 8: 381 and 330 us, 130 x 2100 x 1 107 and 254).
 constexpr std::size_t kMarchMinCells = std::size_t{1} << 21;  // with no tile, or 5-8 sweeps
 
-std::size_t march_min_cells(std::uint32_t sweeps, bool tiled)
+std::size_t march_min_cells(const hbfsim_amd_thermal_grid& g, bool tiled)
 {
-    if (!tiled || sweeps > 4) {
+    if (!tiled || g.sweeps > 4) {
         return kMarchMinCells;
     }
-    return std::size_t{1} << (sweeps <= 2 ? 18 : 20);
+    if (g.sweeps > 2) {
+        return std::size_t{1} << 20;
+    }
+    return g.sweeps == 1 || (g.nz >= 4 && g.nz <= 8) ? std::size_t{1} << 18 : std::size_t{5} << 16;
 }
+
+// Calls of one or two steps at one sweep gain nothing from the march below
+// this size (130 x 2100 x 1, two steps: 28 us in tiles, 31 in single passes).
+constexpr std::size_t kMarchShortCells = std::size_t{1} << 19;
 
 // Fused passes (two steps per read and write of the grid) against single
 // ones: always at 1-3 sweeps (1000 x 1003 x 8: 145 us fused, 235 single for
@@ -745,7 +755,10 @@ std::size_t march_min_cells(std::uint32_t sweeps, bool tiled)
 // and in rows per segment than the traffic they save while temperatures in
 // and out and the power (24 B per cell) stay in the 256 MB of shared cache
 // (1000 x 1003 x 8: 282 single, 326 fused; 500 x 500 x 8 170 and 184); past
-// it the fused pass wins (2000 x 2000 x 8: 941 fused, 1065 single).
+// it the fused pass wins (2000 x 2000 x 8: 941 fused, 1065 single).  A call of
+// just two steps would end in the scratch after its one fused pass and copy
+// the grid back: grids that tiles hold too make two single passes of it
+// (260 x 350 x 4 at 2 sweeps: 40 us fused, 36 single, 45 in tiles).
 constexpr std::size_t kMarchCacheBytes = std::size_t{256} << 20;
 
 bool march_fused(const hbfsim_amd_thermal_grid& g)
@@ -759,7 +772,7 @@ std::size_t march_lds(const hbfsim_amd_thermal_grid& g, std::size_t lds_limit, b
 {
     const std::size_t cells = static_cast<std::size_t>(g.nx) * g.ny * g.nz;
     if (march_kernel(g.sweeps, f) == nullptr || g.nz > 16 ||
-        cells < march_min_cells(g.sweeps, tiled)) {
+        cells < march_min_cells(g, tiled)) {
         return 0;
     }
     const std::uint32_t levels = g.sweeps * static_cast<std::uint32_t>(f);
@@ -1199,6 +1212,7 @@ struct thermal {
     // marching stencil (uncoupled steps on large grids), set up at the first step
     bool march_checked = false;
     bool march = false;
+    bool tiled = false;            // tiles hold the grid too
     MArgs m[2] = {};               // [0] one step per pass, [1] two (m_lds[1] == 0: none)
     std::uint32_t m_blocks[2] = {}, m_threads[2] = {};
     std::size_t m_lds[2] = {};
@@ -1367,9 +1381,16 @@ hipError_t setup_march_form(thermal* th, bool tiled, int f)
     // A segment walks 2 L rows more than it writes; shorter ones still pay
     // until 2 L written rows, since a grid of one round takes as long as one
     // segment's walk (six steps of 4 sweeps, segments of >= 8 L rows and of
-    // >= 2 L: 700 x 500 x 8 206 -> 187 us single, 294 -> 204 fused;
-    // 1000 x 1003 x 8 309 -> 282 single)
-    const std::uint64_t max_segs = g.ny / (2ull * levels);
+    // >= 2 L: 700 x 500 x 8 206 -> 187 us single, 294 -> 204 fused; 1000 x 1003
+    // x 8 309 -> 282 single; 2000 x 2000 x 1 at 8 sweeps 463 -> 365).  Not with
+    // one sweep and at most three layers, once segments of 8 L rows give every
+    // SIMD two waves (twelve steps: 4000 x 700 x 1 122 us with 8 L, 131 with
+    // 2 L, 150 x 14000 x 1 106 and 120, 1000 x 1000 x 3 128 and 136; but 600 x
+    // 600 x 8 143 and 125).
+    const std::uint64_t long_segs = g.ny / (8ull * levels);
+    const bool full = strips * long_segs * g.nz >= 8ull * static_cast<std::uint64_t>(th->cus);
+    const std::uint64_t max_segs =
+        g.sweeps == 1 && g.nz <= 3 && full ? long_segs : g.ny / (2ull * levels);
     segs = std::max<std::uint64_t>(1, std::min(segs, max_segs));
     const std::uint32_t seg_len = static_cast<std::uint32_t>((g.ny + segs - 1) / segs);
     segs = (g.ny + seg_len - 1) / seg_len;
@@ -1401,6 +1422,7 @@ hipError_t setup_march(thermal* th)
     }
     std::uint32_t tx, ty;
     (void)choose_step_tile(th->grid, th->lds_per_block, tx, ty);
+    th->tiled = tx != 0;
     hipError_t err = setup_march_form(th, tx != 0, 1);
     if (err == hipSuccess && th->m_lds[0] != 0) {
         if (march_fused(th->grid)) {
@@ -1430,9 +1452,12 @@ int thermal_step(thermal* th, const double* d_power, double* d_temp, std::uint64
     if (!th->march_checked && setup_march(th) != hipSuccess) {
         return HBFSIM_CUDA_ERROR;
     }
+    const std::size_t cells = static_cast<std::size_t>(g.nx) * g.ny * g.nz;
+    const bool march = th->march && !(th->tiled && g.sweeps == 1 && steps <= 2 &&
+                                      cells < kMarchShortCells);
     TArgs a{};
     std::size_t lds = 0;
-    if (!th->march) {
+    if (!march) {
         std::uint32_t tx, ty;
         const bool wide = choose_step_tile(g, th->lds_per_block, tx, ty);
         if (tx == 0) {
@@ -1452,11 +1477,11 @@ int thermal_step(thermal* th, const double* d_power, double* d_temp, std::uint64
             th->wide_ready = true;
         }
     }
-    const std::size_t cells = static_cast<std::size_t>(g.nx) * g.ny * g.nz;
     // Passes: on the marching kernel pairs of steps in fused passes where
     // they pay (the power is the same in both), the others in single-step
     // ones.
-    const std::uint64_t pairs = th->march && th->m_lds[1] != 0 ? steps / 2 : 0;
+    const bool lone_pair = steps == 2 && th->tiled && cells < kMarchMinCells;
+    const std::uint64_t pairs = march && th->m_lds[1] != 0 && !lone_pair ? steps / 2 : 0;
     const std::uint64_t launches = steps - pairs;
     // Each pass reads one buffer and writes another.  An even count
     // alternates d_temp and the scratch and ends in d_temp; an odd count of 3
@@ -1481,7 +1506,7 @@ int thermal_step(thermal* th, const double* d_power, double* d_temp, std::uint64
     (void)hipEventRecord(th->ev[0], stream);
     for (std::uint64_t i = 0; i < launches && err == hipSuccess; ++i) {
         double* dst = target(i);
-        if (th->march) {
+        if (march) {
             const int f = i < pairs ? 2 : 1;
             MArgs m = th->m[f - 1];
             m.power = d_power;

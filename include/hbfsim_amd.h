@@ -569,8 +569,9 @@ typedef struct hbfsim_amd_thermal hbfsim_amd_thermal;
  * tiles of at most 2,048 cells ((t + 2 sweeps)^2 nz for some tile edge t),
  * or, on grids of at least 2^21 cells, on the marching kernel (at most 16
  * layers with 1-4 sweeps, at most 8 with 5-8; nx >= 2 (64 - 2 sweeps),
- * ny >= 8 sweeps).  A grid that both take marches from 2^18 cells with 1-2
- * sweeps, from 2^20 with 3-4. */
+ * ny >= 8 sweeps).  A grid that both take marches from 2^18 cells with 1
+ * sweep (calls of one or two steps from 2^19) and with 2 sweeps on 4-8 layers,
+ * from 5 * 2^16 with 2 sweeps otherwise, from 2^20 with 3-4. */
 int hbfsim_amd_thermal_create(const hbfsim_amd_thermal_grid* grid,
                               hbfsim_amd_thermal** out);
 /* ThermalModel::advance_to (thermal.cpp:127-160) with constant power:
@@ -585,7 +586,8 @@ int hbfsim_amd_thermal_last_ms(const hbfsim_amd_thermal* thermal, float* ms);
 /* Kernel passes the last hbfsim_amd_thermal_step call launched: one per step,
  * except that on the marching kernel with 1-3 sweeps, and with 4 on grids of
  * more than 256 MiB / 24 cells, one pass makes two steps (the power is the
- * same in both).  A diagnostic with no counterpart in the
+ * same in both); a call of just two steps on a grid of less than 2^21 cells
+ * that tiles hold too makes two.  A diagnostic with no counterpart in the
  * reference: it turns last_ms into a per-pass time. */
 int hbfsim_amd_thermal_last_launches(const hbfsim_amd_thermal* thermal, uint64_t* launches);
 void hbfsim_amd_thermal_destroy(hbfsim_amd_thermal* thermal);
