@@ -26,13 +26,15 @@ def test_split_steps(profile, options, kinds):
     try:
         for k in range(2):
             rec = split_stream(31 + k, 1200, ranges, kinds)
-            # 2^18 records and more take the batched passes whatever they hold
+            # (above 2^18 records tiles of runs go to the batched passes)
             rec = np.concatenate([rec] * 4)
             t = rec[: len(rec) // 4, 2].copy()
             for j in range(1, 4):
                 rec[j * len(t):(j + 1) * len(t), 2] = t + j * t[-1]
             g, c = p.run(rec, k * 10**11)
             parity.assert_same(g, c, f"{profile.name} {options} run {k}")
+            if options.get("page_buffers") != 0:  # (without page registers nothing is batched)
+                p.check_batched()
         p.check_state()
     finally:
         p.close()
